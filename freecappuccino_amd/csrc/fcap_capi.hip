@@ -1016,6 +1016,51 @@ extern "C" fc_status fc_dilu_pivots(fc_context *ctx, int n, int nnz, const int *
     return pivots_common(ctx, true, n, nnz, ioffset, ja, diag, a, d);
 }
 
+// The sweeps of one call outside a solve: packed factor, state and outputs for the
+// schedule the context chooses (nothing packed where the structure is not).
+struct SweepFactor {
+    DevBuf af, df, ab, db, sf, tmp, zp;
+    PackedFactor<double> pf;
+    SweepCfg cfg;
+
+    void prepare(fc_context *ctx, const Structure &st, const double *a, const double *d) {
+        if (!packed_sweeps(st)) return;
+        hipStream_t s = ctx->stream;
+        const size_t n = (size_t)st.n;
+        const SweepChoice ch = choose_sweeps(ctx, st);
+        cfg.parts = ch.parts;
+        if (ch.dep) {
+            sf.alloc(sizeof(SyncFree));
+            syncfree_reset(ctx, s, sf.as<SyncFree>());
+            cfg.sf = sf.as<SyncFree>();
+            cfg.waves = ch.parts ? part_wave_count(ctx) : syncfree_wave_count(ctx, st);
+            tmp.alloc(sizeof(double) * (ch.parts ? (size_t)st.pt_npk : n));
+            cfg.tmp = tmp.get();
+        }
+        if (ch.parts) {
+            zp.alloc(sizeof(double) * (size_t)st.pt_npk);
+            cfg.zp = zp.get();
+            af.alloc(sizeof(double) * part_factor_count(st, false));
+            ab.alloc(sizeof(double) * part_factor_count(st, true));
+            pack_factor_parts64(s, st, a, d, af.as<double>(), ab.as<double>(), tmp.as<double>());
+        } else {
+            af.alloc(sizeof(double) * (size_t)st.ell_f * n);
+            ab.alloc(sizeof(double) * (size_t)st.ell_b * n);
+            df.alloc(sizeof(double) * n);
+            db.alloc(sizeof(double) * n);
+            pack_factor64(s, st, a, d, af.as<double>(), df.as<double>(), ab.as<double>(), db.as<double>());
+        }
+        pf = {af.as<double>(), df.as<double>(), ab.as<double>(), db.as<double>()};
+    }
+
+    void check(fc_context *ctx) const {
+        if (!cfg.sf) return;
+        SyncFree h;
+        d2h(&h, sf.get(), sizeof(SyncFree), ctx->stream);
+        FC_REQUIRE(!h.abort, FC_ERR_HIP, "dependency-driven sweep: a wait exceeded its time limit");
+    }
+};
+
 extern "C" fc_status fc_lu_apply(fc_context *ctx, int n, int nnz, const int *ioffset, const int *ja, const int *diag,
                                  const double *a, const double *d, const double *r, double *z) {
     return guarded(ctx, [&]() {
@@ -1028,46 +1073,12 @@ extern "C" fc_status fc_lu_apply(fc_context *ctx, int n, int nnz, const int *iof
         upload_dbl(ctx, dr, r, n);
         dz.alloc(sizeof(double) * n);
         const double small = ctx->variant == FC_VARIANT_TESTS ? kSmallTests : kSmallSrc;
-        // the solvers' sweeps: level-packed operands when the structure has them
-        DevBuf af, df, ab, db;
-        PackedFactor<double> pf;
-        const SweepChoice ch = choose_sweeps(ctx, st);
-        const bool dep = ch.dep, parts = ch.parts;
-        if (packed_sweeps(st)) {
-            af.alloc(sizeof(double) * (size_t)st.ell_f * n);
-            ab.alloc(sizeof(double) * (size_t)st.ell_b * n);
-            df.alloc(sizeof(double) * n);
-            db.alloc(sizeof(double) * n);
-            if (parts)
-                pack_factor_parts64(ctx->stream, st, da.as<double>(), dd.as<double>(), af.as<double>(),
-                                    df.as<double>(), ab.as<double>(), db.as<double>());
-            else
-                pack_factor64(ctx->stream, st, da.as<double>(), dd.as<double>(), af.as<double>(), df.as<double>(),
-                              ab.as<double>(), db.as<double>());
-            pf.af = af.as<double>();
-            pf.df = df.as<double>();
-            pf.ab = ab.as<double>();
-            pf.db = db.as<double>();
-        }
-        SweepCfg cfg;
-        DevBuf sfs, sft;
-        if (dep && pf.af) {
-            sfs.alloc(sizeof(SyncFree));
-            sft.alloc(sizeof(double) * n);
-            syncfree_reset(ctx, ctx->stream, sfs.as<SyncFree>());
-            cfg.sf = sfs.as<SyncFree>();
-            cfg.tmp = sft.get();
-            cfg.waves = parts ? part_wave_count(ctx) : syncfree_wave_count(ctx, st);
-            cfg.parts = parts;
-        }
+        SweepFactor F;
+        F.prepare(ctx, st, da.as<double>(), dd.as<double>());
         lu_launch64(ctx->stream, st, da.as<double>(), dd.as<double>(), small, dr.as<double>(), dz.as<double>(),
-                    nullptr, &cfg, pf.af ? &pf : nullptr);
+                    nullptr, &F.cfg, F.pf.af ? &F.pf : nullptr);
         FC_HIP_CHECK(hipGetLastError());
-        if (cfg.sf) {
-            SyncFree h;
-            d2h(&h, sfs.get(), sizeof(SyncFree), ctx->stream);
-            FC_REQUIRE(!h.abort, FC_ERR_HIP, "dependency-driven sweep: a wait exceeded its time limit");
-        }
+        F.check(ctx);
         download_dbl(ctx, z, dz.get(), n);
         return FC_OK;
     });
@@ -1761,8 +1772,7 @@ extern "C" double fc_sys_sweep_bench(fc_system *sys, int dilu, int reps) {
         const int n = st.n;
         hipStream_t hs = ctx->stream;
         const double *a = sys->a.as<double>();
-        const SweepChoice ch = choose_sweeps(ctx, st);
-        const bool dep = ch.dep, parts = ch.parts;
+        const bool dep = choose_sweeps(ctx, st).dep;
         DevBuf d(sizeof(double) * n), z(sizeof(double) * n), err(sizeof(int)), sfs, sft;
         FC_HIP_CHECK(hipMemsetAsync(err.get(), 0, sizeof(int), hs));
         SweepCfg cfg;
@@ -1778,38 +1788,19 @@ extern "C" double fc_sys_sweep_bench(fc_system *sys, int dilu, int reps) {
         int herr = 0;
         d2h(&herr, err.get(), sizeof(int), hs);
         FC_REQUIRE(!herr, FC_ERR_ZERO_PIVOT, "sweep bench: a pivot is zero or not finite");
-        cfg.waves = parts ? part_wave_count(ctx) : syncfree_wave_count(ctx, st);
-        cfg.parts = parts;
-        DevBuf af, df, ab, db;
-        PackedFactor<double> pf;
-        if (packed_sweeps(st)) {
-            af.alloc(sizeof(double) * (size_t)st.ell_f * n);
-            ab.alloc(sizeof(double) * (size_t)st.ell_b * n);
-            df.alloc(sizeof(double) * n);
-            db.alloc(sizeof(double) * n);
-            if (parts)
-                pack_factor_parts64(hs, st, a, d.as<double>(), af.as<double>(), df.as<double>(), ab.as<double>(),
-                                    db.as<double>());
-            else
-                pack_factor64(hs, st, a, d.as<double>(), af.as<double>(), df.as<double>(), ab.as<double>(),
-                              db.as<double>());
-            pf = {af.as<double>(), df.as<double>(), ab.as<double>(), db.as<double>()};
-        }
-        const SweepCfg *pc = dep && pf.af ? &cfg : nullptr;
+        SweepFactor F;
+        F.prepare(ctx, st, a, d.as<double>());
+        const SweepCfg *pc = F.cfg.sf ? &F.cfg : nullptr;
+        const PackedFactor<double> *pf = F.pf.af ? &F.pf : nullptr;
         const double small = ctx->variant == FC_VARIANT_TESTS ? kSmallTests : kSmallSrc;
         lu_launch64(hs, st, a, d.as<double>(), small, sys->su.as<double>(), z.as<double>(), nullptr, pc,
-                    pf.af ? &pf : nullptr);   // warm-up
+                    pf);   // warm-up
         ctx->timer.start(hs);
         for (int r = 0; r < reps; ++r)
-            lu_launch64(hs, st, a, d.as<double>(), small, sys->su.as<double>(), z.as<double>(), nullptr, pc,
-                        pf.af ? &pf : nullptr);
+            lu_launch64(hs, st, a, d.as<double>(), small, sys->su.as<double>(), z.as<double>(), nullptr, pc, pf);
         FC_HIP_CHECK(hipGetLastError());
         const double ms = ctx->timer.stop_ms(hs);
-        if (pc) {
-            SyncFree h;
-            d2h(&h, sfs.get(), sizeof(SyncFree), hs);
-            FC_REQUIRE(!h.abort, FC_ERR_HIP, "dependency-driven sweep: a wait exceeded its time limit");
-        }
+        F.check(ctx);
         out = ms / reps;
         sys->last_ms[3] = out;
         return FC_OK;

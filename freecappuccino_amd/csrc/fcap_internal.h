@@ -105,16 +105,15 @@ struct Structure {
     DevBuf cnt_f, cnt_b;             // entries per packed row
     DevBuf kpos_f, kpos_b;           // CSR position of each slot
     DevBuf col_f, col_b;             // column of each slot
-    // Part-wise sweeps: the rows split into parts of kPartRows consecutive indices
-    // (in which the forward sweep reads only lower and the backward sweep only
-    // higher indices); each part's rows in the order of their levels, packed like
-    // the level order above (same widths).  int_frac: the fraction of the
-    // triangle's entries whose column lies in the row's own part.  meta: per
-    // packed row, its entry count | its step within its 64-row window << 8 | the
-    // window's number of steps << 16 (the static schedule of the part sweeps).
+    // Part-wise sweeps (fcap_parts.hip): the rows in parts, a part's rows in windows of
+    // 64 slots (pt_npk in all; a window's last row is repeated to its end), both sweeps
+    // over the same slots.  pt_rows: row of a slot; pt_step: rank of the slot's level in
+    // its window; pt_win: first window of every part; pt_codes_*: where a slot's entries
+    // are read from, then its row.  int_frac: the fraction of a triangle's entries read
+    // from the part's own LDS.
     bool parts = false;
-    DevBuf rows_pf, cnt_pf, kpos_pf, col_pf, meta_pf;
-    DevBuf rows_pb, cnt_pb, kpos_pb, col_pb, meta_pb;
+    int pt_npk = 0, pt_nparts = 0;
+    DevBuf pt_rows, pt_step, pt_win, pt_codes_f, pt_codes_b;
     double int_frac_f = 0.0, int_frac_b = 0.0;
 };
 
@@ -187,14 +186,10 @@ struct fc_context {
 
 namespace fcap {
 
-// persistent waves of the part-wise sweeps: the context's setting, else three per
-// two CUs (192^3 box, FP64 IC(0)-PCG with 4,096-row parts: 256 waves 1.03 s, 384
-// 0.93 s, 512 0.95 s, 768 1.03 s; with 2,048-row parts 512 waves were best at
-// 1.15 s, with 1,024-row parts 1.71 s, with 8,192-row parts 1.61 s: bigger parts
-// cross fewer part boundaries until too few of them run at once)
-inline int part_wave_count(const fc_context *ctx) {
-    return ctx->part_waves > 0 ? ctx->part_waves : 3 * ctx->num_cus / 2;
-}
+// persistent workgroups of the part-wise sweeps: the context's setting, else one per CU
+// (per sweep of the 192^3 box: 128 workgroups 373 us, 256 315, 384 364, 512 417: more of
+// them wait, and poll, than the chain of parts can use)
+inline int part_wave_count(const fc_context *ctx) { return ctx->part_waves > 0 ? ctx->part_waves : ctx->num_cus; }
 
 // persistent waves of the row-wise dependency-driven sweeps and pivots: one 64-row
 // block per wave for the rows of an average level, at least one wave per CU and at
@@ -217,6 +212,7 @@ void build_structure_from_faces_dev(fc_context *ctx, Structure &st, int n, int n
                                     const int *owner0_d, const int *neigh0_d, int *ij_slot_d,
                                     int *ji_slot_d);
 void analyse_levels(fc_context *ctx, Structure &st);
+void analyse_parts(fc_context *ctx, Structure &st);   // fcap_parts.hip
 inline void ensure_levels(fc_context *ctx, Structure &st) {
     if (!st.levels_ready) { analyse_levels(ctx, st); st.levels_ready = true; }
 }

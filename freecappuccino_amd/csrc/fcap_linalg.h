@@ -53,7 +53,10 @@ struct SweepCfg {
     SyncFree *sf = nullptr;
     int waves = 0;
     void *tmp = nullptr;
-    bool parts = false;   // part-wise schedule (Structure::rows_pf ...; factor packed in part order)
+    // part-wise schedule: factor packed in part order (pack_factor_parts*); tmp and zp, the
+    // sweeps' packed outputs, have Structure::pt_npk entries
+    bool parts = false;
+    void *zp = nullptr;
 };
 // part-wise sweeps (FC_SWEEP_PARTS): the structure has them, and at least half of each
 // triangle's entries lie in their row's own part (else the dependency-driven schedule)
@@ -104,11 +107,19 @@ void pack_factor64(hipStream_t s, const Structure &st, const double *a, const do
                    double *ab, double *db);
 void pack_factor32(hipStream_t s, const Structure &st, const float *a, const float *d, float *af, float *df,
                    float *ab, float *db);
-// the same values in the part-wise order (Structure::rows_pf / rows_pb)
-void pack_factor_parts64(hipStream_t s, const Structure &st, const double *a, const double *d, double *af,
-                         double *df, double *ab, double *db);
-void pack_factor_parts32(hipStream_t s, const Structure &st, const float *a, const float *d, float *af, float *df,
-                         float *ab, float *db);
+// The same values in the part-wise order, entries and pivot of a slot together
+// (part_factor_count values per triangle, PackedFactor's df and db unused); also
+// marks tmp, the forward sweep's output, as the first sweep expects it.
+size_t part_factor_count(const Structure &st, bool upper);
+void pack_factor_parts64(hipStream_t s, const Structure &st, const double *a, const double *d, double *af, double *ab,
+                         double *tmp);
+void pack_factor_parts32(hipStream_t s, const Structure &st, const float *a, const float *d, float *af, float *ab,
+                         float *tmp);
+// both sweeps in the part-wise schedule (lu_launch* with cfg.parts)
+void lu_parts64(hipStream_t s, const Structure &st, const PackedFactor<double> &pf, double small, const double *rhs,
+                double *w, const Scalars *sc, const SweepCfg &cfg);
+void lu_parts32(hipStream_t s, const Structure &st, const PackedFactor<float> &pf, float small, const float *rhs,
+                float *w, const Scalars *sc, const SweepCfg &cfg);
 
 // DIC (src/iccg.f90:77-83) / DILU (src/bicgstab.f90:68-79) pivots: one launch per
 // level, or with cfg->sf one dependency-driven launch (bit-identical).

@@ -16,6 +16,7 @@
 #include "fcap_internal.h"
 #include "fcap_kernels.h"
 #include "fcap_linalg.h"
+#include "fcap_syncfree.h"
 
 namespace fcap {
 
@@ -469,41 +470,7 @@ void pack_factor_t(hipStream_t s, const Structure &st, const T *a, const T *d, T
 
 // Waves in flight poll the coherent level of the memory system; the fewer there
 // are, the faster the chain of levels advances (192^3 box: 256 waves 1.87 s,
-// 512 1.96 s, 2048 2.55 s, 4096 3.61 s per FP64 IC(0)-PCG solve).  A wait is
-// bounded in wall-clock time (wall_clock64(), a constant-rate counter), not in
-// polls, so the bound does not shrink with a deeper chain or a faster clock:
-// it only ends waits that cannot end otherwise.
-constexpr unsigned long long kSfWaitUs = 2000000ull;   // 2 s
-
-// the wait limit in wall-clock ticks (sf->wait_us microseconds, 0: kSfWaitUs)
-__device__ inline unsigned long long sf_wait_ticks(const SyncFree *sf, unsigned long long rate_khz) {
-    const unsigned long long us = sf->wait_us > 0 ? (unsigned long long)sf->wait_us : kSfWaitUs;
-    return us * rate_khz / 1000ull + 1ull;
-}
-
-template <class T> struct SfBits;
-template <> struct SfBits<double> {
-    using U = unsigned long long;
-    static constexpr U kMark = 0x7FF4DEADBEEF0001ull;   // signalling NaN
-};
-template <> struct SfBits<float> {
-    using U = unsigned;
-    static constexpr U kMark = 0x7FA0BEEFu;               // signalling NaN
-};
-
-template <class T>
-__device__ inline typename SfBits<T>::U sf_load_bits(const T *p) {
-    return __hip_atomic_load(reinterpret_cast<const typename SfBits<T>::U *>(p), __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_AGENT);
-}
-
-template <class T>
-__device__ inline void sf_store(T *p, T v) {
-    using U = typename SfBits<T>::U;
-    U b;
-    __builtin_memcpy(&b, &v, sizeof(U));
-    __hip_atomic_store(reinterpret_cast<U *>(p), b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
+// 512 1.96 s, 2048 2.55 s, 4096 3.61 s per FP64 IC(0)-PCG solve).
 
 template <class T>
 __global__ void k_sf_mark(int n, T *__restrict__ w, const Scalars *__restrict__ sc) {
@@ -592,208 +559,6 @@ __global__ __launch_bounds__(64) void k_sweep_syncfree(int n, const int *__restr
             }
             __builtin_amdgcn_s_sleep(1);
         }
-    }
-    if (lane == 0) {
-        const unsigned f = __hip_atomic_fetch_add(&sf->fin, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        if (f == gridDim.x - 1) {
-            __hip_atomic_store(&sf->ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&sf->fin, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    }
-}
-
-// ---------------------------------------------------- part-wise sweeps
-// One launch per sweep.  The rows are split into parts of kPartRows consecutive
-// indices: the forward sweep reads only rows of lower index and the backward one
-// only rows of higher index, so a part depends only on the parts before it (after
-// it, backward) in index order, and tickets hand the parts out in that order: every
-// part a part reads has been handed to a wave that is running or has finished.
-// A persistent wave computes its part 64 packed rows (a window) at a time, the
-// rows in the order of their levels.  The part's values live in the wave's LDS.
-// A window first waits until every input it reads outside the part is in global
-// memory (polled like k_sweep_syncfree's: the signalling-NaN mark means "not yet"),
-// then computes its rows in the static schedule of Structure::meta_*: at step s the
-// rows of step s, whose inputs inside the part are in LDS by then (earlier steps or
-// earlier windows).  Only this wave touches its LDS and a wave's LDS operations
-// complete in order, so the steps need no barrier.  A row's value is computed
-// exactly as in k_sweep_syncfree and published with one coherent store at the end
-// of its window.
-//
-// The loads run two windows ahead: a window's operands are loaded two windows
-// before it, its right-hand side and the first poll of its outside inputs one
-// window before; three register sets rotate through the unrolled window loop, and
-// every lane issues the same loads and stores on every path (the padding lanes of
-// a part's last window repeat its last row: same loads, same value, same store),
-// so the waits on the vector-memory counter only cover loads issued a window ago.
-// Waits are bounded in wall-clock time as in k_sweep_syncfree.
-template <class T, int W>
-struct PartRow {
-    int i, meta;
-    int cj[W];
-    T ak[W];
-    T di;
-};
-template <class T, int W>
-struct PartWin {
-    PartRow<T, W> o;
-    T rhs;
-    typename SfBits<T>::U pb[W];
-};
-
-template <class T, int W>
-__device__ __forceinline__ void part_row_load(PartRow<T, W> &o, int q, int last, int n, const int *__restrict__ rows,
-                                              const int *__restrict__ meta, const int *__restrict__ col,
-                                              const T *__restrict__ av, const T *__restrict__ dv) {
-    q = min(q, last);
-    o.i = rows[q];
-    o.meta = meta[q];
-    o.di = dv[q];
-#pragma unroll
-    for (int k = 0; k < W; ++k) {
-        o.cj[k] = col[(size_t)k * n + q];
-        o.ak[k] = av[(size_t)k * n + q];
-    }
-}
-
-template <bool BWD>
-__device__ __forceinline__ bool part_inside(int j, int r0, int r1) {
-    return BWD ? j < r1 : j >= r0;
-}
-
-// the right-hand side and the first poll of the row's inputs outside the part:
-// every slot issues a load, of the row's own output where the slot is inside the
-// part or padding, so that every lane issues the same loads (the address is
-// blended arithmetically: a select between two operand fields would keep the
-// register sets in scratch memory)
-template <class T, int W, bool BWD>
-__device__ __forceinline__ void part_inputs(PartWin<T, W> &S, int r0, int r1, const T *__restrict__ in,
-                                            const T *out) {
-    S.rhs = in[S.o.i];
-    const int c = S.o.meta & 255;
-#pragma unroll
-    for (int k = 0; k < W; ++k) {
-        const int j = S.o.cj[k];
-        const int own = -(int)(k >= c || part_inside<BWD>(j, r0, r1));   // all ones or zero
-        S.pb[k] = sf_load_bits(out + (j + ((S.o.i - j) & own)));
-    }
-}
-
-// one window: S0 its operands and inputs, S1 the next window (operands loaded, its
-// inputs issued here), N2 the window after (operands issued here); false: gave up
-template <class T, int W, bool BWD>
-__device__ __forceinline__ bool part_window(PartWin<T, W> &S0, PartWin<T, W> &S1, PartRow<T, W> &N2, int q0, int r0,
-                                            int r1, int n, typename SfBits<T>::U *lv, const int *__restrict__ rows,
-                                            const int *__restrict__ meta, const int *__restrict__ col,
-                                            const T *__restrict__ av, const T *__restrict__ dv,
-                                            const T *__restrict__ in, T small, T *out, SyncFree *sf,
-                                            unsigned long long limit) {
-    using U = typename SfBits<T>::U;
-    const int lane = threadIdx.x;
-    const int c = S0.o.meta & 255, step = (S0.o.meta >> 8) & 255;
-    const int nst = __shfl((S0.o.meta >> 16) & 255, 0);
-    T wk[W];
-    unsigned need = 0;
-#pragma unroll
-    for (int k = 0; k < W; ++k) {
-        wk[k] = __builtin_bit_cast(T, S0.pb[k]);
-        if (k < c && !part_inside<BWD>(S0.o.cj[k], r0, r1) && S0.pb[k] == SfBits<T>::kMark) need |= 1u << k;
-    }
-    if (__any(need != 0)) {
-        const unsigned long long t0 = wall_clock64();
-        do {
-            __builtin_amdgcn_s_sleep(1);
-            U r[W];
-#pragma unroll
-            for (int k = 0; k < W; ++k) r[k] = ((need >> k) & 1u) ? sf_load_bits(out + S0.o.cj[k]) : SfBits<T>::kMark;
-#pragma unroll
-            for (int k = 0; k < W; ++k) {
-                if (((need >> k) & 1u) && r[k] != SfBits<T>::kMark) {
-                    wk[k] = __builtin_bit_cast(T, r[k]);
-                    need &= ~(1u << k);
-                }
-            }
-            const bool give_up = wall_clock64() - t0 > limit ||
-                                 __hip_atomic_load(&sf->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
-            if (__any(give_up)) {
-                if (lane == 0) __hip_atomic_store(&sf->abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                return false;
-            }
-        } while (__any(need != 0));
-    }
-    const int last = r1 - 1;
-    __builtin_amdgcn_sched_barrier(0);
-    part_inputs<T, W, BWD>(S1, r0, r1, in, out);
-    __builtin_amdgcn_sched_barrier(0);
-    part_row_load<T, W>(N2, q0 + 128 + lane, last, n, rows, meta, col, av, dv);
-    __builtin_amdgcn_sched_barrier(0);
-    const T acc = BWD ? S0.rhs / (S0.o.di + small) : S0.rhs;
-    T v = T(0);
-    for (int st = 0; st < nst; ++st) {
-        if (step == st) {
-            U b[W];
-#pragma unroll
-            for (int k = 0; k < W; ++k) {
-                const bool ins = k < c && part_inside<BWD>(S0.o.cj[k], r0, r1);
-                b[k] = lv[ins ? S0.o.cj[k] - r0 : 0];
-            }
-            T r = acc;
-#pragma unroll
-            for (int k = 0; k < W; ++k) {
-                T x = wk[k];
-                if (k < c && part_inside<BWD>(S0.o.cj[k], r0, r1)) x = __builtin_bit_cast(T, b[k]);
-                if (k < c) r = r - S0.o.ak[k] * x;
-            }
-            v = r * S0.o.di;
-            lv[S0.o.i - r0] = __builtin_bit_cast(U, v);
-        }
-    }
-    sf_store(out + S0.o.i, v);
-    return true;
-}
-
-template <class T, int W, bool BWD>
-__global__ __launch_bounds__(64) void k_sweep_parts(int n, const int *__restrict__ rows, const int *__restrict__ meta,
-                                                     const int *__restrict__ col, const T *__restrict__ av,
-                                                     const T *__restrict__ dv, const T *__restrict__ in, T small,
-                                                     T *out, SyncFree *sf, const Scalars *__restrict__ sc) {
-    using U = typename SfBits<T>::U;
-    __shared__ U lv[kPartRows];
-    if (sc && sc->done) return;
-    const int lane = threadIdx.x;
-    const unsigned nparts = (unsigned)((n + kPartRows - 1) / kPartRows);
-    const unsigned long long limit = sf_wait_ticks(sf, sf->rate_khz);
-    for (;;) {
-        unsigned t = 0;
-        if (lane == 0) t = __hip_atomic_fetch_add(&sf->ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        t = __shfl(t, 0);
-        if (t >= nparts) break;
-        const int part = BWD ? (int)(nparts - 1u - t) : (int)t;
-        const int r0 = part * kPartRows, r1 = min(n, r0 + kPartRows);
-        // the same issue order as inside the loop (inputs of A before the operands of
-        // B), so that the loop head's waits on its two entries nearly agree
-        PartWin<T, W> A, B, C;
-        part_row_load<T, W>(A.o, r0 + lane, r1 - 1, n, rows, meta, col, av, dv);
-        __builtin_amdgcn_sched_barrier(0);
-        part_inputs<T, W, BWD>(A, r0, r1, in, out);
-        __builtin_amdgcn_sched_barrier(0);
-        part_row_load<T, W>(B.o, r0 + 64 + lane, r1 - 1, n, rows, meta, col, av, dv);
-        __builtin_amdgcn_sched_barrier(0);
-        bool ok = true;
-        for (int q0 = r0;;) {
-            if (!(ok = part_window<T, W, BWD>(A, B, C.o, q0, r0, r1, n, lv, rows, meta, col, av, dv, in, small, out,
-                                               sf, limit)))
-                break;
-            if ((q0 += 64) >= r1) break;
-            if (!(ok = part_window<T, W, BWD>(B, C, A.o, q0, r0, r1, n, lv, rows, meta, col, av, dv, in, small, out,
-                                               sf, limit)))
-                break;
-            if ((q0 += 64) >= r1) break;
-            if (!(ok = part_window<T, W, BWD>(C, A, B.o, q0, r0, r1, n, lv, rows, meta, col, av, dv, in, small, out,
-                                               sf, limit)))
-                break;
-            if ((q0 += 64) >= r1) break;
-        }
-        if (!ok) break;
     }
     if (lane == 0) {
         const unsigned f = __hip_atomic_fetch_add(&sf->fin, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
@@ -933,43 +698,6 @@ bool part_sweeps(const Structure &st) {
 }
 
 template <class T, int WF, int WB>
-void lu_parts_w(hipStream_t s, const Structure &st, const PackedFactor<T> &pf, T small, const T *rhs, T *w,
-                const Scalars *sc, const SweepCfg &cfg) {
-    const int n = st.n;
-    T *tmp = static_cast<T *>(cfg.tmp);
-    const int nparts = (n + kPartRows - 1) / kPartRows;
-    const int waves = std::max(1, std::min(cfg.waves, nparts));
-    k_sf_mark<T><<<grid_for(n, 256), 256, 0, s>>>(n, tmp, sc);
-    k_sweep_parts<T, WF, false><<<waves, 64, 0, s>>>(n, st.rows_pf.as<int>(), st.meta_pf.as<int>(), st.col_pf.as<int>(),
-                                                       pf.af, pf.df, rhs, small, tmp, cfg.sf, sc);
-    k_sf_mark<T><<<grid_for(n, 256), 256, 0, s>>>(n, w, sc);
-    k_sweep_parts<T, WB, true><<<waves, 64, 0, s>>>(n, st.rows_pb.as<int>(), st.meta_pb.as<int>(), st.col_pb.as<int>(),
-                                                      pf.ab, pf.db, tmp, small, w, cfg.sf, sc);
-}
-
-template <class T, int WF>
-void lu_parts_b(hipStream_t s, const Structure &st, const PackedFactor<T> &pf, T small, const T *rhs, T *w,
-                const Scalars *sc, const SweepCfg &cfg) {
-    switch (st.ell_b) {
-    case 3: lu_parts_w<T, WF, 3>(s, st, pf, small, rhs, w, sc, cfg); break;
-    case 4: lu_parts_w<T, WF, 4>(s, st, pf, small, rhs, w, sc, cfg); break;
-    default: lu_parts_w<T, WF, 8>(s, st, pf, small, rhs, w, sc, cfg); break;
-    }
-}
-
-template <class T>
-void lu_parts(hipStream_t s, const Structure &st, const PackedFactor<T> &pf, T small, const T *rhs, T *w,
-              const Scalars *sc, const SweepCfg &cfg) {
-    FC_REQUIRE(part_sweeps(st) && cfg.tmp && cfg.sf, FC_ERR_ARGUMENT, "part-wise sweeps not set up");
-    switch (st.ell_f) {
-    case 3: lu_parts_b<T, 3>(s, st, pf, small, rhs, w, sc, cfg); break;
-    case 4: lu_parts_b<T, 4>(s, st, pf, small, rhs, w, sc, cfg); break;
-    default: lu_parts_b<T, 8>(s, st, pf, small, rhs, w, sc, cfg); break;
-    }
-    FC_HIP_CHECK(hipGetLastError());
-}
-
-template <class T, int WF, int WB>
 void lu_syncfree_w(hipStream_t s, const Structure &st, const PackedFactor<T> &pf, T small, const T *rhs, T *w,
                    const Scalars *sc, const SweepCfg &cfg) {
     const int n = st.n;
@@ -1010,7 +738,8 @@ template <class T>
 void lu_launch_t(hipStream_t s, const Structure &st, const T *a, const T *d, T small, const T *rhs, T *w,
                  const Scalars *sc, const SweepCfg *cfg, const PackedFactor<T> *pf) {
     if (cfg && cfg->sf && cfg->parts && pf && pf->af) {
-        lu_parts<T>(s, st, *pf, small, rhs, w, sc, *cfg);
+        if constexpr (sizeof(T) == sizeof(double)) lu_parts64(s, st, *pf, small, rhs, w, sc, *cfg);
+        else lu_parts32(s, st, *pf, small, rhs, w, sc, *cfg);
         return;
     }
     if (cfg && cfg->sf && pf && pf->af) {
@@ -1054,27 +783,6 @@ void pack_factor64(hipStream_t s, const Structure &st, const double *a, const do
 void pack_factor32(hipStream_t s, const Structure &st, const float *a, const float *d, float *af, float *df,
                    float *ab, float *db) {
     pack_factor_t<float>(s, st, a, d, af, df, ab, db);
-}
-
-template <class T>
-void pack_factor_parts_t(hipStream_t s, const Structure &st, const T *a, const T *d, T *af, T *df, T *ab, T *db) {
-    FC_REQUIRE(st.parts && packed_sweeps(st), FC_ERR_ARGUMENT, "structure has no part-wise sweeps");
-    const int n = st.n;
-    k_pack_factor<T><<<grid_for(n, 256), 256, 0, s>>>(n, st.ell_f, st.rows_pf.as<int>(), st.cnt_pf.as<int>(),
-                                                      st.kpos_pf.as<int>(), a, d, af, df);
-    k_pack_factor<T><<<grid_for(n, 256), 256, 0, s>>>(n, st.ell_b, st.rows_pb.as<int>(), st.cnt_pb.as<int>(),
-                                                      st.kpos_pb.as<int>(), a, d, ab, db);
-    FC_HIP_CHECK(hipGetLastError());
-}
-
-void pack_factor_parts64(hipStream_t s, const Structure &st, const double *a, const double *d, double *af,
-                         double *df, double *ab, double *db) {
-    pack_factor_parts_t<double>(s, st, a, d, af, df, ab, db);
-}
-
-void pack_factor_parts32(hipStream_t s, const Structure &st, const float *a, const float *d, float *af, float *df,
-                         float *ab, float *db) {
-    pack_factor_parts_t<float>(s, st, a, d, af, df, ab, db);
 }
 
 // ----------------------------------------------------------- reductions

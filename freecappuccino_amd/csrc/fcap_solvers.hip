@@ -577,6 +577,10 @@ static void setup_sweeps(Ctx &c, const Structure &st) {
         c.sw.tmp = c.ws->sf_tmp.get();
         c.sw.waves = syncfree_wave_count(c.ctx, st);
         if (ch.parts) {
+            c.ws->sf_tmp.ensure(sizeof(double) * (size_t)st.pt_npk);
+            c.ws->sf_zp.ensure(sizeof(double) * (size_t)st.pt_npk);
+            c.sw.tmp = c.ws->sf_tmp.get();
+            c.sw.zp = c.ws->sf_zp.get();
             c.sw.parts = true;
             c.sw.waves = part_wave_count(c.ctx);
         }
@@ -601,22 +605,25 @@ static PackedFactor<T> pack_for_solve(Ctx &c, const Structure &st, const T *a, c
     constexpr bool f32 = sizeof(T) == sizeof(float);
     DevBuf &af = f32 ? ws.pk_af32 : ws.pk_af, &df = f32 ? ws.pk_df32 : ws.pk_df;
     DevBuf &ab = f32 ? ws.pk_ab32 : ws.pk_ab, &db = f32 ? ws.pk_db32 : ws.pk_db;
+    if (c.sw.parts) {
+        af.ensure(sizeof(T) * part_factor_count(st, false));
+        ab.ensure(sizeof(T) * part_factor_count(st, true));
+        T *tmp = static_cast<T *>(c.sw.tmp);
+        if constexpr (f32) pack_factor_parts32(c.s, st, a, d, af.as<float>(), ab.as<float>(), tmp);
+        else pack_factor_parts64(c.s, st, a, d, af.as<double>(), ab.as<double>(), tmp);
+        pf.af = af.as<T>();
+        pf.ab = ab.as<T>();
+        return pf;
+    }
     const size_t n = (size_t)st.n;
     af.ensure(sizeof(T) * n * (size_t)st.ell_f);
     ab.ensure(sizeof(T) * n * (size_t)st.ell_b);
     df.ensure(sizeof(T) * n);
     db.ensure(sizeof(T) * n);
-    if constexpr (f32) {
-        if (c.sw.parts)
-            pack_factor_parts32(c.s, st, a, d, af.as<float>(), df.as<float>(), ab.as<float>(), db.as<float>());
-        else
-            pack_factor32(c.s, st, a, d, af.as<float>(), df.as<float>(), ab.as<float>(), db.as<float>());
-    } else {
-        if (c.sw.parts)
-            pack_factor_parts64(c.s, st, a, d, af.as<double>(), df.as<double>(), ab.as<double>(), db.as<double>());
-        else
-            pack_factor64(c.s, st, a, d, af.as<double>(), df.as<double>(), ab.as<double>(), db.as<double>());
-    }
+    if constexpr (f32)
+        pack_factor32(c.s, st, a, d, af.as<float>(), df.as<float>(), ab.as<float>(), db.as<float>());
+    else
+        pack_factor64(c.s, st, a, d, af.as<double>(), df.as<double>(), ab.as<double>(), db.as<double>());
     pf.af = af.as<T>();
     pf.df = df.as<T>();
     pf.ab = ab.as<T>();

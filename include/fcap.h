@@ -400,22 +400,24 @@ fc_status fc_set_fcg_stagnation(fc_context *ctx, int window, double factor);
  *   FC_SWEEP_DEPENDENT one launch per sweep, each row waiting only for the rows
  *                      it reads (packed structures of width 3, 4 or 8; other
  *                      structures keep the level launches);
- *   FC_SWEEP_PARTS     (default) one launch per sweep over parts of 4,096
- *                      consecutive rows, one persistent wave per part at a time,
- *                      64 rows per window in a schedule fixed at analysis:
- *                      inputs inside the part are read from the wave's LDS, only
- *                      inputs from other parts wait on global memory.  Used when
- *                      at least half of each triangle's entries lie inside their
- *                      row's part (meshes numbered with locality, as the
- *                      reference's are); else FC_SWEEP_DEPENDENT where levels
- *                      are narrow (fewer than 65,536 rows on average) and
- *                      FC_SWEEP_LEVELS where they are wide.
+ *   FC_SWEEP_PARTS     (default) one launch per sweep over parts of rows, one
+ *                      persistent workgroup per part at a time, 64 rows per window
+ *                      in a schedule fixed at analysis: inputs inside the part are
+ *                      read from the workgroup's LDS, only inputs from other parts
+ *                      wait on global memory.  Parts are pencils of 64 lines where
+ *                      the numbering has the runs of a structured block, else runs
+ *                      of 4,096 rows.  Used when at least half of each triangle's
+ *                      entries are read from their row's own part (meshes numbered
+ *                      with locality, as the reference's are); else
+ *                      FC_SWEEP_DEPENDENT where levels are narrow (fewer than
+ *                      65,536 rows on average) and FC_SWEEP_LEVELS where they are
+ *                      wide.
  * A wait that runs past its time limit fails the call with FC_ERR_HIP.
  * No counterpart in the reference. */
 enum { FC_SWEEP_LEVELS = 0, FC_SWEEP_DEPENDENT = 2, FC_SWEEP_PARTS = 3 };
 fc_status fc_set_sweep_mode(fc_context *ctx, int mode);
 /* Persistent waves of the dependency-driven sweeps and pivots (0: automatic --
- * two per compute unit for the part-wise sweeps, for the row-wise ones one
+ * one workgroup per compute unit for the part-wise sweeps, for the row-wise ones one
  * 64-row block per wave for an average level's rows, within 1 to 16 per compute
  * unit; at most 65,536).  No counterpart in the reference. */
 fc_status fc_set_sweep_waves(fc_context *ctx, int waves);

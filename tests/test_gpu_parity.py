@@ -719,3 +719,63 @@ def test_part_sweeps_bitwise_on_multi_part_meshes(ctx, mesh):
                 np.testing.assert_array_equal(fcap.lu_apply(csr, mat, d, r, ctx), ref, err_msg=f"mode {mode}")
     finally:
         ctx.set_sweep_mode(fcap.SWEEP_DEFAULT)
+
+
+def _renumbered(m, order):
+    """The mesh with cell `order[k]` numbered k (faces put back into upper-triangular order)."""
+    new = np.empty(m.n_cells, np.int64)
+    new[order] = np.arange(m.n_cells)
+    nif = m.n_inner
+    nodes = m.face_nodes.reshape(m.n_faces, -1)
+    return M._canonical_polymesh(m.points, m.n_cells, new[m.owner[:nif]], new[m.neighbour], nodes[:nif],
+                                 new[m.owner[nif:]], nodes[nif:],
+                                 np.repeat(np.arange(len(m.patches)), [p[1] for p in m.patches]),
+                                 [p[0] for p in m.patches])
+
+
+def _part_meshes():
+    # pencils: full and ragged line and sheet blocks, one sheet, one line, one cell, thin sheets
+    for dims in ((9, 7, 5), (16, 16, 16), (17, 65, 1), (300, 1, 1), (5, 130, 1), (3, 2, 70), (70, 9, 17), (1, 1, 1),
+                 (33, 64, 2), (12, 1, 40)):
+        yield "box_%dx%dx%d" % dims, M.hex_box(*dims)
+    # two blocks numbered one after the other, a sheet of each size: two stacks
+    m = M.hex_box(24, 20, 12)
+    c = np.arange(m.n_cells)
+    i = c % 24
+    yield "two_blocks", _renumbered(m, np.concatenate([c[i < 9], c[i >= 9]]))
+    # numberings without such runs: consecutive parts (z fastest in tiles), scattered rows
+    x, y, z = i, (c // 24) % 20, c // 480
+    yield "tiles", _renumbered(m, np.lexsort((x % 4, z % 4, y % 4, x // 4, y // 4, z // 4)))
+    yield "scattered", _renumbered(m, np.random.default_rng(4).permutation(m.n_cells))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,m", list(_part_meshes()), ids=lambda v: v if isinstance(v, str) else "")
+def test_part_sweeps_bitwise_over_numberings(ctx, name, m):
+    """The part-wise sweeps over every form of parts -- pencils with ragged line and sheet blocks,
+    several stacks, consecutive runs -- give the oracle's DIC and DILU sweeps bit for bit, and the
+    FP32 sweeps inside the mixed solver the same iterates as one launch per level."""
+    geo = O.mesh_geometry(m)
+    csr = O.csr_build(m.n_cells, m.owner[:m.n_inner] + 1, m.neighbour + 1)
+    rng = np.random.default_rng(11)
+    su = rng.uniform(-1, 1, m.n_cells)
+    a, _ = O.laplacian(m, geo, csr, np.full(m.n_cells, -1.0), np.zeros(m.n_cells + m.n_boundary), su)
+    r = rng.uniform(-1, 1, m.n_cells)
+    d = O.dic_pivots(csr, a)
+    np.testing.assert_array_equal(fcap.lu_apply(csr, a, d, r, ctx), O.lu_apply(csr, a, d, r), err_msg=name)
+    skew = a * rng.uniform(0.8, 1.2, a.shape[0])
+    dl = O.dilu_pivots(csr, skew)
+    np.testing.assert_array_equal(fcap.lu_apply(csr, skew, dl, r, ctx), O.lu_apply(csr, skew, dl, r), err_msg=name)
+    s = fcap.System(m, ctx)
+    out = []
+    try:
+        for mode in (fcap.SWEEP_PARTS, fcap.SWEEP_LEVELS):
+            ctx.set_sweep_mode(mode)
+            s.assemble_laplacian(np.full(m.n_cells, -1.0), None, su)
+            s.set_solution(np.zeros(m.n_cells))
+            s.solve(fcap.METHOD_ICCG_MIXED, fcap.STOP_L2, 1e-8, 500)
+            out.append(s.solution())
+    finally:
+        ctx.set_sweep_mode(fcap.SWEEP_DEFAULT)
+        s.close()
+    np.testing.assert_array_equal(out[0], out[1], err_msg=name)
