@@ -21,6 +21,12 @@ constexpr int kSpmvRows = kWave * kSpmvWaves;    // rows per SpMV block
 constexpr int kSpmvCap = 512;                    // LDS entries staged per wave (8 per row on average)
 constexpr int kRedBlock = 256;                   // block size of the reduction kernels
 constexpr int kMaxRedGrid = 2048;                // grid cap of grid-stride reductions
+// Most partials a kernel sums by itself in every block (fused solver iterations): 1,024
+// of them cost each block about 2 us, a finaliser launch of its own 4 to 6 us; the SpMV
+// writes one partial per 256 rows, so systems of more than 524,288 rows keep its finaliser.
+constexpr int kVecGrid = 1024;                   // grid cap of the fused vector kernels
+constexpr int kDirectParts = 2048;               // SpMV partials read directly
+constexpr int kVecParts = 4;                     // values per partial of the fused vector kernels (3 used)
 constexpr int kFcgM = 16;                        // most directions truncated flexible CG can keep
 constexpr double kFcgInnerEta = 1e-2;            // default inner tolerance of flexible CG
 constexpr int kXcds = 8;                         // XCDs of an MI355X (workgroups are dealt round-robin)
@@ -34,6 +40,9 @@ struct Scalars {
     double res0, resl, rsm, resmax, small;
     double s0, sk, bet, alf, pkapk;            // PCG
     double om, gam, beto, ukreso, vr, vv;      // BiCGStab
+    // sums formed by one fused kernel and taken over by the next: the kernel that forms
+    // them still reads the values they replace (sk, beto) in its other blocks
+    double sk_next, beto_next;
     double bnorm2, rnorm2, rel;                // L2 quantities (mixed precision / L2 stop)
     double inner_tol2, inner_r0;               // inner-solve stopping threshold
     double fcg_pr;                             // flexible CG: p.r of this step
@@ -71,6 +80,37 @@ __device__ inline double block_sum(double v, double *sh) {
     }
     __syncthreads();
     return r;
+}
+
+// The first N of the S sums of np partials (S values each), in a fixed order: the same in
+// every block and thread.  sh: N x BLOCK / kWave doubles.
+template <int BLOCK, int N, int S>
+__device__ inline void parts_total(const double *__restrict__ p, int np, double *sh, double (&out)[N]) {
+    constexpr int kW = BLOCK / kWave;
+    double v[N];
+#pragma unroll
+    for (int t = 0; t < N; ++t) v[t] = 0.0;
+    for (int i = threadIdx.x; i < np; i += BLOCK) {
+#pragma unroll
+        for (int t = 0; t < N; ++t) v[t] += p[(size_t)i * S + t];
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+#pragma unroll
+        for (int t = 0; t < N; ++t) v[t] += __shfl_down(v[t], off, kWave);
+    }
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+#pragma unroll
+        for (int t = 0; t < N; ++t) sh[t * kW + threadIdx.x / kWave] = v[t];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < N; ++t) {
+        out[t] = 0.0;
+#pragma unroll
+        for (int w = 0; w < kW; ++w) out[t] += sh[t * kW + w];
+    }
+    __syncthreads();
 }
 
 }  // namespace fcap

@@ -13,7 +13,7 @@ struct Workspace {
     // FP32 vectors and matrix copies
     DevBuf r32, z32, p32, q32, e32, a32, d32;
     // reduction partials, summed scalars, device solver state, error flag
-    DevBuf pa, pb, sums, sc, err;
+    DevBuf pa, pb, pv, pz, pq, pq2, sums, sc, err;
     // dependency-driven sweeps: their ticket state, the forward sweep's result, and the
     // part-wise sweeps' packed backward result
     DevBuf sf, sf_tmp, sf_zp;

@@ -8,6 +8,13 @@
 // the scalar update of the algorithm (beta, alpha, omega, convergence test).
 // Every kernel returns at once when `done` is set, so the host enqueues
 // iterations in batches and reads one flag per batch.
+//
+// Fused iterations (every solve without O-C couplings and with tree-order sums): the
+// finalisers are folded into the kernels that need the sums, each block of which adds
+// the partials itself, in the same order, so all blocks have the same scalars; block 0
+// records them.  An iteration is rotated to begin with A p (PCG) or the new direction
+// (BiCGStab), so that the kernel that ends it also tests for convergence; the
+// recurrences are those of the finalisers.
 
 #include <algorithm>
 #include <chrono>
@@ -265,28 +272,6 @@ __global__ __launch_bounds__(kRedBlock) void k_fcg_xr(int n, float *__restrict__
 }
 
 // x += alf p ; r -= alf q ; partials |r| and r^2 (src/iccg.f90:147-154)
-template <class T, class X>
-__global__ __launch_bounds__(kRedBlock) void k_pcg_xr(int n, X *__restrict__ x, T *__restrict__ r,
-                                                      const T *__restrict__ p, const T *__restrict__ q,
-                                                      const Scalars *__restrict__ sc, double *__restrict__ pa,
-                                                      double *__restrict__ pb) {
-    __shared__ double sh[kRedBlock / kWave];
-    if (sc->done) return;
-    const T alf = (T)sc->alf;
-    double a = 0.0, b = 0.0;
-    for (int i = blockIdx.x * kRedBlock + threadIdx.x; i < n; i += gridDim.x * kRedBlock) {
-        x[i] = x[i] + (X)(alf * p[i]);
-        T rv = r[i] - alf * q[i];
-        r[i] = rv;
-        a += fabs((double)rv);
-        b += (double)rv * (double)rv;
-    }
-    a = block_sum<kRedBlock>(a, sh);
-    b = block_sum<kRedBlock>(b, sh);
-    if (threadIdx.x == 0) { pa[blockIdx.x] = a; pb[blockIdx.x] = b; }
-}
-
-// FP64 variant kept separate so x + alf*p rounds exactly as the reference
 __global__ __launch_bounds__(kRedBlock) void k_pcg_xr64(int n, double *__restrict__ x, double *__restrict__ r,
                                                        const double *__restrict__ p, const double *__restrict__ q,
                                                        const Scalars *__restrict__ sc, double *__restrict__ pa,
@@ -369,6 +354,254 @@ __global__ void k_bicg_xr1(int n, X *__restrict__ fi, T *__restrict__ res, const
     }
 }
 
+// ------------------------------------------------- fused solver iterations
+
+// the end of an iteration with ||r||_1 = a and ||r||_2^2 = b, sc->iters counting it:
+// the status (kStatusRunning: go on), the same in every block
+__device__ inline int end_test(const Scalars *sc, double a, double b, double &rsm, double &rel) {
+    rsm = a / (sc->res0 + sc->small);
+    rel = sc->stop_rule == 1 ? sqrt(b / sc->bnorm2) : sc->rel;
+    const bool conv = sc->stop_rule == 0 ? rsm < sc->resmax : sc->stop_rule == 1 ? rel < sc->resmax : b <= sc->inner_tol2;
+    if (!(isfinite(a) && isfinite(b))) return FC_ERR_NONFINITE;
+    if (conv) return FC_OK;
+    return sc->iters >= sc->nsw ? FC_NOT_CONVERGED : kStatusRunning;
+}
+
+__device__ inline void record_end(Scalars *sc, double a, double b, double rsm, double rel, int status) {
+    sc->resl = a;
+    sc->rnorm2 = b;
+    sc->rsm = rsm;
+    sc->rel = rel;
+    if (status != kStatusRunning) {
+        sc->done = 1;
+        sc->status = status;
+    }
+}
+
+// Partials of the fused vector kernels: block b's |r|_1, |r|_2^2 and r.z (or res.reso) at
+// pv[kVecParts b ..]; one reduction adds what a kernel needs of them.
+__device__ inline void vec_part(double *pv, double a, double b, double c) {
+    double *p = pv + (size_t)kVecParts * blockIdx.x;
+    p[0] = a;
+    p[1] = b;
+    p[2] = c;
+}
+
+// block sums of three values, valid in thread 0
+__device__ inline void block_sum3(double &a, double &b, double &c, double *sh) {
+    constexpr int kW = kRedBlock / kWave;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        a += __shfl_down(a, off, kWave);
+        b += __shfl_down(b, off, kWave);
+        c += __shfl_down(c, off, kWave);
+    }
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+        const int w = threadIdx.x / kWave;
+        sh[w] = a;
+        sh[kW + w] = b;
+        sh[2 * kW + w] = c;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        a = b = c = 0.0;
+        for (int w = 0; w < kW; ++w) {
+            a += sh[w];
+            b += sh[kW + w];
+            c += sh[2 * kW + w];
+        }
+    }
+}
+
+constexpr int kVecShared = 3 * (kRedBlock / kWave);
+
+// Convergence test (not on the first call), bet = r.z / (r.z of the iteration before),
+// p = z + bet p (src/iccg.f90:114-125).  JAC: z = r / d formed here, z then is r, and the
+// partials of r.z are those of pv; otherwise they are pz's (nz of them).
+template <class T, bool JAC>
+__global__ __launch_bounds__(kRedBlock) void k_cg_p(int n, T *__restrict__ p, const T *__restrict__ z,
+                                                   const T *__restrict__ d, Scalars *__restrict__ sc,
+                                                   const double *__restrict__ pv, int nv,
+                                                   const double *__restrict__ pz, int nz, int first) {
+    __shared__ double sh[kVecShared];
+    if (sc->done) return;
+    const bool rec = blockIdx.x == 0 && threadIdx.x == 0;
+    double t[3];
+    if (JAC || !first) parts_total<kRedBlock, 3, kVecParts>(pv, nv, sh, t);
+    if (!first) {
+        double rsm, rel;
+        const int status = end_test(sc, t[0], t[1], rsm, rel);
+        if (rec) record_end(sc, t[0], t[1], rsm, rel, status);
+        if (status != kStatusRunning) return;
+    }
+    double rz[1] = {t[2]};
+    if (!JAC) parts_total<kRedBlock, 1, 1>(pz, nz, sh, rz);
+    const double bet64 = rz[0] / sc->sk;
+    if (rec) {
+        sc->sk_next = rz[0];
+        sc->bet = bet64;
+    }
+    const T bet = (T)bet64;
+    for (int i = blockIdx.x * kRedBlock + threadIdx.x; i < n; i += gridDim.x * kRedBlock)
+        p[i] = (JAC ? z[i] / d[i] : z[i]) + bet * p[i];
+}
+
+// alf = r.z / p.q; x += alf p ; r -= alf q (src/iccg.f90:143-154); partials |r|, r^2 and,
+// JAC, r.z of the next z = r / d.
+template <class T, class X, bool JAC>
+__global__ __launch_bounds__(kRedBlock) void k_cg_xr(int n, X *__restrict__ x, T *__restrict__ r,
+                                                    const T *__restrict__ p, const T *__restrict__ q,
+                                                    const T *__restrict__ d, Scalars *__restrict__ sc,
+                                                    const double *__restrict__ pq, int nq, double *__restrict__ pv) {
+    __shared__ double sh[kVecShared];
+    if (sc->done) return;
+    double pkapk[1];
+    parts_total<kRedBlock, 1, 1>(pq, nq, sh, pkapk);
+    const double sk = sc->sk_next, alf64 = sk / pkapk[0];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        sc->sk = sk;
+        sc->pkapk = pkapk[0];
+        sc->alf = alf64;
+        sc->iters += 1;
+    }
+    const T alf = (T)alf64;
+    double a = 0.0, b = 0.0, c = 0.0;
+    for (int i = blockIdx.x * kRedBlock + threadIdx.x; i < n; i += gridDim.x * kRedBlock) {
+        x[i] = x[i] + (X)(alf * p[i]);
+        const T rv = r[i] - alf * q[i];
+        r[i] = rv;
+        a += fabs((double)rv);
+        b += (double)rv * (double)rv;
+        if (JAC) c += (double)rv * (double)(T)(rv / d[i]);
+    }
+    block_sum3(a, b, c, sh);
+    if (threadIdx.x == 0) vec_part(pv, a, b, c);
+}
+
+// Convergence test (not on the first call), bet = res.reso, om = bet gam / (alf beto +
+// small), pk = res + om (pk - alf uk) (src/bicgstab.f90:101-111)
+template <class T>
+__global__ __launch_bounds__(kRedBlock) void k_bi_p(int n, T *__restrict__ pk, const T *__restrict__ res,
+                                                   const T *__restrict__ uk, Scalars *__restrict__ sc,
+                                                   const double *__restrict__ pv, int nv, int first) {
+    __shared__ double sh[kVecShared];
+    if (sc->done) return;
+    const bool rec = blockIdx.x == 0 && threadIdx.x == 0;
+    double t[3];
+    parts_total<kRedBlock, 3, kVecParts>(pv, nv, sh, t);
+    if (!first) {
+        double rsm, rel;
+        const int status = end_test(sc, t[0], t[1], rsm, rel);
+        if (rec) record_end(sc, t[0], t[1], rsm, rel, status);
+        if (status != kStatusRunning) return;
+    }
+    const double bet = t[2];
+    const double om64 = (bet * sc->gam) / ((sc->alf * sc->beto) + sc->small);
+    if (rec) {
+        sc->om = om64;
+        sc->sk_next = bet;
+        sc->beto_next = bet;
+    }
+    const T om = (T)om64, alf = (T)sc->alf;
+    for (int i = blockIdx.x * kRedBlock + threadIdx.x; i < n; i += gridDim.x * kRedBlock) {
+        T t1 = alf * uk[i];
+        t1 = pk[i] - t1;
+        t1 = om * t1;
+        pk[i] = res[i] + t1;
+    }
+}
+
+// gam = bet / uk.reso; fi += gam zk ; res -= gam uk (src/bicgstab.f90:152-161)
+template <class T, class X>
+__global__ __launch_bounds__(kRedBlock) void k_bi_xr1(int n, X *__restrict__ fi, T *__restrict__ res,
+                                                     const T *__restrict__ zk, const T *__restrict__ uk,
+                                                     Scalars *__restrict__ sc, const double *__restrict__ pq, int nq) {
+    __shared__ double sh[kVecShared];
+    if (sc->done) return;
+    double ukreso[1];
+    parts_total<kRedBlock, 1, 1>(pq, nq, sh, ukreso);
+    const double sk = sc->sk_next, gam64 = sk / ukreso[0];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        sc->ukreso = ukreso[0];
+        sc->sk = sk;
+        sc->gam = gam64;
+        sc->beto = sc->beto_next;
+    }
+    const T gam = (T)gam64;
+    for (int i = blockIdx.x * kRedBlock + threadIdx.x; i < n; i += gridDim.x * kRedBlock) {
+        fi[i] = fi[i] + (X)(gam * zk[i]);
+        res[i] = res[i] - gam * uk[i];
+    }
+}
+
+// alf = vk.res / (vk.vk + small); fi += alf zk ; res -= alf vk (src/bicgstab.f90:200-208);
+// partials |res|, res^2 and res.reso of the next iteration
+template <class T, class X>
+__global__ __launch_bounds__(kRedBlock) void k_bi_xr2(int n, X *__restrict__ fi, T *__restrict__ res,
+                                                     const T *__restrict__ zk, const T *__restrict__ vk,
+                                                     const T *__restrict__ reso, Scalars *__restrict__ sc,
+                                                     const double *__restrict__ pvr, const double *__restrict__ pvv,
+                                                     int nv, double *__restrict__ pv) {
+    __shared__ double sh[kVecShared];
+    if (sc->done) return;
+    double vr[1], vv[1];
+    parts_total<kRedBlock, 1, 1>(pvr, nv, sh, vr);
+    parts_total<kRedBlock, 1, 1>(pvv, nv, sh, vv);
+    const double alf64 = vr[0] / (vv[0] + sc->small);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        sc->vr = vr[0];
+        sc->vv = vv[0];
+        sc->alf = alf64;
+        sc->iters += 1;
+    }
+    const T alf = (T)alf64;
+    double a = 0.0, b = 0.0, c = 0.0;
+    for (int i = blockIdx.x * kRedBlock + threadIdx.x; i < n; i += gridDim.x * kRedBlock) {
+        fi[i] = fi[i] + (X)(alf * zk[i]);
+        const T rv = res[i] - alf * vk[i];
+        res[i] = rv;
+        a += fabs((double)rv);
+        b += (double)rv * (double)rv;
+        c += (double)rv * (double)reso[i];
+    }
+    block_sum3(a, b, c, sh);
+    if (threadIdx.x == 0) vec_part(pv, a, b, c);
+}
+
+// the SpMV's partials as one value each
+__global__ __launch_bounds__(kFinBlock) void k_parts_one(int np, const double *__restrict__ pa,
+                                                        const double *__restrict__ pb, double *__restrict__ out,
+                                                        const Scalars *__restrict__ sc) {
+    __shared__ double sh[kFinBlock / kWave];
+    if (sc->done) return;
+    double a[1], b[1] = {0.0};
+    parts_total<kFinBlock, 1, 1>(pa, np, sh, a);
+    if (pb) parts_total<kFinBlock, 1, 1>(pb, np, sh, b);
+    if (threadIdx.x == 0) {
+        out[0] = a[0];
+        out[1] = b[0];
+    }
+}
+
+// The first iteration's partials: x.y, or with d x.(y / d)
+template <class T>
+__global__ __launch_bounds__(kRedBlock) void k_first_dot(int n, const T *__restrict__ x, const T *__restrict__ y,
+                                                         const T *__restrict__ d, const Scalars *__restrict__ sc,
+                                                         double *__restrict__ pv) {
+    __shared__ double sh[kVecShared];
+    if (sc->done) return;
+    double a = 0.0, b = 0.0, c = 0.0;
+    for (int i = blockIdx.x * kRedBlock + threadIdx.x; i < n; i += gridDim.x * kRedBlock)
+        c += (double)x[i] * (double)(d ? (T)(y[i] / d[i]) : y[i]);
+    block_sum3(a, b, c, sh);
+    if (threadIdx.x == 0) vec_part(pv, a, b, c);
+}
+
+// d = a(diag)
+__global__ void k_diag(int n, const double *__restrict__ a, const int *__restrict__ diag, double *__restrict__ d) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) d[i] = a[diag[i]];
+}
+
 template <class T>
 __global__ void k_copy(int n, const T *__restrict__ x, T *__restrict__ y) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) y[i] = x[i];
@@ -407,7 +640,10 @@ struct Ctx {
     int n;
     Scalars *sc;
     double *pa, *pb;
+    // fused iterations: the vector kernels' partials, r.z, the SpMV's, and the sums of those
+    double *pv, *pz, *pq, *pq2, *one;
     int gv;   // grid of the vector kernels
+    int gf;   // grid of the fused ones
     SweepCfg sw;   // how the triangular sweeps run
 };
 
@@ -418,6 +654,7 @@ Scalars init_scalars(const SolveArgs &args, double small) {
     h.resmax = (args.variant == FC_VARIANT_TESTS) ? (double)1e-13f : args.sor;
     h.nsw = (args.variant == FC_VARIANT_TESTS) ? 100 : args.nsw;
     h.s0 = kS0;
+    h.sk = kS0;   // fused iterations: the r.z before the first
     h.alf = 1.0;
     h.beto = 1.0;
     h.gam = 1.0;
@@ -444,6 +681,24 @@ int read_done(Ctx &c) {
     FC_HIP_CHECK(hipStreamSynchronize(c.s));
     return hf[0];
 }
+
+// the SpMV's partials (pq, and pq2 with two) as the fused kernels read them
+struct SpmvSums {
+    const double *a, *b;
+    int n;
+};
+SpmvSums spmv_sums(Ctx &c, bool two) {
+    const int gs = spmv_grid(c.n);
+    if (gs <= kDirectParts) return {c.pq, c.pq2, gs};
+    k_parts_one<<<1, kFinBlock, 0, c.s>>>(gs, c.pq, two ? c.pq2 : nullptr, c.one, c.sc);
+    return {c.one, c.one + 1, 1};
+}
+
+// whether a solve's iterations are the fused ones
+bool fused(const Ctx &c, const OcView &oc) { return !c.ctx->reduce_seq && !oc.noc; }
+
+// four rows a thread where that still gives every CU two blocks
+int fused_grid(int n) { return std::min(kVecGrid, grid_for(n, n >= 512 * 4 * kRedBlock ? 4 * kRedBlock : 2 * kRedBlock)); }
 
 void fin(Ctx &c, int step, int nparts, bool two) {
     k_fin<<<1, kFinBlock, 0, c.s>>>(step, nparts, c.pa, two ? c.pb : nullptr, c.sc);
@@ -512,6 +767,17 @@ struct GraphExec {
     ~GraphExec() { if (exec) (void)hipGraphExecDestroy(exec); }
 };
 
+struct Events {
+    hipEvent_t e[2] = {nullptr, nullptr};
+    Events() {
+        for (hipEvent_t &x : e) FC_HIP_CHECK(hipEventCreateWithFlags(&x, hipEventDisableTiming));
+    }
+    ~Events() {
+        for (hipEvent_t x : e)
+            if (x) (void)hipEventDestroy(x);
+    }
+};
+
 void run_batches(Ctx &c, int batch, const std::function<void()> &iter) {
     GraphExec ge;
     if (c.ctx->use_graphs && c.s != nullptr) {
@@ -529,14 +795,24 @@ void run_batches(Ctx &c, int batch, const std::function<void()> &iter) {
         (void)hipGraphDestroy(g);
         FC_HIP_CHECK(e);
     }
-    while (true) {
+    // The flag of a batch is read while the next one runs, so the GPU does not idle for
+    // the host's round trip (25 us a batch); past the end it finds `done` set and every
+    // kernel returns.
+    Events ev;
+    int *flags = c.ctx->host_flags;
+    for (int b = 0;; ++b) {
         for (int k = 0; k < batch; ++k) {
             if (ge.exec) FC_HIP_CHECK(hipGraphLaunch(ge.exec, c.s));
             else iter();
         }
         FC_HIP_CHECK(hipGetLastError());
-        if (read_done(c)) break;
+        FC_HIP_CHECK(hipMemcpyAsync(flags + (b & 1), &c.sc->done, sizeof(int), hipMemcpyDeviceToHost, c.s));
+        FC_HIP_CHECK(hipEventRecord(ev.e[b & 1], c.s));
+        if (b == 0) continue;
+        FC_HIP_CHECK(hipEventSynchronize(ev.e[(b - 1) & 1]));
+        if (flags[(b - 1) & 1]) break;
     }
+    FC_HIP_CHECK(hipStreamSynchronize(c.s));
 }
 
 }  // namespace
@@ -554,6 +830,10 @@ void Workspace::ensure(int n_, int nnz_) {
     const int parts = std::max(kFcgM * kMaxRedGrid, spmv_grid(n_));   // kFcgM dot products at once (FCG)
     pa.ensure(sizeof(double) * parts);
     pb.ensure(sizeof(double) * parts);
+    pv.ensure(sizeof(double) * kVecParts * kVecGrid);
+    pz.ensure(sizeof(double) * kVecGrid);
+    pq.ensure(sizeof(double) * spmv_grid(n_));
+    pq2.ensure(sizeof(double) * spmv_grid(n_));
     sums.ensure(sizeof(double) * 4);
     sc.ensure(sizeof(Scalars));
     err.ensure(sizeof(int) * 4);
@@ -565,7 +845,8 @@ void Workspace::ensure(int n_, int nnz_) {
 
 static Ctx make_ctx(fc_context *ctx, int n) {
     Workspace &ws = *ctx->ws;
-    Ctx c{ctx, ctx->stream, &ws, n, ws.sc.as<Scalars>(), ws.pa.as<double>(), ws.pb.as<double>(), red_grid(n), {}};
+    Ctx c{ctx, ctx->stream, &ws, n, ws.sc.as<Scalars>(), ws.pa.as<double>(), ws.pb.as<double>(), ws.pv.as<double>(), ws.pz.as<double>(),
+          ws.pq.as<double>(), ws.pq2.as<double>(), ws.sums.as<double>() + 2, red_grid(n), fused_grid(n), {}};
     return c;
 }
 
@@ -687,6 +968,7 @@ fc_status solve_pcg64(fc_context *ctx, const SolveArgs &args, bool dic, fc_solve
     const double small = args.variant == FC_VARIANT_TESTS ? kSmallTests : kSmallSrc;
     double *r = ws.r.as<double>(), *z = ws.z.as<double>(), *p = ws.p.as<double>(), *q = ws.q.as<double>();
     double *d = ws.d.as<double>();
+    const bool fuse = fused(c, args.oc);
     Scalars h = init_scalars(args, small);
     if (h.stop_rule == 1) h.bnorm2 = norm2_host(c, args.su);
     ctx->timer.start(c.s);
@@ -708,6 +990,37 @@ fc_status solve_pcg64(fc_context *ctx, const SolveArgs &args, bool dic, fc_solve
     }
     const int *ptr = st.ioffset.as<int>(), *ja = st.ja.as<int>(), *dg = st.diag.as<int>();
     const int gs = spmv_grid(n);
+    ctx->timer.start(c.s);
+    if (fuse) {
+        if (!dic) k_diag<<<c.gv, 256, 0, c.s>>>(n, args.a, dg, z);   // z holds the diagonal
+        auto precondition = [&](int first) {
+            if (dic) {
+                lu_launch64(c.s, st, args.a, d, small, r, z, c.sc, &c.sw, pf.af ? &pf : nullptr);
+                k_dot<double><<<c.gf, kRedBlock, 0, c.s>>>(n, r, z, c.sc, c.pz);
+                k_cg_p<double, false><<<c.gf, kRedBlock, 0, c.s>>>(n, p, z, nullptr, c.sc, c.pv, c.gf, c.pz, c.gf, first);
+            } else {
+                if (first) k_first_dot<double><<<c.gf, kRedBlock, 0, c.s>>>(n, r, r, z, c.sc, c.pv);
+                k_cg_p<double, true><<<c.gf, kRedBlock, 0, c.s>>>(n, p, r, z, c.sc, c.pv, c.gf, nullptr, 0, first);
+            }
+        };
+        precondition(1);
+        run_batches(c, dic ? 2 : 4, [&]() {
+            spmv_launch64(c.s, 2, n, ptr, ja, args.a, p, nullptr, p, q, nullptr, c.pq, nullptr, c.sc);
+            const SpmvSums pq = spmv_sums(c, false);
+            if (dic)
+                k_cg_xr<double, double, false><<<c.gf, kRedBlock, 0, c.s>>>(n, args.fi, r, p, q, nullptr, c.sc, pq.a,
+                                                                           pq.n, c.pv);
+            else
+                k_cg_xr<double, double, true><<<c.gf, kRedBlock, 0, c.s>>>(n, args.fi, r, p, q, z, c.sc, pq.a, pq.n,
+                                                                          c.pv);
+            precondition(0);
+        });
+        const double solve_ms = ctx->timer.stop_ms(c.s);
+        check_sweeps(c);
+        Scalars hs = read_scalars(c);
+        fill_info(info, hs, setup_ms, solve_ms);
+        return (fc_status)hs.status;
+    }
     auto iter = [&]() {
         if (dic) {
             lu_launch64(c.s, st, args.a, d, small, r, z, c.sc, &c.sw, pf.af ? &pf : nullptr);
@@ -729,8 +1042,7 @@ fc_status solve_pcg64(fc_context *ctx, const SolveArgs &args, bool dic, fc_solve
         k_pcg_xr64<<<c.gv, kRedBlock, 0, c.s>>>(n, args.fi, r, p, q, c.sc, c.pa, c.pb);
         fin(c, kFinPcgEnd, seq_or(c, c.gv, 1, r, nullptr), true);
     };
-    ctx->timer.start(c.s);
-    run_batches(c, dic ? 1 : 8, iter);
+    run_batches(c, dic ? 2 : 4, iter);
     double solve_ms = ctx->timer.stop_ms(c.s);
     check_sweeps(c);
     Scalars hs = read_scalars(c);
@@ -769,6 +1081,31 @@ fc_status solve_bicgstab64(fc_context *ctx, const SolveArgs &args, fc_solve_info
     }
     const int *ptr = st.ioffset.as<int>(), *ja = st.ja.as<int>();
     const int gs = spmv_grid(n);
+    ctx->timer.start(c.s);
+    if (!c.ctx->reduce_seq) {   // (the reference's BiCGStab applies its O-C couplings to the initial residual alone)
+        auto direction = [&](int first) {
+            k_bi_p<double><<<c.gf, kRedBlock, 0, c.s>>>(n, pk, res, uk, c.sc, c.pv, c.gf, first);
+        };
+        k_first_dot<double><<<c.gf, kRedBlock, 0, c.s>>>(n, res, reso, nullptr, c.sc, c.pv);
+        direction(1);
+        run_batches(c, 2, [&]() {
+            lu_launch64(c.s, st, args.a, d, small, pk, zk, c.sc, &c.sw, ppf);
+            spmv_launch64(c.s, 2, n, ptr, ja, args.a, zk, nullptr, reso, uk, nullptr, c.pq, nullptr, c.sc);
+            const SpmvSums ur = spmv_sums(c, false);
+            k_bi_xr1<double, double><<<c.gf, kRedBlock, 0, c.s>>>(n, args.fi, res, zk, uk, c.sc, ur.a, ur.n);
+            lu_launch64(c.s, st, args.a, d, small, res, zk, c.sc, &c.sw, ppf);
+            spmv_launch64(c.s, 3, n, ptr, ja, args.a, zk, nullptr, res, vk, nullptr, c.pq, c.pq2, c.sc);
+            const SpmvSums v = spmv_sums(c, true);
+            k_bi_xr2<double, double><<<c.gf, kRedBlock, 0, c.s>>>(n, args.fi, res, zk, vk, reso, c.sc, v.a, v.b, v.n,
+                                                                 c.pv);
+            direction(0);
+        });
+        const double solve_ms = ctx->timer.stop_ms(c.s);
+        check_sweeps(c);
+        Scalars hs = read_scalars(c);
+        fill_info(info, hs, setup_ms, solve_ms);
+        return (fc_status)hs.status;
+    }
     auto iter = [&]() {
         k_dot<double><<<c.gv, kRedBlock, 0, c.s>>>(n, res, reso, c.sc, c.pa);
         fin(c, kFinBet, seq_or(c, c.gv, 0, res, reso), false);
@@ -783,8 +1120,7 @@ fc_status solve_bicgstab64(fc_context *ctx, const SolveArgs &args, fc_solve_info
         k_pcg_xr64<<<c.gv, kRedBlock, 0, c.s>>>(n, args.fi, res, zk, vk, c.sc, c.pa, c.pb);
         fin(c, kFinBicgEnd, seq_or(c, c.gv, 1, res, nullptr), true);
     };
-    ctx->timer.start(c.s);
-    run_batches(c, 1, iter);
+    run_batches(c, 2, iter);
     double solve_ms = ctx->timer.stop_ms(c.s);
     check_sweeps(c);
     Scalars hs = read_scalars(c);
@@ -811,7 +1147,7 @@ static int inner_solve32(Ctx &c, const Structure &st, bool bicg, double eta, dou
     std::memset(&h, 0, sizeof(h));
     const bool keep = !bicg && s0_carry && *s0_carry > 0.0;
     h.small = kSmallSrc;
-    h.s0 = keep ? *s0_carry : kS0;
+    h.sk = keep ? *s0_carry : kS0;
     h.alf = 1.0;
     h.beto = 1.0;
     h.gam = 1.0;
@@ -824,40 +1160,42 @@ static int inner_solve32(Ctx &c, const Structure &st, bool bicg, double eta, dou
     k_zero<float><<<c.gv, 256, 0, c.s>>>(n, e);
     if (!keep) k_zero<float><<<c.gv, 256, 0, c.s>>>(n, p);
     if (!bicg) {
-        auto iter = [&]() {
+        auto precondition = [&](int first) {
             lu_launch32(c.s, st, a32, d32, small, r, z, c.sc, &c.sw, pf);
-            k_dot<float><<<c.gv, kRedBlock, 0, c.s>>>(n, r, z, c.sc, c.pa);
-            fin(c, kFinSk, c.gv, false);
-            k_p_update<float><<<c.gv, 256, 0, c.s>>>(n, p, z, c.sc);
-            spmv_launch32(c.s, 2, n, ptr, ja, a32, p, nullptr, p, q, c.pa, nullptr, c.sc);
-            fin(c, kFinAlf, gs, false);
-            k_pcg_xr<float, float><<<c.gv, kRedBlock, 0, c.s>>>(n, e, r, p, q, c.sc, c.pa, c.pb);
-            fin(c, kFinPcgEnd, c.gv, true);
+            k_dot<float><<<c.gf, kRedBlock, 0, c.s>>>(n, r, z, c.sc, c.pz);
+            k_cg_p<float, false><<<c.gf, kRedBlock, 0, c.s>>>(n, p, z, nullptr, c.sc, c.pv, c.gf, c.pz, c.gf, first);
         };
-        run_batches(c, 1, iter);
+        precondition(1);
+        run_batches(c, 2, [&]() {
+            spmv_launch32(c.s, 2, n, ptr, ja, a32, p, nullptr, p, q, c.pq, nullptr, c.sc);
+            const SpmvSums pq = spmv_sums(c, false);
+            k_cg_xr<float, float, false><<<c.gf, kRedBlock, 0, c.s>>>(n, e, r, p, q, nullptr, c.sc, pq.a, pq.n, c.pv);
+            precondition(0);
+        });
     } else {
         float *reso = reinterpret_cast<float *>(ws.tmp.get());   // n floats fit in n doubles
         float *uk = q, *vk = reinterpret_cast<float *>(ws.vk.get());
         k_copy<float><<<c.gv, 256, 0, c.s>>>(n, r, reso);
         k_zero<float><<<c.gv, 256, 0, c.s>>>(n, uk);
-        auto iter = [&]() {
-            k_dot<float><<<c.gv, kRedBlock, 0, c.s>>>(n, r, reso, c.sc, c.pa);
-            fin(c, kFinBet, c.gv, false);
-            k_bicg_p<float><<<c.gv, 256, 0, c.s>>>(n, p, r, uk, c.sc);
-            lu_launch32(c.s, st, a32, d32, small, p, z, c.sc, &c.sw, pf);
-            spmv_launch32(c.s, 2, n, ptr, ja, a32, z, nullptr, reso, uk, c.pa, nullptr, c.sc);
-            fin(c, kFinGam, gs, false);
-            k_bicg_xr1<float, float><<<c.gv, 256, 0, c.s>>>(n, e, r, z, uk, c.sc);
-            lu_launch32(c.s, st, a32, d32, small, r, z, c.sc, &c.sw, pf);
-            spmv_launch32(c.s, 3, n, ptr, ja, a32, z, nullptr, r, vk, c.pa, c.pb, c.sc);
-            fin(c, kFinAlfB, gs, true);
-            k_pcg_xr<float, float><<<c.gv, kRedBlock, 0, c.s>>>(n, e, r, z, vk, c.sc, c.pa, c.pb);
-            fin(c, kFinBicgEnd, c.gv, true);
+        auto direction = [&](int first) {
+            k_bi_p<float><<<c.gf, kRedBlock, 0, c.s>>>(n, p, r, uk, c.sc, c.pv, c.gf, first);
         };
-        run_batches(c, 1, iter);
+        k_first_dot<float><<<c.gf, kRedBlock, 0, c.s>>>(n, r, reso, nullptr, c.sc, c.pv);
+        direction(1);
+        run_batches(c, 2, [&]() {
+            lu_launch32(c.s, st, a32, d32, small, p, z, c.sc, &c.sw, pf);
+            spmv_launch32(c.s, 2, n, ptr, ja, a32, z, nullptr, reso, uk, c.pq, nullptr, c.sc);
+            const SpmvSums ur = spmv_sums(c, false);
+            k_bi_xr1<float, float><<<c.gf, kRedBlock, 0, c.s>>>(n, e, r, z, uk, c.sc, ur.a, ur.n);
+            lu_launch32(c.s, st, a32, d32, small, r, z, c.sc, &c.sw, pf);
+            spmv_launch32(c.s, 3, n, ptr, ja, a32, z, nullptr, r, vk, c.pq, c.pq2, c.sc);
+            const SpmvSums v = spmv_sums(c, true);
+            k_bi_xr2<float, float><<<c.gf, kRedBlock, 0, c.s>>>(n, e, r, z, vk, reso, c.sc, v.a, v.b, v.n, c.pv);
+            direction(0);
+        });
     }
     Scalars hs = read_scalars(c);
-    if (s0_carry) *s0_carry = bicg || hs.status != FC_OK ? 0.0 : hs.s0;
+    if (s0_carry) *s0_carry = bicg || hs.status != FC_OK ? 0.0 : hs.sk;
     return hs.iters;
 }
 
@@ -1011,7 +1349,7 @@ static int inner_fcg32(Ctx &c, const Structure &st, const PrecondHook &P, double
             iter();
         }
     };
-    run_batches(c, std::max(1, 4 / period), group);
+    run_batches(c, std::max(1, 2 / period), group);
     Scalars hs = read_scalars(c);
     iters += hs.iters;
     return hs.status;
@@ -1116,8 +1454,9 @@ constexpr size_t kNoAllocVec = sizeof(double) * (size_t)kNoAllocCells;
 constexpr int kNoAllocParts = kNoAllocCells / kSpmvRows > kMaxRedGrid ? kNoAllocCells / kSpmvRows : kMaxRedGrid;
 constexpr size_t kNoAllocPartBytes = sizeof(double) * (size_t)kNoAllocParts;
 constexpr size_t kNoAllocTail = 1024;   // Scalars, then three sums
+static_assert(kVecParts * kVecGrid <= kNoAllocParts, "scratch partials");
 static_assert(sizeof(Scalars) + 3 * sizeof(double) <= kNoAllocTail, "scratch tail");
-constexpr size_t kNoAllocBytes = 4 * kNoAllocVec + 2 * kNoAllocPartBytes + kNoAllocTail;
+constexpr size_t kNoAllocBytes = 4 * kNoAllocVec + 4 * kNoAllocPartBytes + kNoAllocTail;
 
 // Each GPU holds its own copy of this array until the process ends.  Host code
 // never uses its name as an address: it uses the per-device pointer that
@@ -1165,11 +1504,13 @@ fc_status solve_dpcg_noalloc(fc_context *ctx, int n, int nnz, const int *ioffset
     double *q = reinterpret_cast<double *>(b + 3 * kNoAllocVec);
     double *pa = reinterpret_cast<double *>(b + 4 * kNoAllocVec);
     double *pb = reinterpret_cast<double *>(b + 4 * kNoAllocVec + kNoAllocPartBytes);
-    Scalars *sc = reinterpret_cast<Scalars *>(b + 4 * kNoAllocVec + 2 * kNoAllocPartBytes);
-    double *sums = reinterpret_cast<double *>(b + 4 * kNoAllocVec + 2 * kNoAllocPartBytes + sizeof(Scalars));
+    double *pv = reinterpret_cast<double *>(b + 4 * kNoAllocVec + 2 * kNoAllocPartBytes);
+    double *pq = reinterpret_cast<double *>(b + 4 * kNoAllocVec + 3 * kNoAllocPartBytes);
+    Scalars *sc = reinterpret_cast<Scalars *>(b + 4 * kNoAllocVec + 4 * kNoAllocPartBytes);
+    double *sums = reinterpret_cast<double *>(b + 4 * kNoAllocVec + 4 * kNoAllocPartBytes + sizeof(Scalars));
     const double *a1 = a - 1;    // a1[k], k a 1-based position
     const int *ja1 = ja - 1;     // ja1[k] a 1-based column
-    Ctx c{ctx, s, nullptr, n, sc, pa, pb, red_grid(n), {}};
+    Ctx c{ctx, s, nullptr, n, sc, pa, pb, pv, nullptr, pq, nullptr, sums, red_grid(n), fused_grid(n), {}};
     SolveArgs args;
     args.sor = sor;
     args.nsw = nsw;
@@ -1182,7 +1523,22 @@ fc_status solve_dpcg_noalloc(fc_context *ctx, int n, int nnz, const int *ioffset
     spmv_launch64(s, 1, n, ioffset, ja1, a1, fi - 1, su, nullptr, r, nullptr, pa, pb, nullptr);
     fin(c, kFinRes0, seq_or(c, spmv_grid(n), 1, r, nullptr), true);
     const int gs = spmv_grid(n);
-    if (!read_done(c)) {
+    if (!read_done(c) && !ctx->reduce_seq) {
+        // the fused iterations of solve_pcg64, the diagonal in z
+        k_diag<<<c.gv, 256, 0, s>>>(n, a1, diag, z);
+        k_first_dot<double><<<c.gf, kRedBlock, 0, s>>>(n, r, r, z, sc, pv);
+        k_cg_p<double, true><<<c.gf, kRedBlock, 0, s>>>(n, p, r, z, sc, pv, c.gf, nullptr, 0, 1);
+        for (;;) {
+            for (int k = 0; k < 8; ++k) {
+                spmv_launch64(s, 2, n, ioffset, ja1, a1, p - 1, nullptr, p, q, nullptr, pq, nullptr, sc);
+                const SpmvSums v = spmv_sums(c, false);
+                k_cg_xr<double, double, true><<<c.gf, kRedBlock, 0, s>>>(n, fi, r, p, q, z, sc, v.a, v.n, pv);
+                k_cg_p<double, true><<<c.gf, kRedBlock, 0, s>>>(n, p, r, z, sc, pv, c.gf, nullptr, 0, 0);
+            }
+            FC_HIP_CHECK(hipGetLastError());
+            if (read_done(c)) break;
+        }
+    } else if (!read_done(c)) {
         for (;;) {
             for (int k = 0; k < 8; ++k) {
                 k_jacobi<double, double><<<c.gv, kRedBlock, 0, s>>>(n, r, a1, diag, z, sc, pa);
