@@ -1268,11 +1268,36 @@ __global__ void k_gnn_diag(int n, const float *__restrict__ x, const float *__re
         y[i] = DIV ? x[i] / d[i] : x[i] * d[i];
 }
 
+// Block sums of N values a thread (256 threads), column c's in FP64 to put(c, sum) by one
+// thread each: 32 columns at a time go through an LDS tile whose columns four threads sum a
+// quarter of each, so the block has two barriers per 32 columns (a block_sum per column had
+// three per column and took most of the first layer's and the decoder's time).
+constexpr int kColTile = 32, kColPad = 257;
+template <int N, class Put>
+__device__ inline void block_columns(const float *v, float *tile, Put &&put) {
+    const int t = threadIdx.x;
+#pragma unroll
+    for (int c0 = 0; c0 < N; c0 += kColTile) {
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < kColTile; ++c)
+            if (c0 + c < N) tile[c * kColPad + t] = v[c0 + c];
+        __syncthreads();
+        double s = 0.0;
+        const int c = (t >> 2) & (kColTile - 1), part = t & 3;
+        if (t < 4 * kColTile && c0 + c < N)
+            for (int k = 0; k < 64; ++k) s += (double)tile[c * kColPad + 4 * k + part];
+        s += __shfl_down(s, 2, 4);
+        s += __shfl_down(s, 1, 4);
+        if (t < 4 * kColTile && part == 0 && c0 + c < N) put(c0 + c, s);
+    }
+}
+
 // decoder: dy = s dz ; dh4 = dy w_dec ; partials of d w_dec (32) and d b_dec (1) per block
 __global__ __launch_bounds__(256) void k_gnn_dec_bwd(int n, const bf16_t *__restrict__ h4, const float *__restrict__ dz,
                                                      const float *__restrict__ s_ptr, const bf16_t *__restrict__ w,
                                                      float *__restrict__ dh, float *__restrict__ part) {
-    __shared__ double sh[256 / 64];
+    __shared__ float tile[kColTile * kColPad];
     const float sv = s_ptr[0];
     float acc[H + 1];
 #pragma unroll
@@ -1288,10 +1313,7 @@ __global__ __launch_bounds__(256) void k_gnn_dec_bwd(int n, const bf16_t *__rest
         }
         acc[H] += dy;
     }
-    for (int c = 0; c <= H; ++c) {
-        double v = block_sum<256>((double)acc[c], sh);
-        if (threadIdx.x == 0) part[(size_t)blockIdx.x * (H + 1) + c] = (float)v;
-    }
+    block_columns<H + 1>(acc, tile, [&](int c, double v) { part[(size_t)blockIdx.x * (H + 1) + c] = (float)v; });
 }
 
 // Layer backward, part 1 (one wave per 64 cells, chunks strided over the grid):
@@ -1330,8 +1352,6 @@ __global__ __launch_bounds__(256) void k_gnn_bwd1(int n, GnnEll E, const float *
         bf16x4 bfr[4][2];
         load_b_frags(lw, lane, bfr);
         layer_gemm(X, bfr, lane, acc);
-        // output tile goes through smd's rows is too small: use a register pass instead --
-        // each lane needs out[node=lane][c]; route via the X tile after the weight-grad GEMM
         __syncthreads();
         // d_out needs out of the lane's own cell: stage out in the D tile region as FP32? D is
         // 64 x 40 bf16 = 5120 bytes < 64 x 32 floats; so stage out in X temporarily (X is
@@ -1410,12 +1430,21 @@ __global__ __launch_bounds__(256) void k_gnn_bwd1(int n, GnnEll E, const float *
                     for (int j = 0; j < 4; ++j)
                         C[(16 * t + 4 * q + j) * kLdC + nn * 16 + r16] = iacc[t][2 * half + nn][j];
             __syncthreads();
-            if (valid) {
+            // eight lanes a row: whole rows per store
 #pragma unroll
-                for (int c = 0; c < H; ++c) {
-                    const float v = C[lane * kLdC + c];
-                    if (half == 0) dh_part[(size_t)node * H + c] = dh_out[(size_t)node * H + c] + v;
-                    else dagg[(size_t)node * H + c] = v;
+            for (int it = 0; it < 8; ++it) {
+                const int rr = 8 * it + (lane >> 3), c4 = 4 * (lane & 7);
+                const int cell = chunk * 256 + wv * 64 + rr;
+                if (cell < n) {
+                    float4 v = *reinterpret_cast<const float4 *>(C + rr * kLdC + c4);
+                    const size_t o = (size_t)cell * H + c4;
+                    if (half == 0) {
+                        const float4 g = *reinterpret_cast<const float4 *>(dh_out + o);
+                        v = make_float4(g.x + v.x, g.y + v.y, g.z + v.z, g.w + v.w);
+                        *reinterpret_cast<float4 *>(dh_part + o) = v;
+                    } else {
+                        *reinterpret_cast<float4 *>(dagg + o) = v;
+                    }
                 }
             }
             __syncthreads();
@@ -1440,87 +1469,131 @@ __global__ __launch_bounds__(256) void k_gnn_bwd1(int n, GnnEll E, const float *
     }
 }
 
-// Layer backward, part 2 (one thread per cell j): messages flow back along the
-// transposed entries, dh_in_j = dh_part_j + sum_{k in row j} c_{t(k)} d_agg_{ja[k]},
-// and the gate gradient dc_t = d_agg_i . h_j.  First layer: encoder gradients.
+// Layer backward, part 2 (eight lanes per cell j, four channels each, so that a row is
+// read and written whole): messages flow back along the transposed entries, dh_in_j =
+// dh_part_j + sum_{k in row j} c_{t(k)} d_agg_{ja[k]}, and the gate gradient dc_t =
+// d_agg_i . h_j (linear in the lanes' parts, which are added at the end).  First layer:
+// encoder gradients.  Bound by the rows gathered (6 x 128 B a cell): 33 us at
+// 64^3, with a thread per cell and a wave per SIMD 48 us (81 us in the first layer).
 template <bool FIRST>
 __global__ __launch_bounds__(256) void k_gnn_bwd2(int n, GnnEll E, const float *__restrict__ u,
                                                   const bf16_t *__restrict__ h_in, const float *__restrict__ dh_part,
                                                   const float *__restrict__ dagg, const bf16_t *__restrict__ w,
                                                   int layer, float *__restrict__ dh_in, float *__restrict__ gpart) {
-    __shared__ double sh[256 / 64];
+    __shared__ double sh[4][3 + 2 * H];
     const bf16_t *lw = w + kGnnOffLayer0 + layer * kGnnLayerStride;
     const float g0 = bf2f(lw[2 * H * H + H]), g1 = bf2f(lw[2 * H * H + H + 1]), g2 = bf2f(lw[2 * H * H + H + 2]);
-    float dg[3] = {0.f, 0.f, 0.f};
-    float denc[2 * H];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, q = lane & 7, c0 = 4 * q;
+    float ew[4], eb[4];
 #pragma unroll
-    for (int c = 0; c < 2 * H; ++c) denc[c] = 0.f;
-    for (int j = blockIdx.x * 256 + threadIdx.x; j < n; j += gridDim.x * 256) {
-        float hj[H], d[H], pre[H];
+    for (int t = 0; t < 4; ++t) {
+        ew[t] = bf2f(w[kGnnOffEncW + c0 + t]);
+        eb[t] = bf2f(w[kGnnOffEncB + c0 + t]);
+    }
+    float dg[3] = {0.f, 0.f, 0.f}, denc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int j = blockIdx.x * 32 + (threadIdx.x >> 3); j < n; j += gridDim.x * 32) {
+        float hj[4], pre[4], uj = 0.f;
         if (FIRST) {
-            const float uj = u[j];
+            uj = u[j];
 #pragma unroll
-            for (int c = 0; c < H; ++c) {
-                pre[c] = bf2f(w[kGnnOffEncW + c]) * uj + bf2f(w[kGnnOffEncB + c]);
-                hj[c] = bfround(fmaxf(pre[c], 0.f));
+            for (int t = 0; t < 4; ++t) {
+                pre[t] = ew[t] * uj + eb[t];
+                hj[t] = bfround(fmaxf(pre[t], 0.f));
             }
         } else {
-            load_hrow(h_in + (size_t)j * H, hj);
+            // channels 4q .. 4q + 3 of a stored row: half q / 4 of its group q % 4
+            const uint2 raw = *reinterpret_cast<const uint2 *>(h_in + (size_t)j * H + 8 * (q & 3) + 4 * (q >> 2));
+            hj[0] = __uint_as_float(raw.x << 16);
+            hj[1] = __uint_as_float(raw.x & 0xffff0000u);
+            hj[2] = __uint_as_float(raw.y << 16);
+            hj[3] = __uint_as_float(raw.y & 0xffff0000u);
         }
-#pragma unroll
-        for (int c = 0; c < H; ++c) d[c] = dh_part[(size_t)j * H + c];
+        const float4 dp = *reinterpret_cast<const float4 *>(dh_part + (size_t)j * H + c0);
+        float d[4] = {dp.x, dp.y, dp.z, dp.w};
         const int cnt = E.cnt[j];
         for (int k = 0; k < cnt; ++k) {
             // slot k of cell j: neighbour i, and the features of entry (i, j) of row i
             const int i = E.nbr[(size_t)k * E.n + j];
             const uint32_t e = E.eft[(size_t)k * E.n + j];
+            const float4 da = *reinterpret_cast<const float4 *>(dagg + (size_t)i * H + c0);
             const float e1 = bf2f((bf16_t)(e & 0xffffu)), e2 = bf2f((bf16_t)(e >> 16));
             const float ct = edge_gate(g0, g1, g2, e);
-            float dc = 0.f;
-#pragma unroll
-            for (int c = 0; c < H; ++c) {
-                const float da = dagg[(size_t)i * H + c];
-                d[c] += ct * da;
-                dc += da * hj[c];
-            }
+            d[0] += ct * da.x;
+            d[1] += ct * da.y;
+            d[2] += ct * da.z;
+            d[3] += ct * da.w;
+            const float dc = (da.x * hj[0] + da.y * hj[1]) + (da.z * hj[2] + da.w * hj[3]);
             dg[0] += dc;
             dg[1] += dc * e1;
             dg[2] += dc * e2;
         }
         if (!FIRST) {
-#pragma unroll
-            for (int c = 0; c < H; ++c) dh_in[(size_t)j * H + c] = d[c];
+            *reinterpret_cast<float4 *>(dh_in + (size_t)j * H + c0) = make_float4(d[0], d[1], d[2], d[3]);
         } else {
-            const float uj = u[j];
 #pragma unroll
-            for (int c = 0; c < H; ++c) {
-                const float dp_ = pre[c] > 0.f ? d[c] : 0.f;
-                denc[c] += dp_ * uj;
-                denc[H + c] += dp_;
+            for (int t = 0; t < 4; ++t) {
+                const float dp_ = pre[t] > 0.f ? d[t] : 0.f;
+                denc[t] += dp_ * uj;
+                denc[4 + t] += dp_;
             }
         }
     }
-    const int stride = 3 + 2 * H;
+    // block sums in FP64: the lanes of one channel group, then the four waves
+#pragma unroll
     for (int c = 0; c < 3; ++c) {
-        double v = block_sum<256>((double)dg[c], sh);
-        if (threadIdx.x == 0) gpart[(size_t)blockIdx.x * stride + c] = (float)v;
+        const double v = wave_sum((double)dg[c]);
+        if (lane == 0) sh[wv][c] = v;
     }
     if (FIRST) {
-        for (int c = 0; c < 2 * H; ++c) {
-            double v = block_sum<256>((double)denc[c], sh);
-            if (threadIdx.x == 0) gpart[(size_t)blockIdx.x * stride + 3 + c] = (float)v;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            double v = (double)denc[t];
+#pragma unroll
+            for (int off = 32; off >= 8; off >>= 1) v += __shfl_down(v, off, kWave);
+            if (lane < 8) sh[wv][3 + (t >> 2) * H + c0 + (t & 3)] = v;
         }
     }
+    __syncthreads();
+    const int stride = 3 + 2 * H;
+    const int c = threadIdx.x;
+    if (c < (FIRST ? stride : 3))
+        gpart[(size_t)blockIdx.x * stride + c] = (float)((sh[0][c] + sh[1][c]) + (sh[2][c] + sh[3][c]));
 }
 
-// grad[off + c] += sum_p part[p * stride + col0 + c], c < width (fixed order over p)
-__global__ void k_gnn_reduce(int nparts, int stride, int col0, int width, const float *__restrict__ part,
-                             float *__restrict__ grad, int off) {
-    int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= width) return;
+// grad[off + c] += sum_p part[p * stride + col0 + c], c < width (fixed order over p): a
+// block takes 64 columns, sixteen waves a sixteenth of the partials each, eight rows in
+// flight: 9.5 us for 2,048 rows of 2,080 columns (one thread per column adding 1,024 rows
+// one by one took 134 us a launch, ten launches a gradient)
+constexpr int kReduceRows = 16;
+__global__ __launch_bounds__(64 * kReduceRows) void k_gnn_reduce(int nparts, int stride, int col0, int width,
+                                                                 const float *__restrict__ part,
+                                                                 float *__restrict__ grad, int off) {
+    __shared__ double sh[kReduceRows][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int c = blockIdx.x * 64 + lane;
+    const int per = (nparts + kReduceRows - 1) / kReduceRows;
+    const int p1 = min(nparts, (w + 1) * per);
     double s = 0.0;
-    for (int p = 0; p < nparts; ++p) s += part[(size_t)p * stride + col0 + c];
-    grad[off + c] += (float)s;
+    if (c < width) {
+        const float *src = part + col0 + c;
+        int p = w * per;
+        for (; p + 8 <= p1; p += 8) {
+            float v[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[k] = src[(size_t)(p + k) * stride];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) s += (double)v[k];
+        }
+        for (; p < p1; ++p) s += (double)src[(size_t)p * stride];
+    }
+    sh[w][lane] = s;
+    __syncthreads();
+    if (w == 0 && c < width) {
+        double t = 0.0;
+#pragma unroll
+        for (int k = 0; k < kReduceRows; ++k) t += sh[k][lane];
+        grad[off + c] += (float)t;
+    }
 }
 
 __global__ void k_gnn_adam(int np, float *__restrict__ th, const float *__restrict__ g, float *__restrict__ m,
@@ -1755,7 +1828,9 @@ struct fc_gnn {
 
 namespace {
 
-constexpr int kBwdGrid = 256;   // blocks of the backward kernels (grid-strided over cells)
+// blocks of the backward kernels (grid-strided over cells): what fits the CUs at once
+// (layer part 1 holds 57 KB of LDS)
+constexpr int kBwdGrid = 512, kBwd2Grid = 2048, kDecGrid = 1024;
 
 void gnn_normalise(fc_gnn *net, hipStream_t s, const GnnGraph &g, const float *r, const Scalars *sc) {
     const int gp = std::min(kMaxRedGrid, grid_for(g.n, 256));
@@ -1928,6 +2003,10 @@ void gnn_forward(fc_gnn *net, hipStream_t s, const GnnGraph &g, const float *r, 
     FC_HIP_CHECK(hipGetLastError());
 }
 
+void reduce_parts(hipStream_t s, int nparts, int stride, int col0, int width, const float *part, float *grad, int off) {
+    k_gnn_reduce<<<grid_for(width, 64), 64 * kReduceRows, 0, s>>>(nparts, stride, col0, width, part, grad, off);
+}
+
 // Loss of one pair and its gradient, accumulated into net->grad (scaled by coef_batch).
 void gnn_backward_pair(fc_gnn *net, hipStream_t s, GnnGraph &g, const float *r, const float *e, double eAe,
                        float batch, double *loss_dev_slot) {
@@ -1978,10 +2057,10 @@ void gnn_backward_pair(fc_gnn *net, hipStream_t s, GnnGraph &g, const float *r, 
     // decoder
     const bf16_t *w = net->wbf.as<bf16_t>();
     float *grad = net->grad.as<float>();
-    net->gpart.ensure(sizeof(float) * (size_t)kBwdGrid * (3 + 2 * kGnnH + 64));
-    k_gnn_dec_bwd<<<kBwdGrid, 256, 0, s>>>(n, net->h[kGnnL].as<bf16_t>(), net->dz.as<float>(), net->s.as<float>(), w,
+    net->gpart.ensure(sizeof(float) * (size_t)kBwd2Grid * (3 + 2 * kGnnH));
+    k_gnn_dec_bwd<<<kDecGrid, 256, 0, s>>>(n, net->h[kGnnL].as<bf16_t>(), net->dz.as<float>(), net->s.as<float>(), w,
                                            net->dha.as<float>(), net->gpart.as<float>());
-    k_gnn_reduce<<<1, 64, 0, s>>>(kBwdGrid, kGnnH + 1, 0, kGnnH + 1, net->gpart.as<float>(), grad, kGnnOffDecW);
+    reduce_parts(s, kDecGrid, kGnnH + 1, 0, kGnnH + 1, net->gpart.as<float>(), grad, kGnnOffDecW);
     // layers, last to first
     net->wpart.ensure(sizeof(float) * (size_t)kBwdGrid * kWaves * (2 * kGnnH * kGnnH + kGnnH));
     const GnnEll E = ell_of(g);
@@ -1998,19 +2077,18 @@ void gnn_backward_pair(fc_gnn *net, hipStream_t s, GnnGraph &g, const float *r, 
                                                        net->wpart.as<float>());
         const int loff = kGnnOffLayer0 + l * kGnnLayerStride;
         const int wstride = 2 * kGnnH * kGnnH + kGnnH;
-        k_gnn_reduce<<<grid_for(wstride, 256), 256, 0, s>>>(kBwdGrid * kWaves, wstride, 0, wstride,
-                                                            net->wpart.as<float>(), grad, loff);
+        reduce_parts(s, kBwdGrid * kWaves, wstride, 0, wstride, net->wpart.as<float>(), grad, loff);
         // dh_in of this layer goes into dh_out's buffer (no longer needed)
         if (l == 0)
-            k_gnn_bwd2<true><<<kBwdGrid, 256, 0, s>>>(n, E, u, hin, dpart, net->dagg.as<float>(), w, l, dh_out,
+            k_gnn_bwd2<true><<<kBwd2Grid, 256, 0, s>>>(n, E, u, hin, dpart, net->dagg.as<float>(), w, l, dh_out,
                                                       net->gpart.as<float>());
         else
-            k_gnn_bwd2<false><<<kBwdGrid, 256, 0, s>>>(n, E, u, hin, dpart, net->dagg.as<float>(), w, l, dh_out,
+            k_gnn_bwd2<false><<<kBwd2Grid, 256, 0, s>>>(n, E, u, hin, dpart, net->dagg.as<float>(), w, l, dh_out,
                                                        net->gpart.as<float>());
         const int gstride = 3 + 2 * kGnnH;
-        k_gnn_reduce<<<1, 64, 0, s>>>(kBwdGrid, gstride, 0, 3, net->gpart.as<float>(), grad, loff + 2 * kGnnH * kGnnH + kGnnH);
+        reduce_parts(s, kBwd2Grid, gstride, 0, 3, net->gpart.as<float>(), grad, loff + 2 * kGnnH * kGnnH + kGnnH);
         if (l == 0)
-            k_gnn_reduce<<<1, 64, 0, s>>>(kBwdGrid, gstride, 3, 2 * kGnnH, net->gpart.as<float>(), grad, kGnnOffEncW);
+            reduce_parts(s, kBwd2Grid, gstride, 3, 2 * kGnnH, net->gpart.as<float>(), grad, kGnnOffEncW);
     }
     FC_HIP_CHECK(hipGetLastError());
 }

@@ -235,6 +235,31 @@ def test_loss_and_gradient_match_oracle(ctx, small, pseed, smooth):
     net.close()
 
 
+@pytest.mark.parametrize("dims", [(2, 1, 1), (16, 16, 1), (257, 1, 1), (41, 41, 40), (51, 51, 51)])
+def test_gradient_over_cell_counts(ctx, dims):
+    """The backward kernels and their reductions where a cell count can go wrong: less than a
+    wave, one block of 256 and one cell more, and the second pass over the grid of the layers'
+    second part (65,536 cells) and first part (131,072 cells).  Tolerances as above."""
+    m = M.hex_box(dims[0], dims[1], dims[2], perturb=0.1, seed=3)
+    geo, csr, a, A, graph, feats = gnn_case(m)
+    s = _system(m, ctx)
+    th = _params(9)
+    net = gnn.Network(th, ctx)
+    try:
+        rng = np.random.default_rng(m.n_cells)
+        r = rng.standard_normal(m.n_cells).astype(np.float32)
+        e = rng.standard_normal(m.n_cells).astype(np.float32)
+        loss_gpu, g_gpu = net.loss_grad(s, r, e)
+        loss_ref, g_ref = G.loss_and_grad(th, graph, A, [(r, e)], bf=True)
+        rel = np.linalg.norm(g_gpu - g_ref) / np.linalg.norm(g_ref)
+        print(f"{dims}: loss {abs(loss_gpu - loss_ref) / abs(loss_ref):.2e} gradient {rel:.2e}")
+        assert abs(loss_gpu - loss_ref) <= LOSS_RTOL * abs(loss_ref)
+        assert rel < GRAD_RTOL, rel
+    finally:
+        net.close()
+        s.close()
+
+
 def test_samples_are_ic0_pcg_iterates_of_the_homogeneous_system(ctx, small):
     """r = A e for every pair; e starts standard normal and gets smoother with the iteration count
     (the Rayleigh quotient e^T A^2 e / e^T A e falls as IC(0)-PCG removes the rough components)."""
