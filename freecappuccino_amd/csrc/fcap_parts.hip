@@ -2,7 +2,7 @@
 // into parts and windows, the packed factor, and the sweep kernel.
 //
 // A sweep is a chain of levels (3N - 2 on an N^3 box), so its time is the chain's
-// latency, not its bytes.  One persistent wave computes a part 64 rows (a window)
+// latency, not its bytes.  One persistent workgroup computes a part 64 rows (a window)
 // at a time; what it reads of its own part comes from LDS, so the chain inside a
 // part costs LDS round trips, and only the chain from part to part costs round
 // trips through the coherent level of the memory system.  The parts are therefore
@@ -150,29 +150,34 @@ struct PartView {
     const unsigned char *step;
 };
 
-// A workgroup of four waves computes a part.  Wave 0 does nothing but the chain: per
-// window it reads its operands and the inputs' values from LDS, forms the rows'
-// values, puts them into the ring and publishes them.  Waves 1 to 3 feed it, each a
-// batch of kBatch windows in turn: operands, right-hand side and the inputs from
-// other parts from memory into the stage, kStage windows ahead at most; they also
-// store what need not be early (the result in row order, the marks for the next
-// sweep).  A wave issues one instruction in four cycles at most: with one wave per
-// part doing all of it a window took 330 ns (of about 110 instructions), with the
-// chain apart 160 ns.
+// A workgroup computes a part.  Wave 0 does nothing but the chain: per window it reads
+// its operands and the inputs' values from LDS, forms the rows' values, puts them into
+// the ring and publishes them.  The pollers fetch the inputs from other parts, each a
+// window in turn.  The feeders stage the windows, each kBatch in turn: operands and
+// right-hand side from memory, kStage windows ahead at most; they also store what need
+// not be early (the result in row order, the marks for the next sweep).  A wave issues
+// one instruction in four cycles at most: with one wave per part doing all of it a window
+// took 330 ns (of about 110 instructions), with the chain apart 160 ns.  The polls are
+// apart from the feeders because memory answers a wave in order: a poll repeated behind
+// the prefetch of the next windows waits for that prefetch, which cost about 1 us more at
+// each entry of the chain into another part.
 //
-// What bounds a sweep: the windows along its longest chain, 160 ns each, and a round
-// trip of about 2.5 us through the coherent level of the memory system where the chain
-// enters another part; from some 5 M rows also the bytes (about 80 a row at W = 3 in
-// FP64, 165 us for the 192^3 box with every input there).  Per sweep, before (runs of
-// 4,096 rows, one wave each) and now: 40^3 box 107 and 45 us, 96 x 80 x 72 459 and 98,
-// 128^3 430 and 190, 192^3 728 and 315, 163 x 75 x 1 78 and 49.  Batches of 1, 2, 3 and
-// 4 windows at 128^3: 206, 192, 190, 196 us; at 163 x 75 x 1: 63, 52, 49, 48.
+// What bounds a sweep: the windows along its longest chain, 160 to 180 ns each, and about
+// 2 us where the chain enters another part (a value stored by one workgroup is seen by
+// another's poll 0.6 to 0.75 us later); from some 5 M rows also the bytes (about 80 a row
+// at W = 3 in FP64, 165 us for the 192^3 box with every input there).  Per sweep, with the
+// polls in three feeders and now: 40^3 box 45 and 36 us, 96 x 80 x 72 98 and 77, 128^3 190
+// and 139, 192^3 315 and 261, 163 x 75 x 1 49 and 43.  Feeders x batch, pollers at 128^3:
+// 3 x 3, 2 pollers of 4 windows 173; 6 x 2, 2 of 4 167; 6 x 2, 4 of 2 142; 6 x 2, 6 of 1
+// 139; 6 x 2, 8 of 1 142; 4 x 3, 11 of 1 148 us.
 template <int W> struct PartShape {
-    static constexpr int kFeeders = 3;
-    static constexpr int kBatch = W <= 4 ? 3 : 2;
+    // waves that stage windows and windows a turn of one; waves that poll for inputs.  Thirteen
+    // waves leave 128 registers a lane (W = 3 takes 106), twelve 168, eight 256.
+    static constexpr int kFeeders = W <= 4 ? 6 : 3, kBatch = 2;
+    static constexpr int kPollers = W <= 3 ? 6 : W <= 4 ? 5 : 4;
     static constexpr int kStage = kFeeders * kBatch;
+    static constexpr int kBlock = 64 * (1 + kPollers + kFeeders);
 };
-constexpr int kPartBlock = 64 * (1 + PartShape<3>::kFeeders);
 
 template <class T, int W>
 struct PartLds {
@@ -191,7 +196,8 @@ struct PartLds {
     // the ring of the part's values, a zero (padding entries), and the staged inputs from
     // other parts: everything a staged code points to (byte offsets)
     T x[kRing + 2 + K * W * 64];
-    int flag[K];     // window index + 1 when the stage holds it
+    int fed[K];      // window index + 1 when the stage holds its operands
+    int flag[K];     // the same when its inputs from other parts are there too
     int progress;    // windows the chain has finished
     int give_up, ticket;
 };
@@ -226,12 +232,6 @@ struct PartRow {
     T val[W + 1];      // the entries' values, then the pivot
     int step;
 };
-template <class T, int W>
-struct PartIn {
-    T rhs;
-    typename SfBits<T>::U pb[W];
-};
-
 template <class T>
 struct PartRun {
     int w0, nw;   // the part's first window and its windows
@@ -248,19 +248,27 @@ struct PartRun {
     }
 };
 
-// polls of the inputs from other parts that are not there yet
+// A window's inputs from other parts: their codes (a code < 0 names a packed slot of
+// another part) and the bits found there so far.
 template <class T, int W>
-__device__ __forceinline__ void part_poll(PartIn<T, W> &I, const PartRow<T, W> &o, const T *out) {
+struct PartIn {
+    int code[W];
+    typename SfBits<T>::U pb[W];
+};
+
+// polls of the inputs that are not there yet
+template <class T, int W>
+__device__ __forceinline__ void part_poll(PartIn<T, W> &I, const T *out) {
 #pragma unroll
     for (int k = 0; k < W; ++k)
-        if (o.code[k] < 0 && I.pb[k] == SfBits<T>::kMark) I.pb[k] = sf_load_bits(out + (o.code[k] & 0x7fffffff));
+        if (I.code[k] < 0 && I.pb[k] == SfBits<T>::kMark) I.pb[k] = sf_load_bits(out + (I.code[k] & 0x7fffffff));
 }
 
 template <class T, int W>
-__device__ __forceinline__ bool part_missing(const PartIn<T, W> &I, const PartRow<T, W> &o) {
+__device__ __forceinline__ bool part_missing(const PartIn<T, W> &I) {
     bool miss = false;
 #pragma unroll
-    for (int k = 0; k < W; ++k) miss |= o.code[k] < 0 && I.pb[k] == SfBits<T>::kMark;
+    for (int k = 0; k < W; ++k) miss |= I.code[k] < 0 && I.pb[k] == SfBits<T>::kMark;
     return __any(miss);
 }
 
@@ -307,7 +315,8 @@ __device__ __forceinline__ void stage_put(typename PartLds<T, W>::Slot &s, int l
 template <class T, int W, bool BWD>
 __device__ __forceinline__ void part_feed(const PartRun<T> &R, PartLds<T, W> &L, int feeder) {
     using S = PartShape<W>;
-    constexpr int B = S::kBatch, K = S::kStage, V = PartLds<T, W>::V;
+    using U = typename SfBits<T>::U;
+    constexpr int B = S::kBatch, K = S::kStage;
     const int lane = threadIdx.x & 63;
     PartRow<T, W> cur[B], nxt[B];
     int row[B];            // rows of the batch before the current one
@@ -325,65 +334,38 @@ __device__ __forceinline__ void part_feed(const PartRun<T> &R, PartLds<T, W> &L,
         row[u] = 0;
     }
     for (; j0 < R.nw; j0 += K) {
-        PartIn<T, W> in[B];
+        T rhs[B];
 #pragma unroll
-        for (int u = 0; u < B; ++u) {
-            in[u].rhs = BWD ? R.in[(size_t)R.template at<BWD>(j0 + u) * 64 + lane] : R.in[cur[u].code[W]];
-#pragma unroll
-            for (int k = 0; k < W; ++k) in[u].pb[k] = SfBits<T>::kMark;
-            part_poll<T, W>(in[u], cur[u], R.out);
-        }
+        for (int u = 0; u < B; ++u)
+            rhs[u] = BWD ? R.in[(size_t)R.template at<BWD>(j0 + u) * 64 + lane] : R.in[cur[u].code[W]];
 #pragma unroll
         for (int u = 0; u < B; ++u) load(nxt[u], j0 + K + u);
 #pragma unroll
         for (int u = 0; u < B; ++u) {
             const int j = j0 + u;
             if (j < R.nw) {
-                // The inputs, polled again until they are there, with those of the batch's
-                // later windows; by the first feeder alone while the part has not begun: a
-                // part that waits must not flood the memory system
-                if (part_missing<T, W>(in[u], cur[u])) {
-                    const unsigned long long t0 = wall_clock64();
-                    do {
-                        if (j > 0 && lds_get(&L.flag[0]) == 0) {
-                            __builtin_amdgcn_s_sleep(1);
-                            if (lds_get(&L.give_up)) return;
-                            continue;
-                        }
+                T vals[W + 2];
 #pragma unroll
-                        for (int v = 0; v < B; ++v)
-                            if (v >= u) part_poll<T, W>(in[v], cur[v], R.out);
-                        const bool late = __any(wall_clock64() - t0 > R.limit ||
-                                                __hip_atomic_load(&R.sf->abort, __ATOMIC_RELAXED,
-                                                                  __HIP_MEMORY_SCOPE_AGENT) != 0);
-                        if (late || lds_get(&L.give_up)) {
-                            if (late)
-                                __hip_atomic_store(&R.sf->abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                            lds_set(&L.give_up, 1);
-                            return;
-                        }
-                    } while (part_missing<T, W>(in[u], cur[u]));
-                }
+                for (int k = 0; k < W; ++k) vals[k] = cur[u].val[k];
+                vals[W] = cur[u].val[W];
+                vals[W + 1] = BWD ? rhs[u] / (cur[u].val[W] + R.small) : rhs[u];
                 // room in the stage
                 if (!part_finished(L, j - K)) return;
                 const int slot = j % K;
                 const int xbase = kRing + 2 + slot * W * 64 + lane;
                 int ints[W + 1];
-                T vals[W + 2];
 #pragma unroll
                 for (int k = 0; k < W; ++k) {
                     const bool outside = cur[u].code[k] < 0;
                     ints[k] = (int)sizeof(T) * (outside ? xbase + k * 64 : cur[u].code[k]);
-                    L.x[xbase + k * 64] = __builtin_bit_cast(T, in[u].pb[k]);
-                    vals[k] = cur[u].val[k];
+                    // the slot's code until the poller puts its value there
+                    reinterpret_cast<U *>(L.x)[xbase + k * 64] = (U)(unsigned)cur[u].code[k];
                 }
                 const int top = __builtin_amdgcn_readlane(cur[u].step, 63);
                 ints[W] = (BWD ? top - cur[u].step : cur[u].step) | top << 8;
-                vals[W] = cur[u].val[W];
-                vals[W + 1] = BWD ? in[u].rhs / (cur[u].val[W] + R.small) : in[u].rhs;
                 stage_put<T, W>(L.stage[slot], lane, ints, vals);
                 lds_order();
-                lds_set(&L.flag[slot], j + 1);
+                lds_set(&L.fed[slot], j + 1);
             } else if (before >= 0 && !part_finished(L, j - K)) {
                 return;
             }
@@ -405,6 +387,54 @@ __device__ __forceinline__ void part_feed(const PartRun<T> &R, PartLds<T, W> &L,
             if (!part_finished(L, before + u)) return;
             part_retire<T, W, BWD>(R, L, before + u, row[u]);
         }
+    }
+}
+
+// The inputs from other parts, a window per turn of a poller: polled until they are there
+// and put where the staged codes point to.  By the first poller alone while the part has
+// not begun: a part that waits must not flood the memory system.  The window's operands
+// are waited for here (fed), so the chain waits for one flag only.
+template <class T, int W>
+__device__ __forceinline__ void part_inputs(const PartRun<T> &R, PartLds<T, W> &L, int poller) {
+    using U = typename SfBits<T>::U;
+    constexpr int K = PartShape<W>::kStage;
+    const int lane = threadIdx.x & 63;
+    for (int j = poller; j < R.nw; j += PartShape<W>::kPollers) {
+        const int slot = j % K, xbase = kRing + 2 + slot * W * 64 + lane;
+        while (lds_get(&L.fed[slot]) != j + 1)
+            if (lds_get(&L.give_up)) return;
+        lds_order();
+        PartIn<T, W> in;
+#pragma unroll
+        for (int k = 0; k < W; ++k) {
+            in.code[k] = (int)reinterpret_cast<const U *>(L.x)[xbase + k * 64];
+            in.pb[k] = SfBits<T>::kMark;
+        }
+        if (part_missing<T, W>(in)) {
+            const unsigned long long t0 = wall_clock64();
+            int polls = 0;
+            do {
+                bool late = false;
+                if (j > 0 && lds_get(&L.flag[0]) == 0) {
+                    __builtin_amdgcn_s_sleep(1);
+                } else {
+                    part_poll<T, W>(in, R.out);
+                    if ((++polls & 7) == 0)
+                        late = __any(wall_clock64() - t0 > R.limit ||
+                                     __hip_atomic_load(&R.sf->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0);
+                }
+                if (late || lds_get(&L.give_up)) {
+                    if (late) __hip_atomic_store(&R.sf->abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    lds_set(&L.give_up, 1);
+                    return;
+                }
+            } while (part_missing<T, W>(in));
+        }
+#pragma unroll
+        for (int k = 0; k < W; ++k)
+            if (in.code[k] < 0) L.x[xbase + k * 64] = __builtin_bit_cast(T, in.pb[k]);
+        lds_order();
+        lds_set(&L.flag[slot], j + 1);
     }
 }
 
@@ -539,7 +569,7 @@ __device__ __forceinline__ void part_chain(const PartRun<T> &R, PartLds<T, W> &L
 // k_sweep_syncfree forms it: padding entries subtract 0 * 0, which leaves every value
 // as it is.
 template <class T, int W, bool BWD>
-__global__ __launch_bounds__(kPartBlock) void k_sweep_parts(int nparts, PartView P, const int *__restrict__ win_ptr,
+__global__ __launch_bounds__(PartShape<W>::kBlock) void k_sweep_parts(int nparts, PartView P, const int *__restrict__ win_ptr,
                                                             const T *__restrict__ vals, const T *in, T small, T *out,
                                                             T *mk, T *z, SyncFree *sf,
                                                             const Scalars *__restrict__ sc) {
@@ -565,7 +595,10 @@ __global__ __launch_bounds__(kPartBlock) void k_sweep_parts(int nparts, PartView
             L.ticket = (int)__hip_atomic_fetch_add(&sf->ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             L.progress = 0;
         }
-        if (threadIdx.x < (unsigned)PartShape<W>::kStage) L.flag[threadIdx.x] = 0;
+        if (threadIdx.x < (unsigned)PartShape<W>::kStage) {
+            L.fed[threadIdx.x] = 0;
+            L.flag[threadIdx.x] = 0;
+        }
         __syncthreads();
         const int t = __builtin_amdgcn_readfirstlane(L.ticket);
         if ((unsigned)t >= (unsigned)nparts) break;
@@ -574,8 +607,10 @@ __global__ __launch_bounds__(kPartBlock) void k_sweep_parts(int nparts, PartView
         R.nw = win_ptr[part + 1] - R.w0;
         if (wave == 0)
             part_chain<T, W, BWD>(R, L);
+        else if (wave <= PartShape<W>::kPollers)
+            part_inputs<T, W>(R, L, wave - 1);
         else
-            part_feed<T, W, BWD>(R, L, wave - 1);
+            part_feed<T, W, BWD>(R, L, wave - 1 - PartShape<W>::kPollers);
         __syncthreads();
         if (L.give_up) break;
     }
@@ -765,8 +800,8 @@ void lu_parts_w(hipStream_t s, const Structure &st, const PackedFactor<T> &pf, T
     const PartView F{st.pt_npk, st.pt_codes_f.as<int>(), st.pt_step.as<unsigned char>()};
     const PartView B{st.pt_npk, st.pt_codes_b.as<int>(), st.pt_step.as<unsigned char>()};
     const int *win = st.pt_win.as<int>();
-    k_sweep_parts<T, WF, false><<<waves, kPartBlock, 0, s>>>(np, F, win, pf.af, rhs, small, tmp, zp, nullptr, cfg.sf, sc);
-    k_sweep_parts<T, WB, true><<<waves, kPartBlock, 0, s>>>(np, B, win, pf.ab, tmp, small, zp, tmp, w, cfg.sf, sc);
+    k_sweep_parts<T, WF, false><<<waves, PartShape<WF>::kBlock, 0, s>>>(np, F, win, pf.af, rhs, small, tmp, zp, nullptr, cfg.sf, sc);
+    k_sweep_parts<T, WB, true><<<waves, PartShape<WB>::kBlock, 0, s>>>(np, B, win, pf.ab, tmp, small, zp, tmp, w, cfg.sf, sc);
 }
 
 template <class T, int WF>
