@@ -891,13 +891,12 @@ extern "C" fc_status fc_grad_gauss(fc_context *ctx, int numCells, int numFaces, 
             for (int f : hf) FC_REQUIRE(f >= 1 && f <= nf, FC_ERR_ARGUMENT, "O-C face number out of range");
         }
         double *g = dg.as<double>();
-        grad_gauss_dev(ctx, st, nif, own.as<int>(), nei.as<int>(), kface.as<int>(),
-                       needs ? kord.as<int>() : nullptr, dx[3].as<double>(), dx[4].as<double>(), dx[5].as<double>(),
-                       dx[0].as<double>(), dx[1].as<double>(), dx[2].as<double>(), dfi.as<double>(),
-                       dc[0].as<double>(), dc[1].as<double>(), dc[2].as<double>(), dc[3].as<double>(),
-                       du.as<double>(), G, cb_ptr.get() ? cb_ptr.as<int>() : nullptr,
-                       cb_q.get() ? cb_q.as<int>() : nullptr, oc, noc > 0 ? ocf.as<int>() : nullptr, nigrad, g,
-                       g + n, g + 2 * (size_t)n);
+        grad_gauss_dev(ctx, st, nif, own.as<int>(), nei.as<int>(), kface.as<int>(), needs ? kord.as<int>() : nullptr, dx[3].as<double>(),
+                       dx[4].as<double>(), dx[5].as<double>(), dx[0].as<double>(), dx[1].as<double>(),
+                       dx[2].as<double>(), dfi.as<double>(), dc[0].as<double>(), dc[1].as<double>(),
+                       dc[2].as<double>(), dc[3].as<double>(), du.as<double>(), (size_t)numTotal, G,
+                       cb_ptr.get() ? cb_ptr.as<int>() : nullptr, cb_q.get() ? cb_q.as<int>() : nullptr, oc,
+                       noc > 0 ? ocf.as<int>() : nullptr, nigrad, g, false);
         download_dbl(ctx, dudx, g, n);
         download_dbl(ctx, dudy, g + n, n);
         download_dbl(ctx, dudz, g + 2 * (size_t)n, n);
@@ -1302,7 +1301,9 @@ static fc_status sys_calcp_assemble(bool piso, fc_system *sys, const double *den
         F.dwdx = dgf[2];
         F.dpdx = dgf[3];
         ctx->timer.start(ctx->stream);
-        FC_HIP_CHECK(hipMemsetAsync(sys->a.get(), 0, sizeof(double) * sys->st.nnz, ctx->stream));   // calcp:34
+        // a = 0 (calcp:34): needed only where the faces and diagonals leave slots unwritten
+        if ((long long)sys->st.nnz != (long long)n + 2ll * nif)
+            FC_HIP_CHECK(hipMemsetAsync(sys->a.get(), 0, sizeof(double) * sys->st.nnz, ctx->stream));
         calcp_dev(ctx, sys->st, nif, sys->mesh.owner.as<int>(), sys->mesh.neighbour.as<int>(), sys->ij.as<int>(),
                   sys->ji.as<int>(), sys->kface.as<int>(), sys->needs_order ? sys->kord.as<int>() : nullptr,
                   g.xf.as<double>(), g.yf.as<double>(), g.zf.as<double>(), g.arx.as<double>(), g.ary.as<double>(),
@@ -1438,18 +1439,16 @@ static void sys_grad(fc_system *sys, const int *bnd, const double *du, int nigra
         build_boundary_lists(ctx, G, sys->mesh.owner.as<int>(), n, sys->grad_cb_ptr, sys->grad_cb_q);
         std::copy(bnd, bnd + 10, sys->grad_bnd);
     }
-    sys->grad_xyz.ensure(sizeof(double) * 3 * (size_t)n);
-    double *g = sys->grad_xyz.as<double>();
     GeometryDev &geo = sys->mesh.g;
     OcDev none;
     grad_gauss_dev(ctx, sys->st, nif, sys->mesh.owner.as<int>(), sys->mesh.neighbour.as<int>(), sys->kface.as<int>(),
-                   sys->needs_order ? sys->kord.as<int>() : nullptr, geo.xf.as<double>(), geo.yf.as<double>(),
-                   geo.zf.as<double>(), geo.arx.as<double>(), geo.ary.as<double>(), geo.arz.as<double>(),
-                   geo.facint.as<double>(), geo.xc.as<double>(), geo.yc.as<double>(), geo.zc.as<double>(),
-                   geo.vol.as<double>(), du, G, sys->grad_cb_ptr.get() ? sys->grad_cb_ptr.as<int>() : nullptr,
-                   sys->grad_cb_q.get() ? sys->grad_cb_q.as<int>() : nullptr, none, nullptr, nigrad, g, g + n,
-                   g + 2 * (size_t)n, &sys->grad_scratch);
-    interleave3_dev(ctx, n, g, g + n, g + 2 * (size_t)n, out);
+                   sys->needs_order ? sys->kord.as<int>() : nullptr,
+                   geo.xf.as<double>(), geo.yf.as<double>(), geo.zf.as<double>(), geo.arx.as<double>(),
+                   geo.ary.as<double>(), geo.arz.as<double>(), geo.facint.as<double>(), geo.xc.as<double>(),
+                   geo.yc.as<double>(), geo.zc.as<double>(), geo.vol.as<double>(), du, (size_t)sys->ntotal, G,
+                   sys->grad_cb_ptr.get() ? sys->grad_cb_ptr.as<int>() : nullptr,
+                   sys->grad_cb_q.get() ? sys->grad_cb_q.as<int>() : nullptr, none, nullptr, nigrad, out, true,
+                   &sys->grad_scratch);
 }
 
 extern "C" fc_status fc_sys_grad_gauss(fc_system *sys, const int *bnd, const double *u, int nigrad,

@@ -290,16 +290,14 @@ struct GradGroups {
 // per-cell lists of boundary items, each in sequence order
 void build_boundary_lists(fc_context *ctx, const GradGroups &G, const int *owner0_all, int n, DevBuf &cb_ptr,
                           DevBuf &cb_q);
-// (x, y, z component arrays of n) -> out(3, n), component fastest
-void interleave3_dev(fc_context *ctx, int n, const double *gx, const double *gy, const double *gz, double *out);
-// grad_gauss: nigrad iterations of the Gauss gradient of u (cells, then boundary values)
+// grad_gauss: nigrad passes of the Gauss gradient of u (nu values: cells, then boundary
+// values) into grad, 3 n values: (3, n) component fastest (interleaved) or x, y, z in turn
 void grad_gauss_dev(fc_context *ctx, const Structure &st, int nif, const int *owner0, const int *neigh0,
                     const int *kface, const int *kface_order, const double *xf, const double *yf,
                     const double *zf, const double *arx, const double *ary, const double *arz, const double *facint,
                     const double *xc, const double *yc, const double *zc, const double *vol, const double *u,
-                    const GradGroups &G, const int *cb_ptr, const int *cb_q, const OcDev &oc, const int *ocface,
-                    int nigrad, double *dudx, double *dudy, double *dudz,
-                    GradScratch *scratch = nullptr);
+                    size_t nu, const GradGroups &G, const int *cb_ptr, const int *cb_q, const OcDev &oc,
+                    const int *ocface, int nigrad, double *grad, bool interleaved, GradScratch *scratch = nullptr);
 // one velocity component's diagonal, source and 1/a_P (calcuvw), a's diagonal slots updated
 void momentum_rows_dev(fc_context *ctx, const Structure &st, double *a, const double *sp, const double *src,
                        const double *phi, double urf, double *su, double *ap);

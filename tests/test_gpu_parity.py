@@ -611,6 +611,33 @@ def test_grad_gauss_bitwise_vs_reference(ctx, golden_loader, case, nigrad):
         np.testing.assert_array_equal(a, g.out(s, k), err_msg=k)
 
 
+@pytest.mark.parametrize("legs", [1, 7, 8, 9, 16, 41])
+@pytest.mark.parametrize("shuffled", [False, True])
+def test_grad_gauss_rows_of_any_length(ctx, legs, shuffled):
+    """Rows of up to 41 faces (the row kernel takes eight a turn), faces in canonical order and
+    shuffled, one to three passes: the oracle's bits.  The geometry is arbitrary numbers."""
+    rng = np.random.default_rng(legs)
+    n = legs + 1
+    pairs = [(0, i) for i in range(1, n)] + [(i, i + 1) for i in range(1, n - 1)]
+    order = rng.permutation(len(pairs)) if shuffled else np.arange(len(pairs))
+    own, nei = np.array(pairs, np.int32)[order].T
+    nif, nb = len(pairs), 3
+    owner = np.concatenate([own, [0, 0, n - 1]]).astype(np.int32)
+    m = M.PolyMesh(np.zeros((3, 3)), np.arange(0, 3 * (nif + nb) + 1, 3, dtype=np.int32),
+                   np.zeros(3 * (nif + nb), np.int32), owner, np.ascontiguousarray(nei), n,
+                   [("inlet", 1, nif), ("wall", 2, nif + 1)])
+    face = lambda: rng.standard_normal(nif + nb)  # noqa: E731
+    cell = lambda: rng.standard_normal(n)  # noqa: E731
+    geo = fcap.Geometry(face(), face(), face(), face(), face(), face(), 0.5 + rng.random(n), cell(), cell(), cell(),
+                        rng.random(nif))
+    u = rng.standard_normal(n + nb)
+    for nigrad in (1, 2, 3):
+        out = fcap.grad_gauss(m, geo, u, nigrad, ctx=ctx)
+        ref = O.grad_gauss(m, geo, u, nigrad)
+        for a, b, k in zip(out, ref, ("dudx", "dudy", "dudz")):
+            np.testing.assert_array_equal(a, b, err_msg=f"{k} nigrad={nigrad}")
+
+
 def test_grad_gauss_oc_cuts_match_oracle(ctx):
     m = M.hex_box(5, perturb=0.2, seed=12)
     og = O.mesh_geometry(m)

@@ -417,6 +417,36 @@ def test_grad_resident_bitwise_vs_reference(ctx, golden_loader, name, nigrad):
         s.close()
 
 
+@pytest.mark.parametrize("nigrad", [1, 2, 3])
+@pytest.mark.parametrize("shift", [None, 0, 100])
+def test_grad_resident_into_memory_that_overlaps_the_field(ctx, nigrad, shift):
+    """The resident gradient with its result in device memory of its own (None), or starting
+    at the field's value `shift`: the oracle's bits all the same."""
+    import ctypes as C
+    m = M.hex_box(7, 6, 5, perturb=0.2, seed=4)
+    geo = O.mesh_geometry(m)
+    n = m.n_cells
+    u = np.random.default_rng(2).standard_normal(n + m.n_boundary)
+    ref = np.stack(O.grad_gauss(m, geo, u, nigrad), axis=1)
+    hip = C.CDLL("libamdhip64.so")
+    hip.hipMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t]
+    hip.hipMemcpy.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int]
+    hip.hipFree.argtypes = [C.c_void_p]
+    at = u.size if shift is None else shift
+    buf, p = np.zeros(u.size + 3 * n + 100), C.c_void_p()
+    buf[:u.size] = u
+    s = fcap.System(m, ctx)
+    assert hip.hipMalloc(C.byref(p), buf.nbytes) == 0
+    try:
+        assert hip.hipMemcpy(p, buf.ctypes.data, buf.nbytes, 1) == 0
+        assert s.grad_gauss(p.value, nigrad, out=p.value + 8 * at) is None
+        assert hip.hipMemcpy(buf.ctypes.data, p, buf.nbytes, 2) == 0
+        np.testing.assert_array_equal(buf[at:at + 3 * n].reshape(n, 3), ref)
+    finally:
+        hip.hipFree(p)
+        s.close()
+
+
 def test_resident_gradients_feed_the_assembly(case):
     """The step's chain on the resident system, grad(U) .. grad(P) then the assembly, against
     the oracle's gradients and assembly bit for bit; then the same chain with every field and
