@@ -759,9 +759,15 @@ double norm2_host(Ctx &c, const double *v) {
     return h[0];
 }
 
-// Runs `iter` until the device sets `done`.  One iteration is captured into a
-// HIP graph and replayed (the level-scheduled sweeps make an iteration hundreds
-// of small launches); the null stream cannot be captured, so it launches directly.
+// Runs `iter` until the device sets `done`, `per_graph` iterations captured into a HIP
+// graph and `launches` of them a batch; the null stream cannot be captured, so it launches
+// directly.  Between two graphs the GPU idles 5 to 7 us, inside one it does not: 8
+// Jacobi-PCG iterations a graph instead of 1 (four launches a batch) took 24.5 against
+// 27.7 ms on 97 x 83 x 61 (4: 25.7, 16: 24.1), 4 DIC-PCG iterations 10.8 against 11.4 ms
+// on 40^3 (2: 11.1, 6: 10.9) and 1.60 against 1.73 ms on 20 x 20 x 1 (6: 1.68, 8: 1.75:
+// what a batch launches past the end returns at once, but not for nothing).  One a graph
+// where an iteration is many launches (level sweeps) or a solve few iterations (BiCGStab:
+// 6.1 against 6.2 to 6.5 ms with 2 to 4), which a larger graph's set-up outweighs.
 struct GraphExec {
     hipGraphExec_t exec = nullptr;
     ~GraphExec() { if (exec) (void)hipGraphExecDestroy(exec); }
@@ -778,13 +784,13 @@ struct Events {
     }
 };
 
-void run_batches(Ctx &c, int batch, const std::function<void()> &iter) {
+void run_batches(Ctx &c, int per_graph, int launches, const std::function<void()> &iter) {
     GraphExec ge;
     if (c.ctx->use_graphs && c.s != nullptr) {
         hipGraph_t g = nullptr;
         FC_HIP_CHECK(hipStreamBeginCapture(c.s, hipStreamCaptureModeThreadLocal));
         try {
-            iter();
+            for (int k = 0; k < per_graph; ++k) iter();
         } catch (...) {
             (void)hipStreamEndCapture(c.s, &g);
             if (g) (void)hipGraphDestroy(g);
@@ -801,7 +807,7 @@ void run_batches(Ctx &c, int batch, const std::function<void()> &iter) {
     Events ev;
     int *flags = c.ctx->host_flags;
     for (int b = 0;; ++b) {
-        for (int k = 0; k < batch; ++k) {
+        for (int k = 0; k < (ge.exec ? launches : launches * per_graph); ++k) {
             if (ge.exec) FC_HIP_CHECK(hipGraphLaunch(ge.exec, c.s));
             else iter();
         }
@@ -1004,7 +1010,8 @@ fc_status solve_pcg64(fc_context *ctx, const SolveArgs &args, bool dic, fc_solve
             }
         };
         precondition(1);
-        run_batches(c, dic ? 2 : 4, [&]() {
+        const bool level = dic && !c.sw.sf;
+        run_batches(c, level ? 1 : dic ? 4 : 8, level ? 2 : 1, [&]() {
             spmv_launch64(c.s, 2, n, ptr, ja, args.a, p, nullptr, p, q, nullptr, c.pq, nullptr, c.sc);
             const SpmvSums pq = spmv_sums(c, false);
             if (dic)
@@ -1042,7 +1049,7 @@ fc_status solve_pcg64(fc_context *ctx, const SolveArgs &args, bool dic, fc_solve
         k_pcg_xr64<<<c.gv, kRedBlock, 0, c.s>>>(n, args.fi, r, p, q, c.sc, c.pa, c.pb);
         fin(c, kFinPcgEnd, seq_or(c, c.gv, 1, r, nullptr), true);
     };
-    run_batches(c, dic ? 2 : 4, iter);
+    run_batches(c, 1, dic ? 2 : 4, iter);
     double solve_ms = ctx->timer.stop_ms(c.s);
     check_sweeps(c);
     Scalars hs = read_scalars(c);
@@ -1088,7 +1095,7 @@ fc_status solve_bicgstab64(fc_context *ctx, const SolveArgs &args, fc_solve_info
         };
         k_first_dot<double><<<c.gf, kRedBlock, 0, c.s>>>(n, res, reso, nullptr, c.sc, c.pv);
         direction(1);
-        run_batches(c, 2, [&]() {
+        run_batches(c, 1, 2, [&]() {
             lu_launch64(c.s, st, args.a, d, small, pk, zk, c.sc, &c.sw, ppf);
             spmv_launch64(c.s, 2, n, ptr, ja, args.a, zk, nullptr, reso, uk, nullptr, c.pq, nullptr, c.sc);
             const SpmvSums ur = spmv_sums(c, false);
@@ -1120,7 +1127,7 @@ fc_status solve_bicgstab64(fc_context *ctx, const SolveArgs &args, fc_solve_info
         k_pcg_xr64<<<c.gv, kRedBlock, 0, c.s>>>(n, args.fi, res, zk, vk, c.sc, c.pa, c.pb);
         fin(c, kFinBicgEnd, seq_or(c, c.gv, 1, res, nullptr), true);
     };
-    run_batches(c, 2, iter);
+    run_batches(c, 1, 2, iter);
     double solve_ms = ctx->timer.stop_ms(c.s);
     check_sweeps(c);
     Scalars hs = read_scalars(c);
@@ -1166,7 +1173,7 @@ static int inner_solve32(Ctx &c, const Structure &st, bool bicg, double eta, dou
             k_cg_p<float, false><<<c.gf, kRedBlock, 0, c.s>>>(n, p, z, nullptr, c.sc, c.pv, c.gf, c.pz, c.gf, first);
         };
         precondition(1);
-        run_batches(c, 2, [&]() {
+        run_batches(c, c.sw.sf ? 4 : 1, c.sw.sf ? 1 : 2, [&]() {
             spmv_launch32(c.s, 2, n, ptr, ja, a32, p, nullptr, p, q, c.pq, nullptr, c.sc);
             const SpmvSums pq = spmv_sums(c, false);
             k_cg_xr<float, float, false><<<c.gf, kRedBlock, 0, c.s>>>(n, e, r, p, q, nullptr, c.sc, pq.a, pq.n, c.pv);
@@ -1182,7 +1189,7 @@ static int inner_solve32(Ctx &c, const Structure &st, bool bicg, double eta, dou
         };
         k_first_dot<float><<<c.gf, kRedBlock, 0, c.s>>>(n, r, reso, nullptr, c.sc, c.pv);
         direction(1);
-        run_batches(c, 2, [&]() {
+        run_batches(c, 1, 2, [&]() {
             lu_launch32(c.s, st, a32, d32, small, p, z, c.sc, &c.sw, pf);
             spmv_launch32(c.s, 2, n, ptr, ja, a32, z, nullptr, reso, uk, c.pq, nullptr, c.sc);
             const SpmvSums ur = spmv_sums(c, false);
@@ -1349,7 +1356,7 @@ static int inner_fcg32(Ctx &c, const Structure &st, const PrecondHook &P, double
             iter();
         }
     };
-    run_batches(c, std::max(1, 2 / period), group);
+    run_batches(c, 1, std::max(1, 2 / period), group);
     Scalars hs = read_scalars(c);
     iters += hs.iters;
     return hs.status;
