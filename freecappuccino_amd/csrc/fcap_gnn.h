@@ -4,6 +4,7 @@
 #include "fcap_coarse.h"
 #include "fcap_internal.h"
 #include "fcap_kernels.h"
+#include "fcap_linalg.h"
 
 namespace fcap {
 
@@ -23,6 +24,9 @@ struct GnnGraph {
     int n = 0, nnz = 0;
     const int *ptr = nullptr, *ja = nullptr, *diagpos = nullptr;
     DevBuf ef, dg, trans, a32;
+    // the matrix in slices for the damped-Jacobi steps (slices.w = 0: CSR)
+    SliceView slices;
+    DevBuf as32;
     // The off-diagonal entries again as an ELL over the cells: slot k of cell i
     // at [k * n + i], in CSR order; padding slots hold the cell itself and zero
     // features and lie past ecnt[i].  Lanes of a wave own consecutive cells, so
@@ -74,7 +78,7 @@ void sort_pairs_u64(hipStream_t s, const unsigned long long *key_in, unsigned lo
                     int *val_out, int n, DevBuf &tmp);
 
 // Build the graph data of an assembled system (device arrays of the system).
-void gnn_prepare_graph(fc_context *ctx, GnnGraph &g, const Structure &st, const int *kface, const int *owner0,
+void gnn_prepare_graph(fc_context *ctx, GnnGraph &g, Structure &st, const int *kface, const int *owner0,
                        const int *ij, const int *ji, int nif, const double *arx, const double *ary,
                        const double *arz, const double *xc, const double *yc, const double *zc, const double *a);
 

@@ -1676,7 +1676,7 @@ void build_clusters(hipStream_t s, GnnGraph &g, const double *xc, const double *
 
 }  // namespace
 
-void gnn_prepare_graph(fc_context *ctx, GnnGraph &g, const Structure &st, const int *kface, const int *owner0,
+void gnn_prepare_graph(fc_context *ctx, GnnGraph &g, Structure &st, const int *kface, const int *owner0,
                        const int *ij, const int *ji, int nif, const double *arx, const double *ary, const double *arz,
                        const double *xc, const double *yc, const double *zc, const double *a) {
     (void)owner0;
@@ -1695,6 +1695,11 @@ void gnn_prepare_graph(fc_context *ctx, GnnGraph &g, const Structure &st, const 
     k_gnn_edges<<<grid_for(st.n, 256), 256, 0, s>>>(st.n, g.ptr, g.ja, g.diagpos, kface, arx, ary, arz, xc, yc, zc, a,
                                                     g.ef.as<uint32_t>(), g.dg.as<float>());
     k_cast_df<<<std::min(grid_for(st.nnz, 256), 8192), 256, 0, s>>>(st.nnz, a, g.a32.as<float>());
+    g.slices = slices_for(ctx, st);
+    if (g.slices.w) {
+        g.as32.ensure(sizeof(float) * slice_count(st.n, g.slices));
+        slice_values32(s, st.n, g.slices, a, g.as32.as<float>());
+    }
     if (new_structure) {
         g.trans.ensure(sizeof(int) * (size_t)st.nnz);
         k_gnn_trans_init<<<grid_for(st.nnz, 256), 256, 0, s>>>(st.nnz, g.trans.as<int>());
@@ -2120,8 +2125,12 @@ void precondition_tail(fc_system *sys, hipStream_t s, const float *r, float *z, 
     const int steps = c->gnn_smooth;
     float *buf[2] = {z, g.zscratch.as<float>()};
     for (int k = 0; k < steps; ++k)
-        jacobi_step32(s, g.n, g.ptr, g.ja, g.a32.as<float>(), buf[k & 1], r, g.dg.as<float>(), c->gnn_omega,
-                      buf[(k + 1) & 1], sc);
+        if (g.slices.w)
+            sliced_jacobi32(s, g.n, g.slices, g.as32.as<float>(), buf[k & 1], r, g.dg.as<float>(), c->gnn_omega,
+                            buf[(k + 1) & 1], sc);
+        else
+            jacobi_step32(s, g.n, g.ptr, g.ja, g.a32.as<float>(), buf[k & 1], r, g.dg.as<float>(), c->gnn_omega,
+                          buf[(k + 1) & 1], sc);
     float *zf = buf[steps & 1];
     if (g.coarse.ok)
         coarse_apply(s, g.coarse, r, zf, z, sc);

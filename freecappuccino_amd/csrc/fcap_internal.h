@@ -115,6 +115,10 @@ struct Structure {
     int pt_npk = 0, pt_nparts = 0;
     DevBuf pt_rows, pt_step, pt_win, pt_codes_f, pt_codes_b;
     double int_frac_f = 0.0, int_frac_b = 0.0;
+    // rows in slices of 64 (fcap_slices.hip): width (0: not sliced), column bases, offsets
+    bool sl_ready = false;
+    int sl_w = 0;
+    DevBuf sl_base, sl_off;
 };
 
 struct Workspace;   // solver vectors, partial sums, device scalars

@@ -32,6 +32,26 @@ void residual32(hipStream_t s, int n, const int *ptr, const int *ja, const float
                 float *y, const Scalars *sc);
 void oc_launch64(hipStream_t s, int n, const OcView &oc, const double *x, double *y, int sign, const Scalars *sc);
 
+// A matrix's rows in slices of 64 (fcap_slices.hip): columns of the structure (built once
+// for it) and values per solve; w = 0: the rows are too long or too uneven for slices.
+struct SliceView {
+    int w = 0;
+    const int *base = nullptr, *ptr = nullptr, *ja = nullptr;
+    const unsigned *off = nullptr;
+};
+SliceView slices_for(fc_context *ctx, Structure &st);
+size_t slice_count(int n, const SliceView &S);   // values of the matrix
+void slice_values64(hipStream_t s, int n, const SliceView &S, const double *a, double *v);
+void slice_values32(hipStream_t s, int n, const SliceView &S, const double *a, float *v);
+// y = A x with partials of y.b (pa) and, with pb, of y.y: spmv_launch* modes 2 and 3 bit for bit
+void sliced_product64(hipStream_t s, int n, const SliceView &S, const double *v, const double *x, const double *b,
+                      double *y, double *pa, double *pb, const Scalars *sc);
+void sliced_product32(hipStream_t s, int n, const SliceView &S, const float *v, const float *x, const float *b,
+                      float *y, double *pa, double *pb, const Scalars *sc);
+// jacobi_step32 bit for bit
+void sliced_jacobi32(hipStream_t s, int n, const SliceView &S, const float *v, const float *x, const float *b,
+                     const float *d, float omega, float *y, const Scalars *sc);
+
 // State of the dependency-driven sweeps: the next block of 64 packed rows to
 // hand out, the number of waves that have left the kernel (the last one resets
 // both for the next launch), a sticky abort flag raised when a wait exceeds

@@ -670,6 +670,7 @@ void build_structure_from_host_csr(fc_context *ctx, Structure &st, int n, int nn
     check_err(ctx, err, "CSR");
     st.levels_ready = false;
     st.has_tpos = false;
+    st.sl_ready = false;
 }
 
 void build_structure_from_faces_dev(fc_context *ctx, Structure &st, int n, int nif, const int *own0,
@@ -699,6 +700,7 @@ void build_structure_from_faces_dev(fc_context *ctx, Structure &st, int n, int n
     FC_HIP_CHECK(hipGetLastError());
     st.levels_ready = false;
     st.has_tpos = false;
+    st.sl_ready = false;
 }
 
 void upload_mesh(fc_context *ctx, MeshDev &m, int nnodes, const double *xyz, int nfaces, int nif,

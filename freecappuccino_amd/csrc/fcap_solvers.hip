@@ -918,6 +918,50 @@ static PackedFactor<T> pack_for_solve(Ctx &c, const Structure &st, const T *a, c
     return pf;
 }
 
+// The matrix of a solve as its iterations multiply by it: in slices where the structure has
+// them, else the CSR arrays.
+template <class T> struct Matrix {
+    SliceView S;
+    const T *v = nullptr;          // sliced values
+    const int *ptr, *ja;
+    const T *a = nullptr;          // CSR values
+};
+static Matrix<double> matrix64(Ctx &c, const Structure &st, const double *a) {
+    Matrix<double> A{{}, nullptr, st.ioffset.as<int>(), st.ja.as<int>(), a};
+    A.S = slices_for(c.ctx, const_cast<Structure &>(st));
+    if (A.S.w) {
+        c.ws->as64.ensure(sizeof(double) * slice_count(st.n, A.S));
+        slice_values64(c.s, st.n, A.S, a, c.ws->as64.as<double>());
+        A.v = c.ws->as64.as<double>();
+    }
+    return A;
+}
+// csr: the FP32 CSR values are wanted too
+static Matrix<float> matrix32(Ctx &c, const Structure &st, const double *a, bool csr) {
+    Matrix<float> A{{}, nullptr, st.ioffset.as<int>(), st.ja.as<int>(), c.ws->a32.as<float>()};
+    A.S = slices_for(c.ctx, const_cast<Structure &>(st));
+    if (A.S.w) {
+        c.ws->as32.ensure(sizeof(float) * slice_count(st.n, A.S));
+        slice_values32(c.s, st.n, A.S, a, c.ws->as32.as<float>());
+        A.v = c.ws->as32.as<float>();
+    }
+    if (csr || !A.S.w)
+        k_cast<double, float><<<std::min(grid_for(st.nnz, 256), 8192), 256, 0, c.s>>>(st.nnz, a,
+                                                                                     c.ws->a32.as<float>());
+    return A;
+}
+// y = A x with partials of y.b (pa) and, with pb, of y.y
+static void product(Ctx &c, const Matrix<double> &A, const double *x, const double *b, double *y, double *pa,
+                    double *pb = nullptr) {
+    if (A.S.w) sliced_product64(c.s, c.n, A.S, A.v, x, b, y, pa, pb, c.sc);
+    else spmv_launch64(c.s, pb ? 3 : 2, c.n, A.ptr, A.ja, A.a, x, nullptr, b, y, nullptr, pa, pb, c.sc);
+}
+static void product(Ctx &c, const Matrix<float> &A, const float *x, const float *b, float *y, double *pa,
+                    double *pb = nullptr) {
+    if (A.S.w) sliced_product32(c.s, c.n, A.S, A.v, x, b, y, pa, pb, c.sc);
+    else spmv_launch32(c.s, pb ? 3 : 2, c.n, A.ptr, A.ja, A.a, x, nullptr, b, y, pa, pb, c.sc);
+}
+
 static void check_pivots(Ctx &c) {
     int h = 0;
     FC_HIP_CHECK(hipMemcpyAsync(&h, c.ws->err.get(), sizeof(int), hipMemcpyDeviceToHost, c.s));
@@ -998,6 +1042,7 @@ fc_status solve_pcg64(fc_context *ctx, const SolveArgs &args, bool dic, fc_solve
     const int gs = spmv_grid(n);
     ctx->timer.start(c.s);
     if (fuse) {
+        const Matrix<double> A = matrix64(c, st, args.a);
         if (!dic) k_diag<<<c.gv, 256, 0, c.s>>>(n, args.a, dg, z);   // z holds the diagonal
         auto precondition = [&](int first) {
             if (dic) {
@@ -1012,7 +1057,7 @@ fc_status solve_pcg64(fc_context *ctx, const SolveArgs &args, bool dic, fc_solve
         precondition(1);
         const bool level = dic && !c.sw.sf;
         run_batches(c, level ? 1 : dic ? 4 : 8, level ? 2 : 1, [&]() {
-            spmv_launch64(c.s, 2, n, ptr, ja, args.a, p, nullptr, p, q, nullptr, c.pq, nullptr, c.sc);
+            product(c, A, p, p, q, c.pq);
             const SpmvSums pq = spmv_sums(c, false);
             if (dic)
                 k_cg_xr<double, double, false><<<c.gf, kRedBlock, 0, c.s>>>(n, args.fi, r, p, q, nullptr, c.sc, pq.a,
@@ -1090,6 +1135,7 @@ fc_status solve_bicgstab64(fc_context *ctx, const SolveArgs &args, fc_solve_info
     const int gs = spmv_grid(n);
     ctx->timer.start(c.s);
     if (!c.ctx->reduce_seq) {   // (the reference's BiCGStab applies its O-C couplings to the initial residual alone)
+        const Matrix<double> A = matrix64(c, st, args.a);
         auto direction = [&](int first) {
             k_bi_p<double><<<c.gf, kRedBlock, 0, c.s>>>(n, pk, res, uk, c.sc, c.pv, c.gf, first);
         };
@@ -1097,11 +1143,11 @@ fc_status solve_bicgstab64(fc_context *ctx, const SolveArgs &args, fc_solve_info
         direction(1);
         run_batches(c, 1, 2, [&]() {
             lu_launch64(c.s, st, args.a, d, small, pk, zk, c.sc, &c.sw, ppf);
-            spmv_launch64(c.s, 2, n, ptr, ja, args.a, zk, nullptr, reso, uk, nullptr, c.pq, nullptr, c.sc);
+            product(c, A, zk, reso, uk, c.pq);
             const SpmvSums ur = spmv_sums(c, false);
             k_bi_xr1<double, double><<<c.gf, kRedBlock, 0, c.s>>>(n, args.fi, res, zk, uk, c.sc, ur.a, ur.n);
             lu_launch64(c.s, st, args.a, d, small, res, zk, c.sc, &c.sw, ppf);
-            spmv_launch64(c.s, 3, n, ptr, ja, args.a, zk, nullptr, res, vk, nullptr, c.pq, c.pq2, c.sc);
+            product(c, A, zk, res, vk, c.pq, c.pq2);
             const SpmvSums v = spmv_sums(c, true);
             k_bi_xr2<double, double><<<c.gf, kRedBlock, 0, c.s>>>(n, args.fi, res, zk, vk, reso, c.sc, v.a, v.b, v.n,
                                                                  c.pv);
@@ -1140,16 +1186,14 @@ fc_status solve_bicgstab64(fc_context *ctx, const SolveArgs &args, fc_solve_info
 // iteration (<= 0: none), on exit this cycle's.  With a previous value the search
 // direction p is kept and the first step continues it (beta = r.z / s0_carry), so
 // the refinement replaces the residual without discarding the Krylov direction.
-static int inner_solve32(Ctx &c, const Structure &st, bool bicg, double eta, double r32norm2, int cap,
+static int inner_solve32(Ctx &c, const Structure &st, const Matrix<float> &A, bool bicg, double eta, double r32norm2, int cap,
                          const PackedFactor<float> *pf, double *s0_carry = nullptr) {
     Workspace &ws = *c.ws;
     const int n = c.n;
     float *a32 = ws.a32.as<float>(), *d32 = ws.d32.as<float>();
     float *r = ws.r32.as<float>(), *z = ws.z32.as<float>(), *p = ws.p32.as<float>(), *q = ws.q32.as<float>();
     float *e = ws.e32.as<float>();
-    const int *ptr = st.ioffset.as<int>(), *ja = st.ja.as<int>();
     const float small = (float)kSmallSrc;
-    const int gs = spmv_grid(n);
     Scalars h;
     std::memset(&h, 0, sizeof(h));
     const bool keep = !bicg && s0_carry && *s0_carry > 0.0;
@@ -1174,7 +1218,7 @@ static int inner_solve32(Ctx &c, const Structure &st, bool bicg, double eta, dou
         };
         precondition(1);
         run_batches(c, c.sw.sf ? 4 : 1, c.sw.sf ? 1 : 2, [&]() {
-            spmv_launch32(c.s, 2, n, ptr, ja, a32, p, nullptr, p, q, c.pq, nullptr, c.sc);
+            product(c, A, p, p, q, c.pq);
             const SpmvSums pq = spmv_sums(c, false);
             k_cg_xr<float, float, false><<<c.gf, kRedBlock, 0, c.s>>>(n, e, r, p, q, nullptr, c.sc, pq.a, pq.n, c.pv);
             precondition(0);
@@ -1191,11 +1235,11 @@ static int inner_solve32(Ctx &c, const Structure &st, bool bicg, double eta, dou
         direction(1);
         run_batches(c, 1, 2, [&]() {
             lu_launch32(c.s, st, a32, d32, small, p, z, c.sc, &c.sw, pf);
-            spmv_launch32(c.s, 2, n, ptr, ja, a32, z, nullptr, reso, uk, c.pq, nullptr, c.sc);
+            product(c, A, z, reso, uk, c.pq);
             const SpmvSums ur = spmv_sums(c, false);
             k_bi_xr1<float, float><<<c.gf, kRedBlock, 0, c.s>>>(n, e, r, z, uk, c.sc, ur.a, ur.n);
             lu_launch32(c.s, st, a32, d32, small, r, z, c.sc, &c.sw, pf);
-            spmv_launch32(c.s, 3, n, ptr, ja, a32, z, nullptr, r, vk, c.pq, c.pq2, c.sc);
+            product(c, A, z, r, vk, c.pq, c.pq2);
             const SpmvSums v = spmv_sums(c, true);
             k_bi_xr2<float, float><<<c.gf, kRedBlock, 0, c.s>>>(n, e, r, z, vk, reso, c.sc, v.a, v.b, v.n, c.pv);
             direction(0);
@@ -1218,7 +1262,7 @@ fc_status solve_mixed(fc_context *ctx, const SolveArgs &args, bool bicg, fc_solv
     FC_HIP_CHECK(hipMemsetAsync(ws.err.get(), 0, sizeof(int), c.s));
     if (bicg) build_tpos(ctx, const_cast<Structure &>(st));
     pivots_launch(c.s, st, args.a, d, bicg, ws.err.as<int>(), &c.sw);
-    k_cast<double, float><<<std::min(grid_for(st.nnz, 256), 8192), 256, 0, c.s>>>(st.nnz, args.a, ws.a32.as<float>());
+    const Matrix<float> A = matrix32(c, st, args.a, true);
     k_cast<double, float><<<c.gv, 256, 0, c.s>>>(n, d, ws.d32.as<float>());
     const PackedFactor<float> pf = pack_for_solve<float>(c, st, ws.a32.as<float>(), ws.d32.as<float>());
     double setup_ms = ctx->timer.stop_ms(c.s);
@@ -1254,7 +1298,7 @@ fc_status solve_mixed(fc_context *ctx, const SolveArgs &args, bool bicg, fc_solv
         const double rn = std::sqrt(ho.rnorm2);
         if (outer == 0 || bicg) scale = rn;
         k_scale_cast<<<c.gv, 256, 0, c.s>>>(n, r, ws.r32.as<float>(), 1.0 / scale);
-        total_inner += inner_solve32(c, st, bicg, args.inner_eta, ho.rnorm2 / (scale * scale), cap,
+        total_inner += inner_solve32(c, st, A, bicg, args.inner_eta, ho.rnorm2 / (scale * scale), cap,
                                      pf.af ? &pf : nullptr, &s0c);
         k_refine<<<c.gv, 256, 0, c.s>>>(n, args.fi, ws.e32.as<float>(), scale);
         ++outer;
@@ -1294,13 +1338,11 @@ static int fcg_window(const fc_context *ctx) {
 // Truncated FCG in FP32 on A e = r32 (unit-norm r32), preconditioner P.
 // Returns the inner status (FC_OK, FC_NOT_CONVERGED, FC_FALLBACK_USED on
 // stagnation, FC_ERR_NONFINITE) and adds the iterations to `iters`.
-static int inner_fcg32(Ctx &c, const Structure &st, const PrecondHook &P, double eta, int cap, int &iters) {
+static int inner_fcg32(Ctx &c, const Matrix<float> &A, const PrecondHook &P, double eta, int cap, int &iters) {
     Workspace &ws = *c.ws;
     const int n = c.n;
-    float *a32 = ws.a32.as<float>();
     float *r = ws.r32.as<float>(), *z = ws.z32.as<float>(), *p = ws.p32.as<float>(), *q = ws.q32.as<float>();
     float *e = ws.e32.as<float>(), *ph = ws.ph.as<float>(), *qh = ws.qh.as<float>();
-    const int *ptr = st.ioffset.as<int>(), *ja = st.ja.as<int>();
     const int gs = spmv_grid(n);
     Scalars h;
     std::memset(&h, 0, sizeof(h));
@@ -1345,7 +1387,7 @@ static int inner_fcg32(Ctx &c, const Structure &st, const PrecondHook &P, double
         fin(c, kFinFcgBeta, c.gv, false);
         pupd();
         fin(c, kFinFcgPr, c.gv, false);
-        spmv_launch32(c.s, 2, n, ptr, ja, a32, p, nullptr, p, q, c.pa, nullptr, c.sc);
+        product(c, A, p, p, q, c.pa);
         fin(c, kFinFcgAlf, gs, false);
         k_fcg_xr<<<c.gv, kRedBlock, 0, c.s>>>(n, e, r, p, q, ph, qh, c.sc, c.pa, c.pb);
         fin(c, kFinFcgEnd, c.gv, true);
@@ -1373,7 +1415,7 @@ fc_status solve_fcg(fc_context *ctx, const SolveArgs &args, const PrecondHook &P
     ws.ph.ensure(sizeof(float) * (size_t)m * (size_t)n);
     ws.qh.ensure(sizeof(float) * (size_t)m * (size_t)n);
     ctx->timer.start(c.s);
-    k_cast<double, float><<<std::min(grid_for(st.nnz, 256), 8192), 256, 0, c.s>>>(st.nnz, args.a, ws.a32.as<float>());
+    const Matrix<float> A = matrix32(c, st, args.a, false);
     double setup_ms = ctx->timer.stop_ms(c.s);
     Scalars h0 = init_scalars(args, kSmallSrc);
     h0.bnorm2 = norm2_host(c, args.su);
@@ -1402,7 +1444,7 @@ fc_status solve_fcg(fc_context *ctx, const SolveArgs &args, const PrecondHook &P
         const double rn = std::sqrt(ho.rnorm2);
         k_scale_cast<<<c.gv, 256, 0, c.s>>>(n, r, ws.r32.as<float>(), 1.0 / rn);
         const int cap = std::max(1, args.nsw - total_inner);
-        const int ist = inner_fcg32(c, st, P, args.inner_eta, cap, total_inner);
+        const int ist = inner_fcg32(c, A, P, args.inner_eta, cap, total_inner);
         ++outer;
         if (ist == FC_FALLBACK_USED || ist == FC_ERR_NONFINITE) {
             // plain IC(0)-PCG (FP64) finishes the solve from the last refined iterate;

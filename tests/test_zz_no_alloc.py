@@ -91,6 +91,55 @@ def test_noalloc_dpcg_matches_dpcg_on_two_calls():
         ctx.close()
 
 
+def _random_csr(n, matchings, near, seed):
+    """Symmetric, diagonally dominant: the chain i ~ i + 1 and random pairs of rows (any two
+    rows, or at most `near` apart), each row in at most `matchings` of them."""
+    rng = np.random.default_rng(seed)
+    pairs = [np.stack([np.arange(n - 1), np.arange(1, n)], 1)]
+    for _ in range(matchings):
+        key = np.arange(n) + rng.random(n) * near if near else rng.random(n)
+        order = np.argsort(key)
+        pairs.append(np.sort(order[:n // 2 * 2].reshape(-1, 2), axis=1))
+    pq = np.unique(np.concatenate(pairs), axis=0)
+    val = -rng.random(pq.shape[0])
+    row = np.concatenate([pq[:, 0], pq[:, 1], np.arange(n)])
+    col = np.concatenate([pq[:, 1], pq[:, 0], np.arange(n)])
+    a = np.concatenate([val, val, np.zeros(n)])
+    off = np.zeros(n)
+    np.add.at(off, row, np.abs(a))
+    a[-n:] = 1.05 * off + 0.1
+    order = np.lexsort((col, row))
+    ioffset = np.concatenate([[0], np.cumsum(np.bincount(row, minlength=n))])
+    diag = np.flatnonzero((col == row)[order])
+    one = lambda x: np.ascontiguousarray(x + 1, np.int32)  # noqa: E731
+    return fcap.CSR(one(ioffset), one(col[order]), one(diag), np.zeros(0, np.int32), np.zeros(0, np.int32)), a[order]
+
+
+@pytest.mark.parametrize("n,matchings,near", [(1, 0, 0), (2, 0, 0), (63, 1, 0), (64, 3, 5), (65, 4, 0), (255, 5, 20),
+                                              (257, 5, 0), (1000, 6, 0), (1000, 9, 0), (70001, 4, 0),
+                                              (70001, 4, 300), (70001, 0, 0)])
+def test_products_in_slices_give_the_csr_bits(n, matchings, near):
+    """fc_dpcg multiplies by the matrix in slices of 64 rows, fc_dpcg_noalloc by the CSR rows:
+    the same solution, residual and iterations bit for bit.  Rows of 1 to 11 entries (beyond 8
+    there are no slices), a last slice of 1, 63 and 64 rows, columns of a slice within 16 bits
+    and beyond them (pairs of any two of 70,001 rows)."""
+    ctx = fcap.Context(0)
+    dev = _Dev()
+    try:
+        csr, a = _random_csr(n, matchings, near, n + matchings)
+        su = np.random.default_rng(1).standard_normal(n)
+        fi0 = np.zeros(n)
+        ref = fcap.dpcg(csr, a, su, fi0, sor=1e-12, nsw=500, ctx=ctx)
+        rc, fi, res, info = _noalloc(ctx, dev, csr, a, su, fi0, 1e-12, 500)
+        assert rc == ref.status == fcap.FC_OK, (rc, ref.status)
+        assert info["iters"] == ref.info["iters"] > 0
+        np.testing.assert_array_equal(fi, ref.fi)
+        np.testing.assert_array_equal(res, ref.res)
+    finally:
+        dev.close()
+        ctx.close()
+
+
 def test_noalloc_dpcg_refuses_oversize_and_host_arrays():
     ctx = fcap.Context(0)
     dev = _Dev()
