@@ -1048,6 +1048,7 @@ struct SweepFactor {
             df.alloc(sizeof(double) * n);
             db.alloc(sizeof(double) * n);
             pack_factor64(s, st, a, d, af.as<double>(), df.as<double>(), ab.as<double>(), db.as<double>());
+            if (cfg.sf) mark_sweep_input64(s, st.n, tmp.as<double>());
         }
         pf = {af.as<double>(), df.as<double>(), ab.as<double>(), db.as<double>()};
     }

@@ -195,9 +195,8 @@ namespace fcap {
 // them wait, and poll, than the chain of parts can use)
 inline int part_wave_count(const fc_context *ctx) { return ctx->part_waves > 0 ? ctx->part_waves : ctx->num_cus; }
 
-// persistent waves of the row-wise dependency-driven sweeps and pivots: one 64-row
-// block per wave for the rows of an average level, at least one wave per CU and at
-// most sixteen.  A deep chain (192^3 box in natural order: 574 levels of 12K rows)
+// persistent waves of the row-wise dependency-driven sweeps and pivots: twice the
+// 64-row blocks of an average level, at least one wave per CU and at most sixteen.  A deep chain (192^3 box in natural order: 574 levels of 12K rows)
 // then runs with one wave per CU -- more waves only add polling -- and a shallow one
 // (96^3 permuted Kuhn tets: 16 levels of 330K rows) with enough waves to keep its
 // gathers in flight.
@@ -205,7 +204,7 @@ inline int syncfree_wave_count(const fc_context *ctx, const Structure &st) {
     if (ctx->part_waves > 0) return ctx->part_waves;
     const long long nlev = std::max(1, std::max(st.nlev_f, st.nlev_b));
     const long long blocks = ((long long)st.n / nlev + 63) / 64;
-    return (int)std::min<long long>(16LL * ctx->num_cus, std::max<long long>(ctx->num_cus, blocks));
+    return (int)std::min<long long>(16LL * ctx->num_cus, std::max<long long>(ctx->num_cus, 2 * blocks));
 }
 
 // ---------------------------------------------------------------- launchers

@@ -56,11 +56,14 @@ void sliced_jacobi32(hipStream_t s, int n, const SliceView &S, const float *v, c
 // hand out, the number of waves that have left the kernel (the last one resets
 // both for the next launch), a sticky abort flag raised when a wait exceeds
 // its time limit, that limit in microseconds (0: the built-in one) and the
-// rate of the device's wall clock in kHz.
+// rate of the device's wall clock in kHz.  The row-wise sweeps hand their blocks out
+// through counters of their own, kSfTickets for each direction, a cache line apart.
+constexpr int kSfTickets = 8;
 struct SyncFree {
     unsigned ticket, fin;
     int abort, wait_us;
     unsigned rate_khz, pad;
+    unsigned tickets[2][kSfTickets][32];
 };
 // zeroed state with the context's wait limit, on the stream (not for graph capture)
 void syncfree_reset(fc_context *ctx, hipStream_t s, SyncFree *sf);
@@ -135,6 +138,10 @@ void pack_factor_parts64(hipStream_t s, const Structure &st, const double *a, co
                          double *tmp);
 void pack_factor_parts32(hipStream_t s, const Structure &st, const float *a, const float *d, float *af, float *ab,
                          float *tmp);
+// marks SweepCfg::tmp before the first row-wise dependency-driven sweep; each pair of
+// sweeps leaves it marked for the next
+void mark_sweep_input64(hipStream_t s, int n, double *tmp);
+void mark_sweep_input32(hipStream_t s, int n, float *tmp);
 // both sweeps in the part-wise schedule (lu_launch* with cfg.parts)
 void lu_parts64(hipStream_t s, const Structure &st, const PackedFactor<double> &pf, double small, const double *rhs,
                 double *w, const Scalars *sc, const SweepCfg &cfg);

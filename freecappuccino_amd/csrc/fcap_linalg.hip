@@ -458,9 +458,12 @@ void pack_factor_t(hipStream_t s, const Structure &st, const T *a, const T *d, T
 
 // ------------------------------------------- dependency-driven sweeps
 // One launch per sweep.  Persistent one-wave workgroups take blocks of 64
-// consecutive packed rows (level order) from a ticket counter, so every row a
-// block reads lies in a block handed out earlier, to a wave that is running or
-// has finished: the waits always end.  The output starts filled with a
+// consecutive packed rows (level order) from ticket counters: workgroup g from counter
+// g % K (K = kSfTickets, or the grid if smaller), which hands out blocks g % K, + K, ...
+// in turn.  The smallest unfinished block has been handed out, or a running wave of its
+// counter takes it next (the first K workgroups start first), so the waits always end.
+// One counter for all cost 10 ns a ticket one after the other: with marks in launches of
+// their own 34 us a sweep on the 24^3 tets, now 25, on the 40^3 tets 90 and 39.  A sweep clears the other direction's counters.  The output starts filled with a
 // signalling-NaN pattern that arithmetic never produces; a row polls the
 // outputs of the rows it reads until none holds the pattern, computes exactly
 // as k_fwd_packed / k_bwd_packed (same operands, same order), and stores its
@@ -469,8 +472,11 @@ void pack_factor_t(hipStream_t s, const Structure &st, const T *a, const T *d, T
 // flag and leaves; the host then reports the solve as failed.
 
 // Waves in flight poll the coherent level of the memory system; the fewer there
-// are, the faster the chain of levels advances (192^3 box: 256 waves 1.87 s,
-// 512 1.96 s, 2048 2.55 s, 4096 3.61 s per FP64 IC(0)-PCG solve).
+// are, the faster the chain of levels advances, as long as they hold a level
+// (syncfree_wave_count: twice an average level, at least one a CU).  Per sweep: Kuhn
+// tets 24^3, 14 levels of 5,925 rows, 256 waves 25 us, 512 26, 1,024 28; 40^3, 14 of
+// 27,429, 256 62, 428 46, 768 39, 1,024 38, 2,048 44; 96^3 box, 286 of 3,094, 256 468,
+// 512 527, 1,024 627.
 
 template <class T>
 __global__ void k_sf_mark(int n, T *__restrict__ w, const Scalars *__restrict__ sc) {
@@ -481,23 +487,31 @@ __global__ void k_sf_mark(int n, T *__restrict__ w, const Scalars *__restrict__ 
     reinterpret_cast<U *>(w)[i] = SfBits<T>::kMark;
 }
 
+// The other sweep's output takes its marks here: the forward sweep marks w, whose values
+// are spent, the backward one its right-hand side once read (a pass of its own for each
+// took 4.4 us on 83 K rows, beside sweeps of 26 us); mark_sweep_input does it before the
+// first sweep.
 // BWD == false: out[i] = (rhs[i] - sum a w) d over the strict lower triangle;
 // BWD == true:  out[i] = (fwd[i] / (d + small) - sum a w) d over the strict upper one.
 template <class T, int W, bool BWD>
 __global__ __launch_bounds__(64) void k_sweep_syncfree(int n, const int *__restrict__ rows,
                                                         const int *__restrict__ cntp, const int *__restrict__ col,
                                                         const T *__restrict__ av, const T *__restrict__ dv,
-                                                        const T *__restrict__ in, T small, T *out, SyncFree *sf,
+                                                        const T *in, T small, T *out, T *mk, SyncFree *sf,
                                                         const Scalars *__restrict__ sc) {
     if (sc && sc->done) return;
     using U = typename SfBits<T>::U;
     const int lane = threadIdx.x;
     const unsigned nblk = (unsigned)((n + 63) / 64);
     const unsigned long long limit = sf_wait_ticks(sf, sf->rate_khz);
+    const unsigned counters = min((unsigned)kSfTickets, gridDim.x), mine = blockIdx.x % counters;
+    unsigned *ticket = &sf->tickets[BWD][mine][0];
+    if (blockIdx.x == 0 && lane < kSfTickets)
+        __hip_atomic_store(&sf->tickets[!BWD][lane][0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (;;) {
         unsigned b = 0;
-        if (lane == 0) b = __hip_atomic_fetch_add(&sf->ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        b = __shfl(b, 0);
+        if (lane == 0) b = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        b = __shfl(b, 0) * counters + mine;
         if (b >= nblk) break;
         const int p = (int)b * 64 + lane;
         bool done = p >= n;
@@ -517,6 +531,7 @@ __global__ __launch_bounds__(64) void k_sweep_syncfree(int n, const int *__restr
                 wk[k] = T(0);
             }
             acc = BWD ? in[i] / (di + small) : in[i];
+            reinterpret_cast<U *>(mk)[i] = SfBits<T>::kMark;   // behind the load of in[i] (mk may be in)
         }
         int spins = 0;
         const unsigned long long t0 = wall_clock64();
@@ -558,13 +573,6 @@ __global__ __launch_bounds__(64) void k_sweep_syncfree(int n, const int *__restr
                 break;
             }
             __builtin_amdgcn_s_sleep(1);
-        }
-    }
-    if (lane == 0) {
-        const unsigned f = __hip_atomic_fetch_add(&sf->fin, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        if (f == gridDim.x - 1) {
-            __hip_atomic_store(&sf->ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&sf->fin, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
 }
@@ -703,13 +711,12 @@ void lu_syncfree_w(hipStream_t s, const Structure &st, const PackedFactor<T> &pf
     const int n = st.n;
     T *tmp = static_cast<T *>(cfg.tmp);
     const int waves = std::max(1, std::min(cfg.waves, (n + 63) / 64));
-    k_sf_mark<T><<<grid_for(n, 256), 256, 0, s>>>(n, tmp, sc);
     k_sweep_syncfree<T, WF, false><<<waves, 64, 0, s>>>(n, st.rows_f.as<int>(), st.cnt_f.as<int>(),
-                                                          st.col_f.as<int>(), pf.af, pf.df, rhs, small, tmp, cfg.sf,
-                                                          sc);
-    k_sf_mark<T><<<grid_for(n, 256), 256, 0, s>>>(n, w, sc);
+                                                          st.col_f.as<int>(), pf.af, pf.df, rhs, small, tmp, w,
+                                                          cfg.sf, sc);
     k_sweep_syncfree<T, WB, true><<<waves, 64, 0, s>>>(n, st.rows_b.as<int>(), st.cnt_b.as<int>(),
-                                                         st.col_b.as<int>(), pf.ab, pf.db, tmp, small, w, cfg.sf, sc);
+                                                         st.col_b.as<int>(), pf.ab, pf.db, tmp, small, w, tmp, cfg.sf,
+                                                         sc);
 }
 
 template <class T, int WF>
@@ -771,6 +778,15 @@ void lu_launch64(hipStream_t s, const Structure &st, const double *a, const doub
 void lu_launch32(hipStream_t s, const Structure &st, const float *a, const float *d, float small, const float *rhs,
                  float *w, const Scalars *sc, const SweepCfg *cfg, const PackedFactor<float> *pf) {
     lu_launch_t<float>(s, st, a, d, small, rhs, w, sc, cfg, pf);
+}
+
+void mark_sweep_input64(hipStream_t s, int n, double *tmp) {
+    k_sf_mark<double><<<grid_for(n, 256), 256, 0, s>>>(n, tmp, nullptr);
+    FC_HIP_CHECK(hipGetLastError());
+}
+void mark_sweep_input32(hipStream_t s, int n, float *tmp) {
+    k_sf_mark<float><<<grid_for(n, 256), 256, 0, s>>>(n, tmp, nullptr);
+    FC_HIP_CHECK(hipGetLastError());
 }
 
 bool packed_sweeps(const Structure &st) { return st.levels_ready && st.ell_f > 0 && st.ell_b > 0; }

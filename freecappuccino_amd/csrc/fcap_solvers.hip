@@ -902,6 +902,11 @@ static PackedFactor<T> pack_for_solve(Ctx &c, const Structure &st, const T *a, c
         pf.ab = ab.as<T>();
         return pf;
     }
+    if (c.sw.sf) {
+        T *tmp = static_cast<T *>(c.sw.tmp);
+        if constexpr (f32) mark_sweep_input32(c.s, st.n, tmp);
+        else mark_sweep_input64(c.s, st.n, tmp);
+    }
     const size_t n = (size_t)st.n;
     af.ensure(sizeof(T) * n * (size_t)st.ell_f);
     ab.ensure(sizeof(T) * n * (size_t)st.ell_b);

@@ -806,3 +806,32 @@ def test_part_sweeps_bitwise_over_numberings(ctx, name, m):
         ctx.set_sweep_mode(fcap.SWEEP_DEFAULT)
         s.close()
     np.testing.assert_array_equal(out[0], out[1], err_msg=name)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("waves", [0, 1, 2, 7, 8, 9, 300])
+@pytest.mark.parametrize("mesh", ["tets", "box", "row"])
+def test_row_sweeps_bitwise_over_wave_counts(ctx, mesh, waves):
+    """The row-wise dependency-driven sweeps with fewer, as many and more waves than block
+    counters, and more than blocks: pairs of sweeps one after the other inside DIC-PCG, BiCGStab
+    and the mixed solver give the iterates of one launch per level bit for bit."""
+    m = {"tets": lambda: M.tet_box(6, permute_seed=3), "box": lambda: M.hex_box(13, 11, 7, perturb=0.1, seed=1),
+         "row": lambda: M.hex_box(70, 1, 1)}[mesh]()
+    su = np.random.default_rng(5).uniform(-1, 1, m.n_cells)
+    s = fcap.System(m, ctx)
+    out = {}
+    try:
+        ctx.set_sweep_waves(waves)
+        for mode in (fcap.SWEEP_DEPENDENT, fcap.SWEEP_LEVELS):
+            ctx.set_sweep_mode(mode)
+            for method in (fcap.METHOD_ICCG, fcap.METHOD_BICGSTAB, fcap.METHOD_ICCG_MIXED):
+                s.assemble_laplacian(np.full(m.n_cells, -1.0), None, su)
+                s.set_solution(np.zeros(m.n_cells))
+                s.solve(method, fcap.STOP_L2, 1e-8, 500)
+                out.setdefault(method, []).append(s.solution())
+    finally:
+        ctx.set_sweep_waves(0)
+        ctx.set_sweep_mode(fcap.SWEEP_DEFAULT)
+        s.close()
+    for method, (a, b) in out.items():
+        np.testing.assert_array_equal(a, b, err_msg=str(method))
