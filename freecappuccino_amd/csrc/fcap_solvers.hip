@@ -46,9 +46,8 @@ enum FinStep : int {
     kFinBicgEnd = 7,  // BiCGStab: resl, iteration count, convergence
     kFinOuter = 8,    // refinement: true residual norms
     kFinFcgBeta = 9,  // FCG: bet_s = -(z.q_s)/(p_s.q_s) for every stored direction s
-    kFinFcgPr = 10,   // FCG: p.r
-    kFinFcgAlf = 11,  // FCG: alf = p.r / p.q, p.q stored in this iteration's slot
-    kFinFcgEnd = 12   // FCG: residual, convergence, stagnation at the end of each window
+    kFinFcgAlf = 10,  // FCG: alf = p.r / p.q, p.q stored in this iteration's slot
+    kFinFcgEnd = 11   // FCG: residual, convergence, stagnation at the end of each window
 };
 
 // FCG stagnation: window length in fc_context::fcg_stag_window (64 by default)
@@ -68,7 +67,8 @@ __device__ inline void converge_test(Scalars *sc) {
     else if (sc->iters >= sc->nsw) { sc->done = 1; sc->status = FC_NOT_CONVERGED; }
 }
 
-__global__ __launch_bounds__(kFinBlock) void k_fin(int step, int nparts, const double *__restrict__ pa,
+// np2: partials of pb (nparts but where said)
+__global__ __launch_bounds__(kFinBlock) void k_fin(int step, int nparts, const double *__restrict__ pa, int np2,
                                                   const double *__restrict__ pb, Scalars *__restrict__ sc) {
     __shared__ double sh[kFinBlock / kWave];
     if (sc->done) return;
@@ -84,10 +84,9 @@ __global__ __launch_bounds__(kFinBlock) void k_fin(int step, int nparts, const d
         return;
     }
     double a = 0.0, b = 0.0;
-    for (int i = threadIdx.x; i < nparts; i += kFinBlock) {
-        a += pa[i];
-        if (pb) b += pb[i];
-    }
+    for (int i = threadIdx.x; i < nparts; i += kFinBlock) a += pa[i];
+    if (pb)
+        for (int i = threadIdx.x; i < np2; i += kFinBlock) b += pb[i];
     a = block_sum<kFinBlock>(a, sh);
     if (pb) b = block_sum<kFinBlock>(b, sh);
     if (threadIdx.x != 0) return;
@@ -140,12 +139,10 @@ __global__ __launch_bounds__(kFinBlock) void k_fin(int step, int nparts, const d
         sc->resl = a;
         sc->rel = sqrt(b / sc->bnorm2);
         break;
-    case kFinFcgPr:
-        sc->fcg_pr = a;
-        break;
-    case kFinFcgAlf:
+    case kFinFcgAlf:   // pb: the partials of p.r
+        sc->fcg_pr = b;
         sc->pkapk = a;
-        sc->alf = sc->fcg_pr / a;
+        sc->alf = b / a;
         sc->fcg_pqh[sc->iters % sc->fcg_m] = a;
         break;
     case kFinFcgEnd:
@@ -176,7 +173,12 @@ __global__ __launch_bounds__(kFinBlock) void k_fin(int step, int nparts, const d
 // (= sc->iters) the slots s < min(k, m) hold the directions of iterations
 // k-1, ..., k-min(k, m).
 
-// partials of z.q_s for every stored slot s, at pa[s * gridDim.x + block]; M = sc->fcg_m
+// Up to kFcgFold directions k_fcg_p adds the partials of their dot products itself, in every
+// block; more of them go through a finaliser (a launch of 5 us against 2 us a block).
+constexpr int kFcgFold = 4;
+
+// partials of z.q_s for every stored slot s, at pa[s * gridDim.x + block], or at
+// pa[M * block + s] for k_fcg_p; M = sc->fcg_m
 template <int M>
 __global__ __launch_bounds__(kRedBlock) void k_fcg_dots(int n, const float *__restrict__ z,
                                                         const float *__restrict__ qh, const Scalars *__restrict__ sc,
@@ -206,22 +208,31 @@ __global__ __launch_bounds__(kRedBlock) void k_fcg_dots(int n, const float *__re
     for (int s = 0; s < M; ++s) {
         if (s < nwin) {
             const double v = block_sum<kRedBlock>(acc[s], sh);
-            if (threadIdx.x == 0) pa[(size_t)s * gridDim.x + blockIdx.x] = v;
+            if (threadIdx.x == 0) pa[M <= kFcgFold ? (size_t)M * blockIdx.x + s : (size_t)s * gridDim.x + blockIdx.x] = v;
         }
     }
 }
 
-// p = z + sum_s bet_s p_s and the partial of p.r; M = sc->fcg_m
+// p = z + sum_s bet_s p_s (bet_s = -z.q_s / p_s.q_s) and the partial of p.r; M = sc->fcg_m
 template <int M>
 __global__ __launch_bounds__(kRedBlock) void k_fcg_p(int n, float *__restrict__ p, const float *__restrict__ z,
                                                      const float *__restrict__ r, const float *__restrict__ ph,
-                                                     const Scalars *__restrict__ sc, double *__restrict__ pa) {
-    __shared__ double sh[kRedBlock / kWave];
+                                                     const Scalars *__restrict__ sc, const double *__restrict__ pd,
+                                                     int nd, double *__restrict__ pa) {
+    constexpr bool kFold = M <= kFcgFold;
+    __shared__ double sh[(kFold ? M : 1) * (kRedBlock / kWave)];
     if (sc->done) return;
     const int nwin = min(sc->iters, M);
     float bet[M];
+    if constexpr (kFold) {
+        double t[M];
+        parts_total<kRedBlock, M, M>(pd, nd, sh, t);   // (those of slots not yet stored are not used)
 #pragma unroll
-    for (int s = 0; s < M; ++s) bet[s] = s < nwin ? (float)sc->fcg_bet[s] : 0.f;
+        for (int s = 0; s < M; ++s) bet[s] = s < nwin ? (float)(-t[s] / sc->fcg_pqh[s]) : 0.f;
+    } else {
+#pragma unroll
+        for (int s = 0; s < M; ++s) bet[s] = s < nwin ? (float)sc->fcg_bet[s] : 0.f;
+    }
     double acc = 0.0;
     if (nwin == M) {
         for (int i = blockIdx.x * kRedBlock + threadIdx.x; i < n; i += gridDim.x * kRedBlock) {
@@ -701,7 +712,7 @@ bool fused(const Ctx &c, const OcView &oc) { return !c.ctx->reduce_seq && !oc.no
 int fused_grid(int n) { return std::min(kVecGrid, grid_for(n, n >= 512 * 4 * kRedBlock ? 4 * kRedBlock : 2 * kRedBlock)); }
 
 void fin(Ctx &c, int step, int nparts, bool two) {
-    k_fin<<<1, kFinBlock, 0, c.s>>>(step, nparts, c.pa, two ? c.pb : nullptr, c.sc);
+    k_fin<<<1, kFinBlock, 0, c.s>>>(step, nparts, c.pa, nparts, two ? c.pb : nullptr, c.sc);
 }
 
 // Sums in index order, as the reference forms them (sum(res*zk), sum(abs(res)):
@@ -784,9 +795,12 @@ struct Events {
     }
 };
 
-void run_batches(Ctx &c, int per_graph, int launches, const std::function<void()> &iter) {
-    GraphExec ge;
-    if (c.ctx->use_graphs && c.s != nullptr) {
+// `kept`, when given, keeps the graph for the solve's next call with the same iterations
+// (refinement cycles: 170 us a cycle to capture one at 128^3).
+void run_batches(Ctx &c, int per_graph, int launches, const std::function<void()> &iter, GraphExec *kept = nullptr) {
+    GraphExec own;
+    GraphExec &ge = kept ? *kept : own;
+    if (!ge.exec && c.ctx->use_graphs && c.s != nullptr) {
         hipGraph_t g = nullptr;
         FC_HIP_CHECK(hipStreamBeginCapture(c.s, hipStreamCaptureModeThreadLocal));
         try {
@@ -1191,8 +1205,8 @@ fc_status solve_bicgstab64(fc_context *ctx, const SolveArgs &args, fc_solve_info
 // iteration (<= 0: none), on exit this cycle's.  With a previous value the search
 // direction p is kept and the first step continues it (beta = r.z / s0_carry), so
 // the refinement replaces the residual without discarding the Krylov direction.
-static int inner_solve32(Ctx &c, const Structure &st, const Matrix<float> &A, bool bicg, double eta, double r32norm2, int cap,
-                         const PackedFactor<float> *pf, double *s0_carry = nullptr) {
+static int inner_solve32(Ctx &c, const Structure &st, const Matrix<float> &A, bool bicg, double eta, double r32norm2,
+                         int cap, const PackedFactor<float> *pf, double *s0_carry, GraphExec &graph) {
     Workspace &ws = *c.ws;
     const int n = c.n;
     float *a32 = ws.a32.as<float>(), *d32 = ws.d32.as<float>();
@@ -1227,7 +1241,7 @@ static int inner_solve32(Ctx &c, const Structure &st, const Matrix<float> &A, bo
             const SpmvSums pq = spmv_sums(c, false);
             k_cg_xr<float, float, false><<<c.gf, kRedBlock, 0, c.s>>>(n, e, r, p, q, nullptr, c.sc, pq.a, pq.n, c.pv);
             precondition(0);
-        });
+        }, &graph);
     } else {
         float *reso = reinterpret_cast<float *>(ws.tmp.get());   // n floats fit in n doubles
         float *uk = q, *vk = reinterpret_cast<float *>(ws.vk.get());
@@ -1248,7 +1262,7 @@ static int inner_solve32(Ctx &c, const Structure &st, const Matrix<float> &A, bo
             const SpmvSums v = spmv_sums(c, true);
             k_bi_xr2<float, float><<<c.gf, kRedBlock, 0, c.s>>>(n, e, r, z, vk, reso, c.sc, v.a, v.b, v.n, c.pv);
             direction(0);
-        });
+        }, &graph);
     }
     Scalars hs = read_scalars(c);
     if (s0_carry) *s0_carry = bicg || hs.status != FC_OK ? 0.0 : hs.sk;
@@ -1279,6 +1293,7 @@ fc_status solve_mixed(fc_context *ctx, const SolveArgs &args, bool bicg, fc_solv
     int total_inner = 0, outer = 0;
     double res0 = 0.0, resl = 0.0, rel = 0.0;
     double scale = 1.0, s0c = 0.0;   // FP32 residual scale; r.z carried between PCG cycles
+    GraphExec graph;                 // the inner iterations, the same in every cycle
     fc_status status = FC_NOT_CONVERGED;
     ctx->timer.start(c.s);
     for (;;) {
@@ -1304,7 +1319,7 @@ fc_status solve_mixed(fc_context *ctx, const SolveArgs &args, bool bicg, fc_solv
         if (outer == 0 || bicg) scale = rn;
         k_scale_cast<<<c.gv, 256, 0, c.s>>>(n, r, ws.r32.as<float>(), 1.0 / scale);
         total_inner += inner_solve32(c, st, A, bicg, args.inner_eta, ho.rnorm2 / (scale * scale), cap,
-                                     pf.af ? &pf : nullptr, &s0c);
+                                     pf.af ? &pf : nullptr, &s0c, graph);
         k_refine<<<c.gv, 256, 0, c.s>>>(n, args.fi, ws.e32.as<float>(), scale);
         ++outer;
     }
@@ -1343,7 +1358,8 @@ static int fcg_window(const fc_context *ctx) {
 // Truncated FCG in FP32 on A e = r32 (unit-norm r32), preconditioner P.
 // Returns the inner status (FC_OK, FC_NOT_CONVERGED, FC_FALLBACK_USED on
 // stagnation, FC_ERR_NONFINITE) and adds the iterations to `iters`.
-static int inner_fcg32(Ctx &c, const Matrix<float> &A, const PrecondHook &P, double eta, int cap, int &iters) {
+static int inner_fcg32(Ctx &c, const Matrix<float> &A, const PrecondHook &P, double eta, int cap, int &iters,
+                       GraphExec &graph) {
     Workspace &ws = *c.ws;
     const int n = c.n;
     float *r = ws.r32.as<float>(), *z = ws.z32.as<float>(), *p = ws.p32.as<float>(), *q = ws.q32.as<float>();
@@ -1365,20 +1381,22 @@ static int inner_fcg32(Ctx &c, const Matrix<float> &A, const PrecondHook &P, dou
     upload_scalars(c, h);
     k_zero<float><<<c.gv, 256, 0, c.s>>>(n, e);
     // the window is compiled in (h.fcg_m is one of 4, 8, 12, 16: fcg_window)
+    const int gd = h.fcg_m <= kFcgFold ? c.gf : c.gv;
     auto dots = [&]() {
         switch (h.fcg_m) {
-        case 4: k_fcg_dots<4><<<c.gv, kRedBlock, 0, c.s>>>(n, z, qh, c.sc, c.pa); break;
-        case 8: k_fcg_dots<8><<<c.gv, kRedBlock, 0, c.s>>>(n, z, qh, c.sc, c.pa); break;
-        case 12: k_fcg_dots<12><<<c.gv, kRedBlock, 0, c.s>>>(n, z, qh, c.sc, c.pa); break;
-        default: k_fcg_dots<16><<<c.gv, kRedBlock, 0, c.s>>>(n, z, qh, c.sc, c.pa); break;
+        case 4: k_fcg_dots<4><<<gd, kRedBlock, 0, c.s>>>(n, z, qh, c.sc, c.pa); break;
+        case 8: k_fcg_dots<8><<<gd, kRedBlock, 0, c.s>>>(n, z, qh, c.sc, c.pa); break;
+        case 12: k_fcg_dots<12><<<gd, kRedBlock, 0, c.s>>>(n, z, qh, c.sc, c.pa); break;
+        default: k_fcg_dots<16><<<gd, kRedBlock, 0, c.s>>>(n, z, qh, c.sc, c.pa); break;
         }
+        if (h.fcg_m > kFcgFold) fin(c, kFinFcgBeta, gd, false);
     };
-    auto pupd = [&]() {
+    auto pupd = [&]() {   // the partials of p.r go to pb
         switch (h.fcg_m) {
-        case 4: k_fcg_p<4><<<c.gv, kRedBlock, 0, c.s>>>(n, p, z, r, ph, c.sc, c.pa); break;
-        case 8: k_fcg_p<8><<<c.gv, kRedBlock, 0, c.s>>>(n, p, z, r, ph, c.sc, c.pa); break;
-        case 12: k_fcg_p<12><<<c.gv, kRedBlock, 0, c.s>>>(n, p, z, r, ph, c.sc, c.pa); break;
-        default: k_fcg_p<16><<<c.gv, kRedBlock, 0, c.s>>>(n, p, z, r, ph, c.sc, c.pa); break;
+        case 4: k_fcg_p<4><<<gd, kRedBlock, 0, c.s>>>(n, p, z, r, ph, c.sc, c.pa, gd, c.pb); break;
+        case 8: k_fcg_p<8><<<gd, kRedBlock, 0, c.s>>>(n, p, z, r, ph, c.sc, nullptr, 0, c.pb); break;
+        case 12: k_fcg_p<12><<<gd, kRedBlock, 0, c.s>>>(n, p, z, r, ph, c.sc, nullptr, 0, c.pb); break;
+        default: k_fcg_p<16><<<gd, kRedBlock, 0, c.s>>>(n, p, z, r, ph, c.sc, nullptr, 0, c.pb); break;
         }
     };
     // The network runs on the first of every `period` iterations; the others take the
@@ -1389,11 +1407,9 @@ static int inner_fcg32(Ctx &c, const Matrix<float> &A, const PrecondHook &P, dou
     auto iter = [&]() {
         P.apply(P.obj, c.s, r, z, c.sc, light);
         dots();
-        fin(c, kFinFcgBeta, c.gv, false);
         pupd();
-        fin(c, kFinFcgPr, c.gv, false);
-        product(c, A, p, p, q, c.pa);
-        fin(c, kFinFcgAlf, gs, false);
+        product(c, A, p, p, q, c.pq);
+        k_fin<<<1, kFinBlock, 0, c.s>>>(kFinFcgAlf, gs, c.pq, gd, c.pb, c.sc);
         k_fcg_xr<<<c.gv, kRedBlock, 0, c.s>>>(n, e, r, p, q, ph, qh, c.sc, c.pa, c.pb);
         fin(c, kFinFcgEnd, c.gv, true);
     };
@@ -1403,7 +1419,7 @@ static int inner_fcg32(Ctx &c, const Matrix<float> &A, const PrecondHook &P, dou
             iter();
         }
     };
-    run_batches(c, 1, std::max(1, 2 / period), group);
+    run_batches(c, 1, std::max(1, 2 / period), group, &graph);
     Scalars hs = read_scalars(c);
     iters += hs.iters;
     return hs.status;
@@ -1429,6 +1445,7 @@ fc_status solve_fcg(fc_context *ctx, const SolveArgs &args, const PrecondHook &P
     int total_inner = 0, outer = 0, fallback_iters = 0;
     double res0 = 0.0, resl = 0.0, fallback_ms = 0.0;
     bool fell_back = false;
+    GraphExec graph;   // the inner iterations, the same in every cycle
     fc_status status = FC_NOT_CONVERGED;
     ctx->timer.start(c.s);
     for (;;) {
@@ -1449,7 +1466,7 @@ fc_status solve_fcg(fc_context *ctx, const SolveArgs &args, const PrecondHook &P
         const double rn = std::sqrt(ho.rnorm2);
         k_scale_cast<<<c.gv, 256, 0, c.s>>>(n, r, ws.r32.as<float>(), 1.0 / rn);
         const int cap = std::max(1, args.nsw - total_inner);
-        const int ist = inner_fcg32(c, A, P, args.inner_eta, cap, total_inner);
+        const int ist = inner_fcg32(c, A, P, args.inner_eta, cap, total_inner, graph);
         ++outer;
         if (ist == FC_FALLBACK_USED || ist == FC_ERR_NONFINITE) {
             // plain IC(0)-PCG (FP64) finishes the solve from the last refined iterate;
