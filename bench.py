@@ -9,7 +9,7 @@ perturbed by +-20% (seeded), spacing graded along x by ratio 1.05 toward the
 wall (aspect ratio capped at 100), mu = -1, Dirichlet wall at x = 0, RHS = 32
 seeded Gaussian blobs with zero mean.  Four solves run on the same system:
   * ic_pcg_fp64  -- IC(0)-PCG in FP64 (the reference's DIC-PCG; triangular sweeps
-                    with one launch per sweep, each row waiting for the rows it reads);
+                    with one launch per sweep over pencils of 64 lines);
   * ic_pcg_mixed -- FP32 DIC-PCG inside FP64 iterative refinement (same sweeps);
   * fcg_learned  -- flexible CG in FP32 preconditioned by the trained BF16
                     message-passing network followed by three damped-Jacobi
@@ -119,8 +119,9 @@ def calcp_step_bytes(n, nif, nnz, nb):
         "k_calcp_faces": nif * (16 + 56 + 24) + n * 24 * 8,
         # ptr, diag, a and su out; per off-diagonal slot kface (face and side) + a; per face flmass
         "k_calcp_rows": n * (8 + 16) + off * (4 + 8) + nif * 8,
-        # own, nei, geometry, (x, y, z)-products out; u, centre and previous gradient per cell
-        "k_grad_faces": nif * (8 + 56 + 24) + n * 7 * 8,
+        # own, nei, geometry, (x, y, z)-products out; u and centre per cell (the first pass, which
+        # reads no previous gradient)
+        "k_grad_faces": nif * (8 + 56 + 24) + n * 4 * 8,
         # ptr, diag, vol, gradient out; kface per slot; products per face; boundary faces
         # (owner list entry, S, value)
         "k_grad_rows": n * (8 + 8 + 24) + off * 4 + nif * 24 + nb * (4 + 24 + 8),

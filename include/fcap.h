@@ -417,9 +417,9 @@ fc_status fc_set_fcg_stagnation(fc_context *ctx, int window, double factor);
 enum { FC_SWEEP_LEVELS = 0, FC_SWEEP_DEPENDENT = 2, FC_SWEEP_PARTS = 3 };
 fc_status fc_set_sweep_mode(fc_context *ctx, int mode);
 /* Persistent waves of the dependency-driven sweeps and pivots (0: automatic --
- * one workgroup per compute unit for the part-wise sweeps, for the row-wise ones one
- * 64-row block per wave for an average level's rows, within 1 to 16 per compute
- * unit; at most 65,536).  No counterpart in the reference. */
+ * one workgroup per compute unit for the part-wise sweeps, for the row-wise ones two
+ * waves per 64-row block of an average level, within 1 to 16 per compute unit; at
+ * most 65,536).  No counterpart in the reference. */
 fc_status fc_set_sweep_waves(fc_context *ctx, int waves);
 /* Wall-clock limit of one wait of the dependency-driven sweeps, in
  * microseconds (0: the built-in 2 s).  A wait that runs past it ends the
