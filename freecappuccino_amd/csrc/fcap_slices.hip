@@ -26,8 +26,9 @@ inline int grid_for(long long n, int block) { return (int)std::max<long long>(1,
 __host__ __device__ inline int slices_of(int n) { return (n + kWave - 1) / kWave; }
 
 __global__ void k_row_width(int n, const int *__restrict__ ptr, int *__restrict__ w) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    int len = i < n ? ptr[i + 1] - ptr[i] : 0;
+    int len = 0;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+        len = max(len, ptr[i + 1] - ptr[i]);
 #pragma unroll
     for (int off = 32; off; off >>= 1) len = max(len, __shfl_xor(len, off));
     if ((threadIdx.x & 63) == 0) atomicMax(w, len);
@@ -172,7 +173,7 @@ SliceView slices_for(fc_context *ctx, Structure &st) {
         hipStream_t s = ctx->stream;
         DevBuf wd(sizeof(int));
         fill_int(ctx, wd.as<int>(), 1, 0);
-        k_row_width<<<grid_for(st.n, 256), 256, 0, s>>>(st.n, st.ioffset.as<int>(), wd.as<int>());
+        k_row_width<<<std::min(grid_for(st.n, 256), 256), 256, 0, s>>>(st.n, st.ioffset.as<int>(), wd.as<int>());
         int w = 0;
         FC_HIP_CHECK(hipMemcpyAsync(&w, wd.get(), sizeof(int), hipMemcpyDeviceToHost, s));
         FC_HIP_CHECK(hipStreamSynchronize(s));
