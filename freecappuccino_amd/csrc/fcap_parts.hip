@@ -177,6 +177,9 @@ template <int W> struct PartShape {
     static constexpr int kPollers = W <= 3 ? 6 : W <= 4 ? 5 : 4;
     static constexpr int kStage = kFeeders * kBatch;
     static constexpr int kBlock = 64 * (1 + kPollers + kFeeders);
+    // a window's values are read from the ring at the latest when the window kStage further
+    // is staged, so at most kStage - 1 windows have been written since
+    static_assert(kStage <= kRing / 64, "the ring holds every window that is not retired");
 };
 
 template <class T, int W>
@@ -281,16 +284,23 @@ __device__ __forceinline__ bool part_finished(const PartLds<T, W> &L, int j) {
     return true;
 }
 
-// the results of a finished window that need not be early
+// The backward sweep's value of this lane's row in a finished window, while the ring holds
+// it: a window's slots are written again kRing / 64 windows later.
 template <class T, int W, bool BWD>
-__device__ __forceinline__ void part_retire(const PartRun<T> &R, const PartLds<T, W> &L, int j, int row) {
+__device__ __forceinline__ T part_result(const PartRun<T> &R, const PartLds<T, W> &L, int j) {
+    const int q = R.template at<BWD>(j) * 64 + (int)(threadIdx.x & 63);
+    return BWD ? L.x[q & (kRing - 1)] : T(0);
+}
+
+// the results of a finished window that need not be early
+template <class T, bool BWD>
+__device__ __forceinline__ void part_retire(const PartRun<T> &R, int j, int row, T result) {
     using U = typename SfBits<T>::U;
-    const int lane = threadIdx.x & 63;
-    const int q = R.template at<BWD>(j) * 64 + lane;
+    const int q = R.template at<BWD>(j) * 64 + (int)(threadIdx.x & 63);
     // the other direction's output takes its mark for the next sweep: the forward sweep
     // marks the backward one's slots, the backward sweep those it has read
     reinterpret_cast<U *>(R.mk)[q] = SfBits<T>::kMark;
-    if (BWD) R.z[row] = L.x[q & (kRing - 1)];
+    if (BWD) R.z[row] = result;
 }
 
 template <class T, int W>
@@ -343,14 +353,18 @@ __device__ __forceinline__ void part_feed(const PartRun<T> &R, PartLds<T, W> &L,
 #pragma unroll
         for (int u = 0; u < B; ++u) {
             const int j = j0 + u;
-            if (j < R.nw) {
-                T vals[W + 2];
+            T vals[W + 2];
 #pragma unroll
-                for (int k = 0; k < W; ++k) vals[k] = cur[u].val[k];
-                vals[W] = cur[u].val[W];
-                vals[W + 1] = BWD ? rhs[u] / (cur[u].val[W] + R.small) : rhs[u];
-                // room in the stage
-                if (!part_finished(L, j - K)) return;
+            for (int k = 0; k < W; ++k) vals[k] = cur[u].val[k];
+            vals[W] = cur[u].val[W];
+            vals[W + 1] = BWD ? rhs[u] / (cur[u].val[W] + R.small) : rhs[u];
+            // room in the stage
+            if (!part_finished(L, j - K)) return;
+            // Window j - kStage, which this wave fed too, is finished.  Its values are read
+            // before window j is staged: from then on the chain runs on as far as the other
+            // feeders have staged, past where the ring holds them.
+            const T result = before >= 0 ? part_result<T, W, BWD>(R, L, j - K) : T(0);
+            if (j < R.nw) {
                 const int slot = j % K;
                 const int xbase = kRing + 2 + slot * W * 64 + lane;
                 int ints[W + 1];
@@ -366,11 +380,8 @@ __device__ __forceinline__ void part_feed(const PartRun<T> &R, PartLds<T, W> &L,
                 stage_put<T, W>(L.stage[slot], lane, ints, vals);
                 lds_order();
                 lds_set(&L.fed[slot], j + 1);
-            } else if (before >= 0 && !part_finished(L, j - K)) {
-                return;
             }
-            // window j - kStage, which this wave fed too, is finished
-            if (before >= 0) part_retire<T, W, BWD>(R, L, j - K, row[u]);
+            if (before >= 0) part_retire<T, BWD>(R, j - K, row[u], result);
         }
         before = j0;
 #pragma unroll
@@ -385,7 +396,7 @@ __device__ __forceinline__ void part_feed(const PartRun<T> &R, PartLds<T, W> &L,
     for (int u = 0; u < B; ++u) {
         if (before + u < R.nw) {
             if (!part_finished(L, before + u)) return;
-            part_retire<T, W, BWD>(R, L, before + u, row[u]);
+            part_retire<T, BWD>(R, before + u, row[u], part_result<T, W, BWD>(R, L, before + u));
         }
     }
 }
@@ -503,8 +514,8 @@ __device__ __forceinline__ bool part_step(PartLds<T, W> &L, Chain<T, W> &c, cons
         const int step = o.i[W] & 255;
         v = T(0);
         for (int st = 0; st <= top; ++st) {
+            lds_order();
             if (step == st) {
-                lds_order();
 #pragma unroll
                 for (int k = 0; k < W; ++k) x[k] = *reinterpret_cast<const T *>(xs + o.i[k]);
                 v = part_row<T, W>(o, x);

@@ -1,0 +1,76 @@
+// The library's kernels on the CPU (wave_emu.h): their text, cut from the sources by the test
+// that builds this file, and an entry point for each.
+#include "fcap.h"
+#include "fcap_kernels.h"
+
+namespace fcap {
+#include "cut_syncfree.inc"
+namespace parts {
+#include "cut_parts.inc"
+}
+}  // namespace fcap
+
+using namespace fcap;
+
+namespace {
+
+struct Run {
+    int grid, seed, resident, freeze_steps;
+    double freeze, freeze_store;
+    long long wait_ticks, max_steps;
+    const unsigned *order;   // or null
+};
+emu::Policy policy(const Run &r) {
+    emu::Policy p;
+    p.seed = (unsigned)r.seed;
+    p.freeze = r.freeze;
+    p.freeze_store = r.freeze_store;
+    p.freeze_steps = r.freeze_steps;
+    if (r.resident > 0) p.resident = (unsigned)r.resident;
+    if (r.order) p.order.assign(r.order, r.order + r.grid);
+    p.max_steps = r.max_steps;
+    return p;
+}
+SyncFree state(const Run &r) {
+    SyncFree sf{};
+    sf.wait_us = (int)r.wait_ticks;
+    sf.rate_khz = 1000;
+    return sf;
+}
+
+template <class T, int W, bool BWD>
+int parts_sweep(const Run &r, int nparts, int npk, const int *codes, const unsigned char *step, const int *win,
+                const T *vals, const T *in, double small, T *out, T *mk, T *z) {
+    SyncFree sf = state(r);
+    const parts::PartView P{npk, codes, step};
+    const bool ended = emu::launch((unsigned)r.grid, parts::PartShape<W>::kBlock, policy(r), [&]() {
+        parts::k_sweep_parts<T, W, BWD>(nparts, P, win, vals, in, (T)small, out, mk, z, &sf, nullptr);
+    });
+    return !ended ? 2 : sf.abort ? 1 : 0;
+}
+template <class T, int W>
+int parts_either(const Run &r, int bwd, int nparts, int npk, const int *codes, const unsigned char *step,
+                 const int *win, const void *vals, const void *in, double small, void *out, void *mk, void *z) {
+    auto f = [&](auto b) {
+        return parts_sweep<T, W, decltype(b)::value>(r, nparts, npk, codes, step, win, (const T *)vals, (const T *)in,
+                                                     small, (T *)out, (T *)mk, (T *)z);
+    };
+    return bwd ? f(std::true_type{}) : f(std::false_type{});
+}
+
+}  // namespace
+
+extern "C" {
+
+int emu_ring() { return parts::kRing; }
+
+int emu_parts(const Run *r, int f32, int width, int bwd, int nparts, int npk, const int *codes,
+              const unsigned char *step, const int *win, const void *vals, const void *in, double small, void *out,
+              void *mk, void *z) {
+#define CALL(T, W) parts_either<T, W>(*r, bwd, nparts, npk, codes, step, win, vals, in, small, out, mk, z)
+    if (f32) return width == 3 ? CALL(float, 3) : width == 4 ? CALL(float, 4) : CALL(float, 8);
+    return width == 3 ? CALL(double, 3) : width == 4 ? CALL(double, 4) : CALL(double, 8);
+#undef CALL
+}
+
+}  // extern "C"

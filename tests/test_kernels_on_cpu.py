@@ -1,0 +1,124 @@
+"""What the waves of the solvers' kernels may do to each other, on the CPU: the kernels' own text is
+compiled for the CPU (tests/emulate) and run under a scheduler that takes the waves in any order and
+leaves some aside for long times.  The results must not depend on it."""
+import ctypes as C
+import os
+import re
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+import part_model as P
+from freecappuccino_amd import mesh as M
+from oracle import oracle as O
+
+ROOT = os.path.abspath(os.path.join(os.path.dirname(__file__), ".."))
+CSRC = os.path.join(ROOT, "freecappuccino_amd", "csrc")
+EMULATE = os.path.join(ROOT, "tests", "emulate")
+CLANG = shutil.which("clang++") or "/opt/rocm/llvm/bin/clang++"
+MARK = {8: 0x7FF4DEADBEEF0001, 4: 0x7FA0BEEF}
+
+
+def _cut(name, start, end):
+    with open(os.path.join(CSRC, name)) as f:
+        text = f.read()
+    i = text.index(start)
+    return text[i:text.index(end, i)]
+
+
+def _cuts():
+    yield "cut_syncfree.inc", (_cut("fcap_linalg.h", "constexpr int kSfTickets", "// zeroed state") +
+                               _cut("fcap_syncfree.h", "// A wait is bounded", "}  // namespace fcap"))
+    # (the compiler barrier that keeps a wave's LDS accesses in order is a meeting of its lanes here)
+    yield "cut_parts.inc", re.sub(r'__asm__ volatile\("" ::: "memory"\);', "emu::meet(emu::kPoint);",
+                                  _cut("fcap_parts.hip", "constexpr int kBlock", "// " + "-" * 65 + " analysis"))
+
+
+class Run(C.Structure):
+    _fields_ = [("grid", C.c_int), ("seed", C.c_int), ("resident", C.c_int), ("freeze_steps", C.c_int),
+                ("freeze", C.c_double), ("freeze_store", C.c_double), ("wait_ticks", C.c_longlong), ("max_steps", C.c_longlong),
+                ("order", C.c_void_p)]
+
+
+def _run(grid, seed=1, freeze=0.0, freeze_store=0.0, freeze_steps=1, resident=0, wait_ticks=10**9, max_steps=3 * 10**6, order=None):
+    return Run(grid, seed, resident, freeze_steps, freeze, freeze_store, wait_ticks, max_steps,
+               None if order is None else order.ctypes.data)
+
+
+@pytest.fixture(scope="module")
+def emu(tmp_path_factory):
+    if not os.path.exists(CLANG):
+        pytest.skip("no clang++")
+    d = str(tmp_path_factory.mktemp("emulate"))
+    for name, text in _cuts():
+        with open(os.path.join(d, name), "w") as f:
+            f.write(text)
+    lib = os.path.join(d, "kernels.so")
+    p = subprocess.run([CLANG, "-std=c++17", "-O1", "-fPIC", "-shared", "-ffp-contract=off", "-w", "-I", d, "-I",
+                        EMULATE, "-I", CSRC, "-I", os.path.join(ROOT, "include"),
+                        os.path.join(EMULATE, "kernels.cpp"), "-o", lib], capture_output=True, text=True)
+    assert p.returncode == 0, p.stderr[-4000:]
+    return C.CDLL(lib)
+
+
+def _matrix(ioffset, ja, diag, seed):
+    """The structure as the oracle takes it, symmetric values and a right-hand side."""
+    csr = O.CSR(ioffset, ja, diag, np.zeros(0, np.int32), np.zeros(0, np.int32))
+    rng = np.random.default_rng(seed)
+    n = len(diag)
+    row = np.repeat(np.arange(n), np.diff(ioffset))
+    key = np.minimum(row, ja - 1) * n + np.maximum(row, ja - 1)
+    a = -rng.uniform(0.5, 1.0, key.size)[np.unique(key, return_inverse=True)[1]]
+    a[diag - 1] = 20.0 + rng.uniform(0, 1, n)
+    return csr, a, rng.standard_normal(n)
+
+
+def _mesh(m):
+    csr = O.csr_build(m.n_cells, m.owner[:m.n_inner] + 1, m.neighbour + 1)
+    return csr.ioffset, csr.ja, csr.diag
+
+
+def _ptr(x):
+    return x.ctypes.data_as(C.c_void_p)
+
+
+def _part_sweeps(emu, s, width, a, d, r, small, dtype, run):
+    """Both sweeps of the schedule s; (result, forward's and backward's outputs after it, return codes)."""
+    mark = np.uint64(MARK[8]) if dtype == np.float64 else np.uint32(MARK[4])
+    marks = lambda: np.full(s.npk, mark).view(dtype)  # noqa: E731
+    tmp, zp, z = marks(), np.zeros(s.npk, dtype), np.zeros(len(r), dtype)
+    rhs, rc = r.astype(dtype), []
+    for upper, (src, out, mk) in enumerate(((rhs, tmp, zp), (tmp, zp, tmp))):
+        codes = P.packed(s.codes(bool(upper), width, emu.emu_ring()))
+        vals = P.packed(s.values(bool(upper), width, a, d, dtype))
+        rc.append(emu.emu_parts(C.byref(run), dtype == np.float32, width, upper, s.nparts, s.npk, _ptr(codes),
+                                _ptr(s.step), _ptr(s.win), _ptr(vals), _ptr(src), C.c_double(small), _ptr(out),
+                                _ptr(mk), _ptr(z)))
+    return z, tmp, mark, rc
+
+
+def _cases():
+    yield "pencils", _mesh(M.hex_box(70, 13, 7)), 3, P.pencil_parts
+    yield "runs", _mesh(M.tet_box(8)), 4, lambda *zero: P.run_parts(*zero, 2100)
+    yield "wide", P.stencil((6, 6, 65), P.STEPS8), 8, lambda *zero: P.run_parts(*zero, 1900)
+
+
+@pytest.mark.parametrize("name,structure,width,parts", list(_cases()), ids=lambda v: v if isinstance(v, str) else "")
+def test_part_sweeps_whatever_the_waves_do(emu, name, structure, width, parts):
+    """Feeders, pollers and the chain wave left aside at any point of theirs, above all behind a flag
+    they set: the oracle's sweeps bit for bit, and the forward sweep's output marked again.  (Read from
+    the ring behind its flag, a feeder's result was that of a window sixteen further on.)"""
+    csr, a, r = _matrix(*structure, 3)
+    zero = csr.ioffset - 1, csr.ja - 1, csr.diag - 1
+    s = P.Schedule(*zero, *parts(*zero))
+    assert s.nparts > 1 and np.diff(s.win).max() > 32
+    d = O.dic_pivots(csr, a)
+    ref = O.lu_apply(csr, a, d, r)
+    for seed in range(8):
+        run = _run(grid=min(s.nparts, 3), seed=seed, freeze=0.003, freeze_store=0.03, freeze_steps=3000)
+        z, tmp, mark, rc = _part_sweeps(emu, s, width, a, d, r, 1e-20, np.float64, run)
+        assert rc == [0, 0], rc
+        np.testing.assert_array_equal(z, ref, err_msg=f"seed {seed}")
+        assert np.all(tmp.view(mark.dtype) == mark)
