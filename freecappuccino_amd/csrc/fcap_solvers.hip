@@ -389,6 +389,15 @@ __device__ inline void record_end(Scalars *sc, double a, double b, double rsm, d
     }
 }
 
+// Whether the solve has ended, for a kernel whose first block may set `done` while others still
+// begin: read once a block, so a block goes on or returns as a whole (one that goes on comes to
+// the same end by its own test, and returns there).
+__device__ inline bool ended(const Scalars *sc, int *sh) {
+    if (threadIdx.x == 0) *sh = sc->done;
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(*sh) != 0;
+}
+
 // Partials of the fused vector kernels: block b's |r|_1, |r|_2^2 and r.z (or res.reso) at
 // pv[kVecParts b ..]; one reduction adds what a kernel needs of them.
 __device__ inline void vec_part(double *pv, double a, double b, double c) {
@@ -435,7 +444,8 @@ __global__ __launch_bounds__(kRedBlock) void k_cg_p(int n, T *__restrict__ p, co
                                                    const double *__restrict__ pv, int nv,
                                                    const double *__restrict__ pz, int nz, int first) {
     __shared__ double sh[kVecShared];
-    if (sc->done) return;
+    __shared__ int stop;
+    if (ended(sc, &stop)) return;
     const bool rec = blockIdx.x == 0 && threadIdx.x == 0;
     double t[3];
     if (JAC || !first) parts_total<kRedBlock, 3, kVecParts>(pv, nv, sh, t);
@@ -496,7 +506,8 @@ __global__ __launch_bounds__(kRedBlock) void k_bi_p(int n, T *__restrict__ pk, c
                                                    const T *__restrict__ uk, Scalars *__restrict__ sc,
                                                    const double *__restrict__ pv, int nv, int first) {
     __shared__ double sh[kVecShared];
-    if (sc->done) return;
+    __shared__ int stop;
+    if (ended(sc, &stop)) return;
     const bool rec = blockIdx.x == 0 && threadIdx.x == 0;
     double t[3];
     parts_total<kRedBlock, 3, kVecParts>(pv, nv, sh, t);

@@ -8,6 +8,9 @@ namespace fcap {
 namespace parts {
 #include "cut_parts.inc"
 }
+namespace solver {
+#include "cut_solver.inc"
+}
 }  // namespace fcap
 
 using namespace fcap;
@@ -61,6 +64,29 @@ int parts_either(const Run &r, int bwd, int nparts, int npk, const int *codes, c
 }  // namespace
 
 extern "C" {
+
+// the kernels that begin an iteration and end the solve (k_cg_p<float>, k_bi_p<float>), with
+// residual sums a, b in every one of the nv partials; what they leave of `done` and the direction
+int emu_begin(const Run *r, int bicg, int n, float *p, const float *z, double a, double b, double resmax, int nv,
+              int *done) {
+    Scalars sc{};
+    sc.resmax = resmax;
+    sc.res0 = sc.sk = sc.gam = sc.alf = sc.beto = 1.0;
+    sc.nsw = 100;
+    sc.status = kStatusRunning;
+    std::vector<double> pv((size_t)kVecParts * nv), pz(nv, 1.0);
+    for (int i = 0; i < nv; ++i) {
+        pv[(size_t)kVecParts * i] = a;
+        pv[(size_t)kVecParts * i + 1] = b;
+        pv[(size_t)kVecParts * i + 2] = 1.0;
+    }
+    const bool ended = emu::launch((unsigned)r->grid, kRedBlock, policy(*r), [&]() {
+        if (bicg) solver::k_bi_p<float>(n, p, z, z, &sc, pv.data(), nv, 0);
+        else solver::k_cg_p<float, false>(n, p, z, nullptr, &sc, pv.data(), nv, pz.data(), nv, 0);
+    });
+    *done = sc.done;
+    return !ended;
+}
 
 int emu_ring() { return parts::kRing; }
 

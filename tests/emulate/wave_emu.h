@@ -80,7 +80,7 @@ struct Block {
 
 struct Policy {
     unsigned seed = 1;
-    double freeze = 0.0;           // chance that a wave is left aside after a step,
+    double freeze = 0.0;           // chance that a wave is left aside after a step (one in three starts late),
     double freeze_store = 0.0;     // and after a workgroup-scope store (a flag just set)
     int freeze_steps = 0;          // for at most so many steps
     std::vector<unsigned> order;   // workgroups in the order in which they become resident
@@ -173,6 +173,7 @@ inline bool launch(unsigned grid, unsigned threads, Policy p, const std::functio
         for (size_t w = 0; w < b->waves.size(); ++w) {
             Wave &wv = b->waves[w];
             wv.block = b.get();
+            if (p.freeze > 0 && rng() % 3 == 0) wv.frozen = clock_steps + rng() % (unsigned)p.freeze_steps;
             wv.lanes.resize(std::min(64u, threads - 64 * (unsigned)w));
             for (size_t l = 0; l < wv.lanes.size(); ++l) {
                 Lane &ln = wv.lanes[l];

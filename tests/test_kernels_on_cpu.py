@@ -34,6 +34,7 @@ def _cuts():
     # (the compiler barrier that keeps a wave's LDS accesses in order is a meeting of its lanes here)
     yield "cut_parts.inc", re.sub(r'__asm__ volatile\("" ::: "memory"\);', "emu::meet(emu::kPoint);",
                                   _cut("fcap_parts.hip", "constexpr int kBlock", "// " + "-" * 65 + " analysis"))
+    yield "cut_solver.inc", _cut("fcap_solvers.hip", "// the end of an iteration with", "// " + "-" * 65 + " helpers")
 
 
 class Run(C.Structure):
@@ -122,3 +123,25 @@ def test_part_sweeps_whatever_the_waves_do(emu, name, structure, width, parts):
         assert rc == [0, 0], rc
         np.testing.assert_array_equal(z, ref, err_msg=f"seed {seed}")
         assert np.all(tmp.view(mark.dtype) == mark)
+
+
+@pytest.mark.parametrize("bicg", [0, 1])
+@pytest.mark.parametrize("converged", [True, False])
+def test_every_block_ends_the_solve_alike(emu, bicg, converged):
+    """The kernel that begins an iteration tests for convergence in every block, and one block sets
+    `done`, which all of them read first.  Whatever waves are late, the direction is whole: as it was
+    where the solve ends (the refinement cycles carry it on), every entry new where it goes on."""
+    n, grid, nv = 2000, 4, 40
+    rng = np.random.default_rng(2)
+    p0, z = rng.standard_normal((2, n)).astype(np.float32)
+    want, done = None, C.c_int()
+    for seed in range(60):
+        p = p0.copy()
+        run = _run(grid, seed=seed, freeze=0.0 if seed == 0 else 0.05, freeze_steps=400)
+        assert emu.emu_begin(C.byref(run), bicg, n, _ptr(p), _ptr(z), C.c_double(1e-6 if converged else 1.0),
+                             C.c_double(1.0), C.c_double(1e-3), nv, C.byref(done)) == 0
+        assert done.value == converged
+        if seed == 0:
+            want = p0 if converged else p.copy()
+            assert converged or np.all(p != p0)
+        np.testing.assert_array_equal(p, want, err_msg=f"seed {seed}")
