@@ -458,12 +458,22 @@ void pack_factor_t(hipStream_t s, const Structure &st, const T *a, const T *d, T
 
 // ------------------------------------------- dependency-driven sweeps
 // One launch per sweep.  Persistent one-wave workgroups take blocks of 64
-// consecutive packed rows (level order) from ticket counters: workgroup g from counter
-// g % K (K = kSfTickets, or the grid if smaller), which hands out blocks g % K, + K, ...
-// in turn.  The smallest unfinished block has been handed out, or a running wave of its
-// counter takes it next (the first K workgroups start first), so the waits always end.
-// One counter for all cost 10 ns a ticket one after the other: with marks in launches of
-// their own 34 us a sweep on the 24^3 tets, now 25, on the 40^3 tets 90 and 39.  A sweep clears the other direction's counters.  The output starts filled with a
+// consecutive packed rows (level order) from kSfTickets ticket counters: counter c
+// hands out blocks c, c + kSfTickets, ... in turn, workgroup g takes from counter
+// g % kSfTickets.  (One counter for all cost 10 ns a ticket one after the other: with
+// marks in launches of their own 34 us a sweep on the 24^3 tets, now 25, on the 40^3
+// tets 90 and 39.)  A sweep clears the other direction's counters.
+//
+// The waits end whichever workgroups run: the smallest unfinished block has only
+// finished inputs, so the wave that holds it goes on; and if none has taken it, because
+// its counter's workgroups have not started, every wave that waits comes to take it --
+// one whose inputs are late sets its block aside and takes the smallest block before it
+// that is left, from whichever counter.  A block set aside is begun anew later; the
+// blocks a wave holds are of different counters (a counter's later blocks are larger),
+// so there are at most kSfTickets of them.  Fewer workgroups than counters take from all
+// of them from the start.
+//
+// The output starts filled with a
 // signalling-NaN pattern that arithmetic never produces; a row polls the
 // outputs of the rows it reads until none holds the pattern, computes exactly
 // as k_fwd_packed / k_bwd_packed (same operands, same order), and stores its
@@ -487,10 +497,28 @@ __global__ void k_sf_mark(int n, T *__restrict__ w, const Scalars *__restrict__ 
     reinterpret_cast<U *>(w)[i] = SfBits<T>::kMark;
 }
 
-// The other sweep's output takes its marks here: the forward sweep marks w, whose values
-// are spent, the backward one its right-hand side once read (a pass of its own for each
-// took 4.4 us on 83 K rows, beside sweeps of 26 us); mark_sweep_input does it before the
-// first sweep.
+// Takes the smallest block below `limit` that is left, from any counter; `limit`: there is none.
+__device__ inline unsigned sf_take_before(unsigned (*tickets)[32], unsigned limit) {
+    const unsigned lane = threadIdx.x, c = lane & (kSfTickets - 1);
+    for (;;) {
+        unsigned t = __hip_atomic_load(&tickets[c][0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned mine = t * kSfTickets + c;
+        unsigned least = mine;
+#pragma unroll
+        for (int off = kSfTickets / 2; off > 0; off >>= 1) least = min(least, (unsigned)__shfl_xor(least, off));
+        if (least >= limit) return limit;
+        bool got = false;
+        if (lane < kSfTickets && mine == least)
+            got = __hip_atomic_compare_exchange_strong(&tickets[c][0], &t, t + 1u, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                       __HIP_MEMORY_SCOPE_AGENT);
+        if (__any(got)) return least;   // else another wave has moved that counter on
+    }
+}
+
+// The other sweep's output takes its marks here, behind the block's values (a block set
+// aside reads its operands again): the forward sweep marks w, whose values are spent, the
+// backward one its right-hand side (a pass of its own for each took 4.4 us on 83 K rows,
+// beside sweeps of 26 us); mark_sweep_input does it before the first sweep.
 // BWD == false: out[i] = (rhs[i] - sum a w) d over the strict lower triangle;
 // BWD == true:  out[i] = (fwd[i] / (d + small) - sum a w) d over the strict upper one.
 template <class T, int W, bool BWD>
@@ -504,14 +532,26 @@ __global__ __launch_bounds__(64) void k_sweep_syncfree(int n, const int *__restr
     const int lane = threadIdx.x;
     const unsigned nblk = (unsigned)((n + 63) / 64);
     const unsigned long long limit = sf_wait_ticks(sf, sf->rate_khz);
-    const unsigned counters = min((unsigned)kSfTickets, gridDim.x), mine = blockIdx.x % counters;
-    unsigned *ticket = &sf->tickets[BWD][mine][0];
+    const unsigned mine = blockIdx.x % kSfTickets;
+    const bool few = gridDim.x < kSfTickets;
+    // after how many polls (less one) a wave looks for a block to compute first: a level takes
+    // one or two
+    const int patience = few ? 0 : 63;
+    unsigned aside = 0;   // the blocks set aside: the k-th in lane k
+    int naside = 0;
     if (blockIdx.x == 0 && lane < kSfTickets)
         __hip_atomic_store(&sf->tickets[!BWD][lane][0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (;;) {
         unsigned b = 0;
-        if (lane == 0) b = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        b = __shfl(b, 0) * counters + mine;
+        if (naside > 0) {
+            b = __shfl(aside, --naside);
+        } else if (few) {
+            b = sf_take_before(sf->tickets[BWD], nblk);
+        } else {
+            if (lane == 0)
+                b = __hip_atomic_fetch_add(&sf->tickets[BWD][mine][0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            b = __shfl(b, 0) * kSfTickets + mine;
+        }
         if (b >= nblk) break;
         const int p = (int)b * 64 + lane;
         bool done = p >= n;
@@ -531,10 +571,10 @@ __global__ __launch_bounds__(64) void k_sweep_syncfree(int n, const int *__restr
                 wk[k] = T(0);
             }
             acc = BWD ? in[i] / (di + small) : in[i];
-            reinterpret_cast<U *>(mk)[i] = SfBits<T>::kMark;   // behind the load of in[i] (mk may be in)
         }
         int spins = 0;
         const unsigned long long t0 = wall_clock64();
+        unsigned before = b;   // a block taken to be computed first
         for (;;) {
             if (!done) {
                 bool all = true;
@@ -572,8 +612,16 @@ __global__ __launch_bounds__(64) void k_sweep_syncfree(int n, const int *__restr
                 if (lane == 0) __hip_atomic_store(&sf->abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 break;
             }
+            if ((spins & patience) == 0 && (before = sf_take_before(sf->tickets[BWD], b)) < b) break;
             __builtin_amdgcn_s_sleep(1);
         }
+        if (before < b) {
+            if (lane == naside) aside = b;
+            if (lane == naside + 1) aside = before;
+            naside += 2;
+            continue;
+        }
+        if (p < n) reinterpret_cast<U *>(mk)[i] = SfBits<T>::kMark;
     }
 }
 

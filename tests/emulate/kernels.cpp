@@ -8,6 +8,9 @@ namespace fcap {
 namespace parts {
 #include "cut_parts.inc"
 }
+namespace rows {
+#include "cut_rows.inc"
+}
 namespace solver {
 #include "cut_solver.inc"
 }
@@ -39,6 +42,23 @@ SyncFree state(const Run &r) {
     sf.wait_us = (int)r.wait_ticks;
     sf.rate_khz = 1000;
     return sf;
+}
+
+template <int W>
+int rows_sweeps(const Run &r, int n, const int *const rows[2], const int *const cnt[2], const int *const col[2],
+                const double *const val[2], const double *const piv[2], const double *rhs, double small, double *tmp,
+                double *w) {
+    SyncFree sf = state(r);
+    bool ended = emu::launch((unsigned)r.grid, 64, policy(r), [&]() {
+        rows::k_sweep_syncfree<double, W, false>(n, rows[0], cnt[0], col[0], val[0], piv[0], rhs, small, tmp, w, &sf,
+                                                 nullptr);
+    });
+    if (ended && !sf.abort)
+        ended = emu::launch((unsigned)r.grid, 64, policy(r), [&]() {
+            rows::k_sweep_syncfree<double, W, true>(n, rows[1], cnt[1], col[1], val[1], piv[1], tmp, small, w, tmp,
+                                                    &sf, nullptr);
+        });
+    return !ended ? 2 : sf.abort ? 1 : 0;
 }
 
 template <class T, int W, bool BWD>
@@ -86,6 +106,13 @@ int emu_begin(const Run *r, int bicg, int n, float *p, const float *z, double a,
     });
     *done = sc.done;
     return !ended;
+}
+
+int emu_rows(const Run *r, int width, int n, const int *const rows[2], const int *const cnt[2], const int *const col[2],
+             const double *const val[2], const double *const piv[2], const double *rhs, double small, double *tmp,
+             double *w) {
+    if (width == 3) return rows_sweeps<3>(*r, n, rows, cnt, col, val, piv, rhs, small, tmp, w);
+    return rows_sweeps<8>(*r, n, rows, cnt, col, val, piv, rhs, small, tmp, w);
 }
 
 int emu_ring() { return parts::kRing; }

@@ -272,6 +272,15 @@ template <class T, class V> inline T add(T *p, V v) {
     return old;
 }
 
+template <class T, class V> inline bool cas(T *p, T *expected, V v) {
+    if (*p == *expected) {
+        *p = (T)v;
+        return true;
+    }
+    *expected = *p;
+    return false;
+}
+
 }  // namespace emu
 
 struct int4 { int x, y, z, w; };
@@ -292,6 +301,7 @@ inline int4 make_int4(int x, int y, int z, int w) { return {x, y, z, w}; }
 #define __hip_atomic_load(p, order, scope) emu::load(p)
 #define __hip_atomic_store(p, v, order, scope) emu::store(p, v, scope)
 #define __hip_atomic_fetch_add(p, v, order, scope) emu::add(p, v)
+#define __hip_atomic_compare_exchange_strong(p, e, v, order, order2, scope) emu::cas(p, e, v)
 #define atomicAdd(p, v) emu::add(p, v)
 #define atomicOr(p, v) (*(p) |= (v))
 #define __builtin_amdgcn_readfirstlane(v) emu::first(v)

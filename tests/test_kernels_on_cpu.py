@@ -34,6 +34,8 @@ def _cuts():
     # (the compiler barrier that keeps a wave's LDS accesses in order is a meeting of its lanes here)
     yield "cut_parts.inc", re.sub(r'__asm__ volatile\("" ::: "memory"\);', "emu::meet(emu::kPoint);",
                                   _cut("fcap_parts.hip", "constexpr int kBlock", "// " + "-" * 65 + " analysis"))
+    yield "cut_rows.inc", _cut("fcap_linalg.hip", "// " + "-" * 43 + " dependency-driven sweeps",
+                               "// The pivot recurrences")
     yield "cut_solver.inc", _cut("fcap_solvers.hip", "// the end of an iteration with", "// " + "-" * 65 + " helpers")
 
 
@@ -123,6 +125,57 @@ def test_part_sweeps_whatever_the_waves_do(emu, name, structure, width, parts):
         assert rc == [0, 0], rc
         np.testing.assert_array_equal(z, ref, err_msg=f"seed {seed}")
         assert np.all(tmp.view(mark.dtype) == mark)
+
+
+def _levels(csr, upper):
+    """Rows by (level, row) and each one's entries, as the row-wise sweeps have them packed."""
+    ptr, ja, diag = csr.ioffset - 1, csr.ja - 1, csr.diag - 1
+    n = len(diag)
+    lev = np.zeros(n, int)
+    rng = range(n - 1, -1, -1) if upper else range(n)
+    part = lambda i: slice(diag[i] + 1, ptr[i + 1]) if upper else slice(ptr[i], diag[i])  # noqa: E731
+    for i in rng:
+        lev[i] = lev[ja[part(i)]].max(initial=-1) + 1
+    return np.lexsort((np.arange(n), lev)), part
+
+
+def _row_sweeps(emu, csr, a, d, r, width, run):
+    n, small, arrays = len(r), 1e-20, []
+    for upper in (False, True):
+        rows, part = _levels(csr, upper)
+        cnt, col, val = np.zeros(n, np.int32), np.zeros((width, n), np.int32), np.zeros((width, n))
+        for p, i in enumerate(rows):
+            c = part(i).stop - part(i).start
+            cnt[p], col[:c, p], val[:c, p] = c, csr.ja[part(i)] - 1, a[part(i)]
+        arrays.append((rows.astype(np.int32), cnt, col, val, d[rows]))
+    two = lambda k: (C.c_void_p * 2)(arrays[0][k].ctypes.data, arrays[1][k].ctypes.data)  # noqa: E731
+    tmp = np.full(n, np.uint64(MARK[8])).view(np.float64)
+    w = np.zeros(n)
+    rc = emu.emu_rows(C.byref(run), width, n, two(0), two(1), two(2), two(3), two(4), _ptr(r), C.c_double(small),
+                      _ptr(tmp), _ptr(w))
+    return rc, w, tmp
+
+
+@pytest.mark.parametrize("grid,resident,reverse", [(16, 3, False), (40, 5, True), (16, 1, False), (9, 0, False),
+                                                   (8, 8, True), (7, 0, False), (2, 1, True), (1, 0, False)])
+@pytest.mark.parametrize("name,structure,width", [("box", _mesh(M.hex_box(14, 9, 8)), 3),
+                                                  ("wide", P.stencil((9, 8, 9), P.STEPS8), 8)],
+                         ids=lambda v: v if isinstance(v, str) else "")
+def test_row_sweeps_need_no_workgroup_but_the_running_ones(emu, name, structure, width, grid, resident, reverse):
+    """Workgroups that start when others have ended, fewer at once than there are block counters, the
+    first ones last: whichever run compute every row they wait for themselves (the oracle's sweeps bit
+    for bit), and the forward sweep's output is marked again."""
+    csr, a, r = _matrix(*structure, 5)
+    d = O.dic_pivots(csr, a)
+    ref = O.lu_apply(csr, a, d, r)
+    order = np.arange(grid, dtype=np.uint32)[::-1 if reverse else 1].copy()
+    for seed in range(3):
+        run = _run(grid, seed=seed, freeze=0.003 * seed, freeze_steps=2000, resident=resident, wait_ticks=10**6,
+                   order=order)
+        rc, w, tmp = _row_sweeps(emu, csr, a, d, r, width, run)
+        assert rc == 0, "a wait ran past its limit" if rc == 1 else "no end"
+        np.testing.assert_array_equal(w, ref, err_msg=f"seed {seed}")
+        assert np.all(tmp.view(np.uint64) == np.uint64(MARK[8]))
 
 
 @pytest.mark.parametrize("bicg", [0, 1])
