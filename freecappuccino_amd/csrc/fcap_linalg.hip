@@ -492,9 +492,7 @@ template <class T>
 __global__ void k_sf_mark(int n, T *__restrict__ w, const Scalars *__restrict__ sc) {
     if (sc && sc->done) return;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    using U = typename SfBits<T>::U;
-    reinterpret_cast<U *>(w)[i] = SfBits<T>::kMark;
+    if (i < n) sf_mark(w + i);
 }
 
 // Takes the smallest block below `limit` that is left, from any counter; `limit`: there is none.
@@ -621,7 +619,7 @@ __global__ __launch_bounds__(64) void k_sweep_syncfree(int n, const int *__restr
             naside += 2;
             continue;
         }
-        if (p < n) reinterpret_cast<U *>(mk)[i] = SfBits<T>::kMark;
+        if (p < n) sf_mark(mk + i);
     }
 }
 

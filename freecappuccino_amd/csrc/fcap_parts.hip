@@ -138,8 +138,7 @@ __global__ void k_part_vals(int npk, int width, bool upper, const int *__restric
 template <class T>
 __global__ void k_part_mark(int npk, T *__restrict__ w) {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    using U = typename SfBits<T>::U;
-    if (q < npk) reinterpret_cast<U *>(w)[q] = SfBits<T>::kMark;
+    if (q < npk) sf_mark(w + q);
 }
 
 // ------------------------------------------------------------------- kernel
@@ -295,11 +294,10 @@ __device__ __forceinline__ T part_result(const PartRun<T> &R, const PartLds<T, W
 // the results of a finished window that need not be early
 template <class T, bool BWD>
 __device__ __forceinline__ void part_retire(const PartRun<T> &R, int j, int row, T result) {
-    using U = typename SfBits<T>::U;
     const int q = R.template at<BWD>(j) * 64 + (int)(threadIdx.x & 63);
     // the other direction's output takes its mark for the next sweep: the forward sweep
     // marks the backward one's slots, the backward sweep those it has read
-    reinterpret_cast<U *>(R.mk)[q] = SfBits<T>::kMark;
+    sf_mark(R.mk + q);
     if (BWD) R.z[row] = result;
 }
 

@@ -33,6 +33,13 @@ __device__ inline typename SfBits<T>::U sf_load_bits(const T *p) {
                              __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// A plain store of the mark, of the array's own type: a sweep marks what it has read through
+// that type, and a store of the integer type might be moved before the read.
+template <class T>
+__device__ inline void sf_mark(T *p) {
+    *p = __builtin_bit_cast(T, SfBits<T>::kMark);
+}
+
 template <class T>
 __device__ inline void sf_store(T *p, T v) {
     using U = typename SfBits<T>::U;
