@@ -420,12 +420,13 @@ __device__ __forceinline__ void part_inputs(const PartRun<T> &R, PartLds<T, W> &
             in.pb[k] = SfBits<T>::kMark;
         }
         if (part_missing<T, W>(in)) {
-            const unsigned long long t0 = wall_clock64();
+            unsigned long long t0 = wall_clock64();
             int polls = 0;
             do {
                 bool late = false;
                 if (j > 0 && lds_get(&L.flag[0]) == 0) {
                     __builtin_amdgcn_s_sleep(1);
+                    t0 = wall_clock64();   // the first poller's wait, not this one's
                 } else {
                     part_poll<T, W>(in, R.out);
                     if ((++polls & 7) == 0)

@@ -115,6 +115,24 @@ int emu_rows(const Run *r, int width, int n, const int *const rows[2], const int
     return rows_sweeps<8>(*r, n, rows, cnt, col, val, piv, rhs, small, tmp, w);
 }
 
+// The forward part-wise sweep (W = 3, FP64) of one part, with values put into its output from
+// outside: value k at slot at[k] after step when[k].
+int emu_parts_fed(const Run *r, int npk, const int *codes, const unsigned char *step, const int *win,
+                  const double *vals, const double *in, double *out, double *mk, int nfed, const int *at,
+                  const double *value, const long long *when) {
+    SyncFree sf = state(*r);
+    const parts::PartView P{npk, codes, step};
+    emu::Policy p = policy(*r);
+    p.each_step = [&](long long t) {
+        for (int k = 0; k < nfed; ++k)
+            if (t == when[k]) out[at[k]] = value[k];
+    };
+    const bool ended = emu::launch(1, parts::PartShape<3>::kBlock, p, [&]() {
+        parts::k_sweep_parts<double, 3, false>(1, P, win, vals, in, 0.0, out, mk, nullptr, &sf, nullptr);
+    });
+    return !ended ? 2 : sf.abort ? 1 : 0;
+}
+
 int emu_ring() { return parts::kRing; }
 
 int emu_parts(const Run *r, int f32, int width, int bwd, int nparts, int npk, const int *codes,

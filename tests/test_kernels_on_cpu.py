@@ -127,6 +127,34 @@ def test_part_sweeps_whatever_the_waves_do(emu, name, structure, width, parts):
         assert np.all(tmp.view(mark.dtype) == mark)
 
 
+@pytest.mark.parametrize("late", [0.7, 0.9])
+def test_the_limit_is_that_of_one_wait(emu, late):
+    """A part whose first window's inputs come late, and its second's as late after that: each wait is
+    within the limit, so the sweep ends well -- the second's is not charged with the time in which the
+    part had not begun.  One wait past the limit ends the sweep with an error."""
+    limit, windows = 20000, 6
+    n = 64 * windows
+    rows = np.arange(n)
+    codes = np.full((4, n + 128), emu.emu_ring(), np.int32)
+    codes[3, :n] = rows                                   # every row reads one value of another part,
+    outside = n + np.arange(n) % 64 + 64 * (rows >= 64)   # first window's and the others' of their own
+    codes[0, :n] = (outside | 0x80000000).astype(np.uint32).view(np.int32)
+    vals = np.ones((4, n + 128))
+    step, win = np.zeros(n + 128, np.uint8), np.array([0, windows], np.int32)
+    rng = np.random.default_rng(1)
+    rhs, fed = rng.standard_normal(n + 128), rng.standard_normal(128)
+    for second, rc in ((late, 0), (1.2, 1)):
+        out = np.full(n + 128, np.uint64(MARK[8])).view(np.float64)
+        when = np.repeat([int(late * limit), int((late + second) * limit)], 64).astype(np.int64)
+        at = (n + np.arange(128)).astype(np.int32)
+        run = _run(1, wait_ticks=limit)
+        assert emu.emu_parts_fed(C.byref(run), n + 128, _ptr(P.packed(codes)), _ptr(step), _ptr(win),
+                                 _ptr(P.packed(vals)), _ptr(rhs), _ptr(out), _ptr(np.zeros(n + 128)), 128, _ptr(at),
+                                 _ptr(fed), _ptr(when)) == rc
+        if rc == 0:
+            np.testing.assert_array_equal(out[:n], rhs[:n] - fed[outside - n])
+
+
 def _levels(csr, upper):
     """Rows by (level, row) and each one's entries, as the row-wise sweeps have them packed."""
     ptr, ja, diag = csr.ioffset - 1, csr.ja - 1, csr.diag - 1
