@@ -513,10 +513,10 @@ __device__ inline unsigned sf_take_before(unsigned (*tickets)[32], unsigned limi
     }
 }
 
-// The other sweep's output takes its marks here, behind the block's values (a block set
-// aside reads its operands again): the forward sweep marks w, whose values are spent, the
-// backward one its right-hand side (a pass of its own for each took 4.4 us on 83 K rows,
-// beside sweeps of 26 us); mark_sweep_input does it before the first sweep.
+// The other sweep's output takes its marks here: the forward sweep marks w, whose values
+// are spent, the backward one its right-hand side once read (a pass of its own for each
+// took 4.4 us on 83 K rows, beside sweeps of 26 us) and puts it back for a block set aside;
+// mark_sweep_input does it before the first sweep.
 // BWD == false: out[i] = (rhs[i] - sum a w) d over the strict lower triangle;
 // BWD == true:  out[i] = (fwd[i] / (d + small) - sum a w) d over the strict upper one.
 template <class T, int W, bool BWD>
@@ -556,7 +556,7 @@ __global__ __launch_bounds__(64) void k_sweep_syncfree(int n, const int *__restr
         int i = 0, c = 0;
         int cj[W];
         T ak[W], wk[W];
-        T acc = T(0), di = T(0);
+        T rhs = T(0), acc = T(0), di = T(0);
         unsigned ready = 0;
         if (!done) {
             i = rows[p];
@@ -568,7 +568,9 @@ __global__ __launch_bounds__(64) void k_sweep_syncfree(int n, const int *__restr
                 ak[k] = av[(size_t)k * n + p];
                 wk[k] = T(0);
             }
-            acc = BWD ? in[i] / (di + small) : in[i];
+            rhs = in[i];
+            acc = BWD ? rhs / (di + small) : rhs;
+            sf_mark(mk + i);   // behind the load of in[i] (mk may be in)
         }
         int spins = 0;
         const unsigned long long t0 = wall_clock64();
@@ -614,12 +616,11 @@ __global__ __launch_bounds__(64) void k_sweep_syncfree(int n, const int *__restr
             __builtin_amdgcn_s_sleep(1);
         }
         if (before < b) {
+            if (BWD && p < n) mk[i] = rhs;
             if (lane == naside) aside = b;
             if (lane == naside + 1) aside = before;
             naside += 2;
-            continue;
         }
-        if (p < n) sf_mark(mk + i);
     }
 }
 
