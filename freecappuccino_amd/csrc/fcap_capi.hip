@@ -1302,9 +1302,8 @@ static fc_status sys_calcp_assemble(bool piso, fc_system *sys, const double *den
         F.dwdx = dgf[2];
         F.dpdx = dgf[3];
         ctx->timer.start(ctx->stream);
-        // a = 0 (calcp:34): needed only where the faces and diagonals leave slots unwritten
-        if ((long long)sys->st.nnz != (long long)n + 2ll * nif)
-            FC_HIP_CHECK(hipMemsetAsync(sys->a.get(), 0, sizeof(double) * sys->st.nnz, ctx->stream));
+        // (a = 0, calcp:34, has nothing to do here: a system has two slots a face and a diagonal a
+        // cell, duplicate faces being refused, and all of them are written)
         calcp_dev(ctx, sys->st, nif, sys->mesh.owner.as<int>(), sys->mesh.neighbour.as<int>(), sys->ij.as<int>(),
                   sys->ji.as<int>(), sys->kface.as<int>(), sys->needs_order ? sys->kord.as<int>() : nullptr,
                   g.xf.as<double>(), g.yf.as<double>(), g.zf.as<double>(), g.arx.as<double>(), g.ary.as<double>(),

@@ -191,15 +191,17 @@ struct fc_context {
 namespace fcap {
 
 // persistent workgroups of the part-wise sweeps: the context's setting, else one per CU
-// (per sweep of the 192^3 box: 128 workgroups 373 us, 256 315, 384 364, 512 417: more of
-// them wait, and poll, than the chain of parts can use)
+// (pencils, per sweep of the 192^3 box: 128 workgroups 373 us, 256 315, 384 364, 512 417:
+// more of them wait, and poll, than the chain of parts can use; runs of consecutive rows
+// do not mind: 128, 256 and 384 within 1 % on a 40^3 and a 56^3 box in reverse
+// Cuthill-McKee order, tets in that order and a 96 x 96 x 64 box in Morton order)
 inline int part_wave_count(const fc_context *ctx) { return ctx->part_waves > 0 ? ctx->part_waves : ctx->num_cus; }
 
-// persistent waves of the row-wise dependency-driven sweeps and pivots: twice the
-// 64-row blocks of an average level, at least one wave per CU and at most sixteen.  A deep chain (192^3 box in natural order: 574 levels of 12K rows)
-// then runs with one wave per CU -- more waves only add polling -- and a shallow one
-// (96^3 permuted Kuhn tets: 16 levels of 330K rows) with enough waves to keep its
-// gathers in flight.
+// persistent waves of the row-wise dependency-driven sweeps and pivots: twice the 64-row
+// blocks of an average level, at least one wave per CU and at most sixteen.  A deep chain
+// (192^3 box in natural order: 574 levels of 12K rows) then runs with few waves a CU --
+// more only add polling -- and a shallow one (96^3 permuted Kuhn tets: 16 levels of 330K
+// rows) with enough to keep its gathers in flight.
 inline int syncfree_wave_count(const fc_context *ctx, const Structure &st) {
     if (ctx->part_waves > 0) return ctx->part_waves;
     const long long nlev = std::max(1, std::max(st.nlev_f, st.nlev_b));

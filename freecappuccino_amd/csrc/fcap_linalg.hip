@@ -748,6 +748,17 @@ bool syncfree_sweeps(const Structure &st) {
     return packed_sweeps(st) && ok(st.ell_f) && ok(st.ell_b);
 }
 
+// Why half: us a sweep part-wise and row-wise, by the share of entries read from the part's
+// own LDS.  Box in reverse Cuthill-McKee order 24^3 (0.93) 48 and 82, 32^3 (0.87) 96 and
+// 112, 40^3 (0.40) 168 and 142, 48^3 (0.22) 255 and 172, 56^3 (0.14) 350 and 202; Kuhn tets
+// in that order 16^3 (0.92) 66 and 126, 28^3 (0.73) 133 and 229, 40^3 (0.47) 255 and 327, in
+// natural order 16^3 (0.94) 64 and 77, 28^3 (0.70) 170 and 143, 40^3 (0.63) 327 and 199;
+// boxes shuffled within runs of 300 to 500 cells (0.81, 0.57; five entries a triangle) 147
+// and 485, 313 and 513; Morton order (0.96) 45 to 136 and 131 to 406.  No share parts them
+// all: the part-wise time is that of the longest chain through parts, not of the share.
+// A ring of 4,096 slots would count 0.79, 0.69 and 0.58 of the Cuthill-McKee boxes' entries
+// as inside, and take them to the slower schedule: the times are the same to 1 % with rings
+// of 1,024, 2,048 and 4,096 (129 and 147 us on one of the shuffled boxes).
 bool part_sweeps(const Structure &st) {
     return syncfree_sweeps(st) && st.parts && st.int_frac_f >= 0.5 && st.int_frac_b >= 0.5;
 }
