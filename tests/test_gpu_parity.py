@@ -835,3 +835,30 @@ def test_row_sweeps_bitwise_over_wave_counts(ctx, mesh, waves):
         s.close()
     for method, (a, b) in out.items():
         np.testing.assert_array_equal(a, b, err_msg=str(method))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("method", ["ICCG", "DPCG", "BICGSTAB", "ICCG_MIXED", "BICGSTAB_MIXED", "FCG_JACOBI"])
+def test_solves_that_end_before_and_after_the_graph(ctx, method):
+    """Solves of 1 to 12 iterations -- launched one by one, ending as the graph of iterations is set
+    up, and replayed from it -- stop at their limit and give the iterates of launches alone."""
+    m = M.hex_box(13, 11, 9, perturb=0.1, seed=2)
+    su = np.random.default_rng(6).uniform(-1, 1, m.n_cells)
+    s = fcap.System(m, ctx)
+    try:
+        for mode in (fcap.SWEEP_PARTS, fcap.SWEEP_DEPENDENT, fcap.SWEEP_LEVELS):
+            ctx.set_sweep_mode(mode)
+            for nsw in range(1, 13):
+                out = []
+                for graphs in (True, False):
+                    ctx.set_graphs(graphs)
+                    s.assemble_laplacian(np.full(m.n_cells, -1.0), None, su)
+                    s.set_solution(np.zeros(m.n_cells))
+                    _, info = s.solve(getattr(fcap, "METHOD_" + method), fcap.STOP_L2, 1e-15, nsw)
+                    assert info["iters"] == nsw
+                    out.append(s.solution())
+                np.testing.assert_array_equal(out[0], out[1], err_msg=f"mode {mode}, nsw {nsw}")
+    finally:
+        ctx.set_graphs(True)
+        ctx.set_sweep_mode(fcap.SWEEP_DEFAULT)
+        s.close()
