@@ -21,6 +21,8 @@ namespace {
 
 constexpr unsigned kPad = 0xffffu;      // offset of a padding entry
 constexpr int kMinWidth = 4, kMaxWidth = 8;
+// Rows from which a matrix whose slices are mostly wide (below) keeps the CSR rows
+constexpr int kWideRows = 200000;
 
 inline int grid_for(long long n, int block) { return (int)std::max<long long>(1, (n + block - 1) / block); }
 __host__ __device__ inline int slices_of(int n) { return (n + kWave - 1) / kWave; }
@@ -35,9 +37,9 @@ __global__ void k_row_width(int n, const int *__restrict__ ptr, int *__restrict_
 }
 
 // Bases and offsets of a slice, one wave each; base -1: some entry's columns span more
-// than 16 bits, the slice then reads its columns from the CSR array.
+// than 16 bits, the slice then reads its columns from the CSR array (a wide slice; counted).
 __global__ void k_slice_columns(int n, int width, const int *__restrict__ ptr, const int *__restrict__ ja,
-                                int *__restrict__ base, unsigned *__restrict__ off) {
+                                int *__restrict__ base, unsigned *__restrict__ off, int *__restrict__ nwide) {
     const int slice = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, lane = threadIdx.x & 63;
     if (slice * kWave >= n) return;
     const int row = slice * kWave + lane;
@@ -59,8 +61,10 @@ __global__ void k_slice_columns(int n, int width, const int *__restrict__ ptr, c
             off + ((size_t)slice * ((width + 1) / 2) + k / 2) * kWave + lane);
         o16[k & 1] = (unsigned short)d;
     }
-    if (wide && lane == 0)
+    if (wide && lane == 0) {
         for (int k = 0; k < width; ++k) base[slice * width + k] = -1;
+        atomicAdd(nwide, 1);
+    }
 }
 
 template <class T>
@@ -167,7 +171,13 @@ void sliced(hipStream_t s, int n, const SliceView &S, const T *v, const T *x, co
 }  // namespace
 
 // Slices up to eight entries a row (what the kernels hold in registers) where padding is at
-// most a quarter of them: 16-bit columns save as much.
+// most a quarter of them: 16-bit columns save as much.  Not where most slices are wide (a
+// scattered numbering) and the matrix is large: their columns come a row at a time instead of
+// a wave at a time through LDS, beside offsets read for nothing.  In ms, CSR and slices, 200
+// Jacobi-PCG and 60 flexible CG iterations, randomly numbered boxes and tets: 97,336 rows 3.46
+// and 3.48, 4.35 and 4.23; 131,712 (tets) 3.72 and 3.56, 4.43 and 4.35; 195,112 4.75 and 4.78,
+// 5.69 and 5.76; 262,144 5.48 and 5.73, 6.54 and 6.76; 884,736 16.4 and 17.6, 13.6 and 15.4;
+// 2,097,152 46.8 and 48.9, 41.3 and 45.5.
 SliceView slices_for(fc_context *ctx, Structure &st) {
     if (!st.sl_ready) {
         hipStream_t s = ctx->stream;
@@ -181,12 +191,24 @@ SliceView slices_for(fc_context *ctx, Structure &st) {
         st.sl_w = w <= kMaxWidth && 4ll * st.nnz >= 3ll * st.n * w ? w : 0;
         if (st.sl_w) {
             const size_t ns = (size_t)slices_of(st.n);
+            fill_int(ctx, wd.as<int>(), 1, 0);   // now the wide slices
             st.sl_base.alloc(sizeof(int) * ns * w);
             st.sl_off.alloc(sizeof(unsigned) * ns * ((w + 1) / 2) * kWave);
             FC_HIP_CHECK(hipMemsetAsync(st.sl_off.get(), 0xff, sizeof(unsigned) * ns * ((w + 1) / 2) * kWave, s));
             k_slice_columns<<<grid_for((long long)ns * kWave, 256), 256, 0, s>>>(
-                st.n, w, st.ioffset.as<int>(), st.ja.as<int>(), st.sl_base.as<int>(), st.sl_off.as<unsigned>());
+                st.n, w, st.ioffset.as<int>(), st.ja.as<int>(), st.sl_base.as<int>(), st.sl_off.as<unsigned>(),
+                wd.as<int>());
             FC_HIP_CHECK(hipGetLastError());
+            if (st.n >= kWideRows) {
+                int wide = 0;
+                FC_HIP_CHECK(hipMemcpyAsync(&wide, wd.get(), sizeof(int), hipMemcpyDeviceToHost, s));
+                FC_HIP_CHECK(hipStreamSynchronize(s));
+                if (2ll * wide > (long long)ns) {
+                    st.sl_w = 0;
+                    st.sl_base.release();
+                    st.sl_off.release();
+                }
+            }
         }
         st.sl_ready = true;
     }

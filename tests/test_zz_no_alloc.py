@@ -140,6 +140,34 @@ def test_products_in_slices_give_the_csr_bits(n, matchings, near):
         ctx.close()
 
 
+@pytest.mark.parametrize("n,matchings,near", [(199999, 3, 0), (200000, 3, 0), (200001, 4, 300), (524288, 2, 40),
+                                              (524289, 2, 40)])
+def test_large_products_give_the_csr_bits(n, matchings, near):
+    """The same where the route of a product changes: a scattered numbering keeps the CSR rows from
+    200,000 rows on (a local one its slices), and the partials of more than 524,288 rows are added by
+    a launch of their own, with four rows a thread in the vector kernels from there."""
+    import scipy.sparse as sp
+    ctx = fcap.Context(0)
+    dev = _Dev()
+    try:
+        csr, a = _random_csr(n, matchings, near, n + matchings)
+        su = np.random.default_rng(1).standard_normal(n)
+        fi0 = np.zeros(n)
+        ref = fcap.dpcg(csr, a, su, fi0, sor=1e-12, nsw=500, ctx=ctx)
+        rc, fi, res, info = _noalloc(ctx, dev, csr, a, su, fi0, 1e-12, 500)
+        assert rc == ref.status == fcap.FC_OK, (rc, ref.status)
+        assert info["iters"] == ref.info["iters"] > 0
+        np.testing.assert_array_equal(fi, ref.fi)
+        np.testing.assert_array_equal(res, ref.res)
+        A = sp.csr_matrix((a, csr.ja - 1, csr.ioffset - 1), shape=(n, n))
+        r = su - A @ fi
+        # |r|_1 < 1e-12 |su|_1 at the end; rounding of A x adds at most (entries of a row) eps |A| |x|
+        assert np.abs(r).sum() < 1e-12 * np.abs(su).sum() + 12 * 2.3e-16 * (abs(A) @ np.abs(fi)).sum()
+    finally:
+        dev.close()
+        ctx.close()
+
+
 def test_noalloc_dpcg_refuses_oversize_and_host_arrays():
     ctx = fcap.Context(0)
     dev = _Dev()
