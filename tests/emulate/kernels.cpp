@@ -11,6 +11,9 @@ namespace parts {
 namespace rows {
 #include "cut_rows.inc"
 }
+namespace slices {
+#include "cut_slices.inc"
+}
 namespace solver {
 #include "cut_solver.inc"
 }
@@ -42,6 +45,45 @@ SyncFree state(const Run &r) {
     sf.wait_us = (int)r.wait_ticks;
     sf.rate_khz = 1000;
     return sf;
+}
+
+template <class T, int W>
+void sliced_w(int mode, int grid, int n, const slices::SliceView &S, const T *v, const T *x, const T *b, const T *d, T *y,
+              double *pa, double *pb) {
+    const Run r{grid, 1, 2, 1, 0.0, 0.0, 0, 1000000000, nullptr};
+    emu::launch((unsigned)grid, kSpmvRows, policy(r), [&]() {
+        if (mode == 2) slices::k_sliced<T, W, 2>(n, S, v, x, b, d, y, pa, pb, nullptr, 0.f);
+        else if (mode == 3) slices::k_sliced<T, W, 3>(n, S, v, x, b, d, y, pa, pb, nullptr, 0.f);
+        else slices::k_sliced<T, W, 4>(n, S, v, x, b, d, y, pa, pb, nullptr, 0.7f);
+    });
+}
+// y (modes 2, 3: A x; 4: a damped Jacobi step) by the sliced kernels; wide slices found
+template <class T>
+int sliced(int mode, int n, int w, const int *ptr, const int *ja, const double *a, const T *x, const T *b, const T *d,
+           T *y, double *pa, double *pb) {
+    const int ns = (n + 63) / 64, grid = (n + kSpmvRows - 1) / kSpmvRows;
+    std::vector<int> base((size_t)ns * w);
+    std::vector<unsigned> off((size_t)ns * ((w + 1) / 2) * 64, 0xffffffffu);
+    std::vector<T> v((size_t)ns * 64 * w);
+    int wide = 0;
+    const Run r{grid, 1, 2, 1, 0.0, 0.0, 0, 1000000000, nullptr};
+    emu::launch((unsigned)grid, 256, policy(r), [&]() {
+        slices::k_slice_columns(n, w, ptr, ja, base.data(), off.data(), &wide);
+    });
+    emu::launch((unsigned)grid, 256, policy(r), [&]() { slices::k_slice_values<T>(n, w, ptr, a, v.data()); });
+    slices::SliceView S;
+    S.w = w;
+    S.base = base.data();
+    S.off = off.data();
+    S.ptr = ptr;
+    S.ja = ja;
+    switch (w) {
+    case 4: sliced_w<T, 4>(mode, grid, n, S, v.data(), x, b, d, y, pa, pb); break;
+    case 5: sliced_w<T, 5>(mode, grid, n, S, v.data(), x, b, d, y, pa, pb); break;
+    case 7: sliced_w<T, 7>(mode, grid, n, S, v.data(), x, b, d, y, pa, pb); break;
+    default: sliced_w<T, 8>(mode, grid, n, S, v.data(), x, b, d, y, pa, pb); break;
+    }
+    return wide;
 }
 
 template <int W>
@@ -131,6 +173,11 @@ int emu_parts_fed(const Run *r, int npk, const int *codes, const unsigned char *
         parts::k_sweep_parts<double, 3, false>(1, P, win, vals, in, 0.0, out, mk, nullptr, &sf, nullptr);
     });
     return !ended ? 2 : sf.abort ? 1 : 0;
+}
+
+int emu_sliced32(int mode, int n, int w, const int *ptr, const int *ja, const double *a, const float *x, const float *b,
+                 const float *d, float *y, double *pa, double *pb) {
+    return sliced<float>(mode, n, w, ptr, ja, a, x, b, d, y, pa, pb);
 }
 
 int emu_ring() { return parts::kRing; }

@@ -56,6 +56,7 @@ enum Op : int { kNone, kPoint, kStore, kValue, kBarrier };
 struct Wave;
 struct Lane {
     void *sp = nullptr;
+    char *stack = nullptr;
     Wave *wave = nullptr;
     unsigned tid = 0;
     int lane = 0, op = kNone;
@@ -186,9 +187,9 @@ inline bool launch(unsigned grid, unsigned threads, Policy p, const std::functio
                     stacks.push_back((char *)m);
                     spare.push_back((char *)m);
                 }
-                char *s = spare.back();
+                ln.stack = spare.back();
                 spare.pop_back();
-                void **top = (void **)(s + kStack - 16);
+                void **top = (void **)(ln.stack + kStack - 16);
                 *--top = nullptr;                  // return address of lane_main: none
                 *--top = (void *)&lane_main;
                 for (int r = 0; r < 6; ++r) *--top = nullptr;
@@ -243,13 +244,8 @@ inline bool launch(unsigned grid, unsigned threads, Policy p, const std::functio
             in_lds = nullptr;
             for (auto it = live.begin(); it != live.end(); ++it)
                 if (it->get() == &b) {
-                    for (Wave &x : b.waves)   // their stacks: sp lies within
-                        for (Lane &l : x.lanes)
-                            for (char *s : stacks)
-                                if ((char *)l.sp >= s && (char *)l.sp < s + kStack) {
-                                    spare.push_back(s);
-                                    break;
-                                }
+                    for (Wave &x : b.waves)
+                        for (Lane &l : x.lanes) spare.push_back(l.stack);
                     live.erase(it);
                     break;
                 }
@@ -304,6 +300,7 @@ inline int4 make_int4(int x, int y, int z, int w) { return {x, y, z, w}; }
 #define __hip_atomic_compare_exchange_strong(p, e, v, order, order2, scope) emu::cas(p, e, v)
 #define atomicAdd(p, v) emu::add(p, v)
 #define atomicOr(p, v) (*(p) |= (v))
+#define atomicMax(p, v) (*(p) = std::max(*(p), (v)))
 #define __builtin_amdgcn_readfirstlane(v) emu::first(v)
 #define __builtin_amdgcn_readlane(v, l) emu::bring(v).at(l)
 #define __builtin_amdgcn_s_sleep(n) emu::meet(emu::kPoint)

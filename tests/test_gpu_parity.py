@@ -720,9 +720,10 @@ def test_bpres_oc_cuts_match_oracle(ctx, golden_loader):
 
 @pytest.mark.parametrize("mesh", ["hex32", "hex24_graded", "tet12"])
 def test_part_sweeps_bitwise_on_multi_part_meshes(ctx, mesh):
-    """Meshes of several parts of 4,096 rows (hex 32^3: 8 parts; graded 24^3: 4; Kuhn tets 12^3:
-    3): the part-wise sweeps (inputs inside a part through LDS, across parts through global
-    memory) give the DIC and DILU sweeps of the oracle bit for bit, as the other schedules do."""
+    """Meshes of several parts (hex 32^3: 16 pencils; graded 24^3: 9; Kuhn tets 12^3: 3 runs of
+    4,096 rows): the part-wise sweeps (inputs inside a part through LDS, across parts through
+    global memory) give the DIC and DILU sweeps of the oracle bit for bit, as the other schedules
+    do."""
     m = {"hex32": lambda: M.hex_box(32, perturb=0.2, seed=3),
          "hex24_graded": lambda: M.hex_box(24, perturb=0.2, seed=4, grade_axis=0, grade_ratio=1.2,
                                            grade_max_aspect=50.0),
@@ -770,7 +771,8 @@ def _part_meshes():
     c = np.arange(m.n_cells)
     i = c % 24
     yield "two_blocks", _renumbered(m, np.concatenate([c[i < 9], c[i >= 9]]))
-    # numberings without such runs: consecutive parts (z fastest in tiles), scattered rows
+    # numberings without such runs: consecutive parts (z fastest in tiles); scattered rows, which
+    # read too little of their own part and take the row-wise sweeps
     x, y, z = i, (c // 24) % 20, c // 480
     yield "tiles", _renumbered(m, np.lexsort((x % 4, z % 4, y % 4, x // 4, y // 4, z // 4)))
     yield "scattered", _renumbered(m, np.random.default_rng(4).permutation(m.n_cells))
@@ -779,8 +781,8 @@ def _part_meshes():
 @pytest.mark.gpu
 @pytest.mark.parametrize("name,m", list(_part_meshes()), ids=lambda v: v if isinstance(v, str) else "")
 def test_part_sweeps_bitwise_over_numberings(ctx, name, m):
-    """The part-wise sweeps over every form of parts -- pencils with ragged line and sheet blocks,
-    several stacks, consecutive runs -- give the oracle's DIC and DILU sweeps bit for bit, and the
+    """The sweeps the default chooses over every form of parts -- pencils with ragged line and sheet
+    blocks, several stacks, consecutive runs -- and over scattered rows give the oracle's DIC and DILU sweeps bit for bit, and the
     FP32 sweeps inside the mixed solver the same iterates as one launch per level."""
     geo = O.mesh_geometry(m)
     csr = O.csr_build(m.n_cells, m.owner[:m.n_inner] + 1, m.neighbour + 1)
@@ -861,4 +863,124 @@ def test_solves_that_end_before_and_after_the_graph(ctx, method):
     finally:
         ctx.set_graphs(True)
         ctx.set_sweep_mode(fcap.SWEEP_DEFAULT)
+        s.close()
+
+
+def _structure(n, lo, hi):
+    """(ioffset, ja, diag), 1-based, of n rows coupled in the pairs (lo, hi)."""
+    i = np.arange(n)
+    key = np.unique(np.concatenate([lo, hi, i]) * n + np.concatenate([hi, lo, i]))
+    row, col = key // n, key % n
+    one = lambda x: np.ascontiguousarray(x + 1, np.int32)  # noqa: E731
+    return one(np.concatenate([[0], np.cumsum(np.bincount(row))])), one(col), one(np.flatnonzero(row == col))
+
+
+def _hubs(groups, mirrored):
+    """Rows in groups of seven, the last of a group coupled to the six before it, and every row to the
+    one 200 on: seven entries in a strict lower triangle's widest row and two in the upper's, or
+    mirrored the other way round."""
+    n = 7 * groups
+    i = np.arange(n)
+    lo, hi = np.concatenate([np.stack([i[:-200], i[200:]])] + [np.stack([i[k::7], i[6::7]]) for k in range(6)], axis=1)
+    return _structure(n, n - 1 - lo, n - 1 - hi) if mirrored else _structure(n, lo, hi)
+
+
+def _shuffled(structure, run):
+    """The structure with its rows in random order within runs of consecutive ones."""
+    ioffset, ja, diag = structure
+    n = len(diag)
+    new = np.empty(n, np.int64)
+    new[np.lexsort((np.random.default_rng(n).random(n), np.arange(n) // run))] = np.arange(n)
+    return _structure(n, new[np.repeat(np.arange(n), np.diff(ioffset))], new[ja - 1])
+
+
+def _wide_structures():
+    import part_model as P
+    yield "four", P.stencil((24, 20, 40), P.STEPS6[:4]), 4, 4
+    yield "six", P.stencil((24, 20, 40), P.STEPS6), 8, 8
+    yield "eight", P.stencil((20, 17, 41), P.STEPS8), 8, 8
+    yield "four_runs", _shuffled(P.stencil((90, 150, 1), P.STEPS6[:2]), 200), 4, 4
+    yield "eight_runs", _shuffled(P.stencil((20, 18, 40), P.STEPS6[:4]), 150), 8, 8
+    yield "hubs", _hubs(2000, False), 8, 3
+    yield "mirrored_hubs", _hubs(2000, True), 3, 8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,structure,wf,wb", list(_wide_structures()), ids=lambda v: v if isinstance(v, str) else "")
+def test_part_sweeps_bitwise_over_row_widths(ctx, name, structure, wf, wb):
+    """Part-wise sweeps whose rows have four to eight entries in a triangle, the same width in both or
+    not, pencils and runs, in several parts each longer than the ring in LDS: the oracle's DIC and DILU sweeps bit
+    for bit.  The schedule chosen is the part-wise one by the rule restated here."""
+    import part_model as P
+    ioffset, ja, diag = structure
+    oc = O.CSR(ioffset, ja, diag, np.zeros(0, np.int32), np.zeros(0, np.int32))
+    zero = ioffset - 1, ja - 1, diag - 1
+    low, up = (zero[2] - zero[0][:-1]).max(), (zero[0][1:] - 1 - zero[2]).max()
+    assert [3 if w <= 3 else 4 if w <= 4 else 8 for w in (low, up)] == [wf, wb] and max(low, up) <= 8
+    s = P.Schedule(*zero, *(P.pencil_parts(*zero) or P.run_parts(*zero)))
+    for upper, width in ((False, wf), (True, wb)):
+        s.codes(upper, width, 1024)
+        assert s.inside >= 0.5, (name, s.inside)
+    assert s.nparts >= 3 and np.diff(s.win).max() > 16
+    n = len(diag)
+    rng = np.random.default_rng(7)
+    row = np.repeat(np.arange(n), np.diff(ioffset))
+    key = np.minimum(row, ja - 1) * n + np.maximum(row, ja - 1)
+    a = -rng.uniform(0.5, 1.0, ja.size)[np.unique(key, return_inverse=True)[1]]
+    a[zero[2]] = 20.0
+    r = rng.standard_normal(n)
+    csr = fcap.CSR(ioffset, ja, diag, oc.ij_slot, oc.ji_slot)
+    for mat, pivots in ((a, O.dic_pivots), (a * rng.uniform(0.8, 1.2, a.size), O.dilu_pivots)):
+        d = pivots(oc, mat)
+        np.testing.assert_array_equal(fcap.lu_apply(csr, mat, d, r, ctx), O.lu_apply(oc, mat, d, r), err_msg=name)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["box", "tets"])
+def test_part_sweeps_of_wide_rows_in_the_solvers(ctx, name):
+    """Meshes shuffled within runs of 300 cells (up to six neighbours before a cell; up to four in
+    the tets): the solvers' FP64 and FP32 part-wise sweeps give the iterates of one launch per level."""
+    m = M.hex_box(24, 20, 40) if name == "box" else M.tet_box(14)
+    c = np.arange(m.n_cells)
+    m = _renumbered(m, np.lexsort((np.random.default_rng(3).random(m.n_cells), c // 300)))
+    su = np.random.default_rng(8).uniform(-1, 1, m.n_cells)
+    s = fcap.System(m, ctx)
+    out = {}
+    try:
+        for mode in (fcap.SWEEP_PARTS, fcap.SWEEP_LEVELS):
+            ctx.set_sweep_mode(mode)
+            for method in (fcap.METHOD_ICCG, fcap.METHOD_ICCG_MIXED, fcap.METHOD_BICGSTAB_MIXED):
+                s.assemble_laplacian(np.full(m.n_cells, -1.0), None, su)
+                s.set_solution(np.zeros(m.n_cells))
+                s.solve(method, fcap.STOP_L2, 1e-8, 500)
+                out.setdefault(method, []).append(s.solution())
+    finally:
+        ctx.set_sweep_mode(fcap.SWEEP_DEFAULT)
+        s.close()
+    for method, (x, y) in out.items():
+        np.testing.assert_array_equal(x, y, err_msg=str(method))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims", [(128, 64, 64), (129, 64, 64)])
+@pytest.mark.parametrize("method", ["BICGSTAB", "BICGSTAB_MIXED", "ICCG_MIXED"])
+def test_solves_around_the_limit_of_direct_sums(ctx, dims, method):
+    """524,288 and 528,384 rows: up to the first the vector kernels add the product's partials (one or
+    two sums) themselves, beyond it a launch of its own does; the residual reached is the one asked for."""
+    import scipy.sparse as sp
+    m = M.hex_box(*dims)
+    n = m.n_cells
+    su = np.random.default_rng(9).uniform(-1, 1, n)
+    su -= su.mean()
+    s = fcap.System(m, ctx)
+    try:
+        s.assemble_laplacian(np.full(n, -1.0), None, su)
+        rc, info = s.solve(getattr(fcap, "METHOD_" + method), fcap.STOP_L2, 1e-6, 2000)
+        assert rc == fcap.FC_OK, (rc, info)
+        A = sp.csr_matrix((s.get("a"), s.get("ja") - 1, s.get("ioffset") - 1), shape=(n, n))
+        b = s.get("su")
+        # the recurrence's residual and the true one part by rounding: at most iterations x eps x |A||x|
+        rel = np.linalg.norm(b - A @ s.solution()) / np.linalg.norm(b)
+        assert rel < 1e-6 * 1.01, (rel, info)
+    finally:
         s.close()

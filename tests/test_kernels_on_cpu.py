@@ -36,6 +36,8 @@ def _cuts():
                                   _cut("fcap_parts.hip", "constexpr int kBlock", "// " + "-" * 65 + " analysis"))
     yield "cut_rows.inc", _cut("fcap_linalg.hip", "// " + "-" * 43 + " dependency-driven sweeps",
                                "// The pivot recurrences")
+    yield "cut_slices.inc", (_cut("fcap_linalg.h", "struct SliceView", "SliceView slices_for") +
+                             _cut("fcap_slices.hip", "constexpr unsigned kPad", "template <class T, int MODE>\nvoid sliced"))
     yield "cut_solver.inc", _cut("fcap_solvers.hip", "// the end of an iteration with", "// " + "-" * 65 + " helpers")
 
 
@@ -226,3 +228,38 @@ def test_every_block_ends_the_solve_alike(emu, bicg, converged):
             want = p0 if converged else p.copy()
             assert converged or np.all(p != p0)
         np.testing.assert_array_equal(p, want, err_msg=f"seed {seed}")
+
+
+@pytest.mark.parametrize("n,spread,longest", [(1, 1, 1), (64, 5, 4), (65, 40, 5), (255, 9, 7), (700, 300, 8),
+                                              (70001, 70000, 5), (3000, 200, 7)])
+def test_single_precision_products_in_slices(emu, n, spread, longest):
+    """FP32 products, their partials and damped-Jacobi steps over slices: the row's entries one by one
+    in order, in the precision of the CSR kernels, bit for bit.  Columns within 16 bits of each other
+    and, with 70,001 rows, beyond (wide slices); ragged rows and last slices."""
+    rng = np.random.default_rng(n)
+    cnt = rng.integers(1, longest + 1, n)
+    ptr = np.concatenate([[0], np.cumsum(cnt)]).astype(np.int32)
+    row = np.repeat(np.arange(n), cnt)
+    ja = np.clip(row + rng.integers(-spread, spread + 1, row.size), 0, n - 1).astype(np.int32)
+    a = rng.standard_normal(row.size)
+    x, b = rng.standard_normal((2, n)).astype(np.float32)
+    d = (1.0 + rng.random(n)).astype(np.float32)
+    a32 = a.astype(np.float32)
+    grid = -(-n // 256)
+    for mode in (2, 3, 4):
+        y, pa, pb = np.zeros(n, np.float32), np.zeros(grid), np.zeros(grid)
+        wide = emu.emu_sliced32(mode, n, max(4, longest), _ptr(ptr), _ptr(ja), _ptr(a), _ptr(x), _ptr(b), _ptr(d),
+                                _ptr(y), _ptr(pa), _ptr(pb))
+        assert (wide > 0) == (spread > 65535)
+        acc = b.copy() if mode == 4 else np.zeros(n, np.float32)
+        for k in range(longest):
+            has = k < cnt
+            p = a32[ptr[:-1][has] + k] * x[ja[ptr[:-1][has] + k]]
+            acc[has] = acc[has] - p if mode == 4 else acc[has] + p
+        want = x + np.float32(0.7) * (acc / d) if mode == 4 else acc
+        np.testing.assert_array_equal(y, want, err_msg=f"mode {mode}")
+        if mode != 4:
+            starts = np.arange(0, n, 256)
+            np.testing.assert_allclose(pa, np.add.reduceat(acc.astype(float) * b, starts), rtol=0, atol=1e-11 * n)
+        if mode == 3:
+            np.testing.assert_allclose(pb, np.add.reduceat(acc.astype(float) ** 2, starts), rtol=1e-13)
