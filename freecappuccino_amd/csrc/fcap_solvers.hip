@@ -1145,7 +1145,8 @@ fc_status solve_pcg64(fc_context *ctx, const SolveArgs &args, bool dic, fc_solve
         k_pcg_xr64<<<c.gv, kRedBlock, 0, c.s>>>(n, args.fi, r, p, q, c.sc, c.pa, c.pb);
         fin(c, kFinPcgEnd, seq_or(c, c.gv, 1, r, nullptr), true);
     };
-    run_batches(c, 0, 1, dic ? 2 : 4, iter);
+    const bool level = dic && !c.sw.sf;
+    run_batches(c, level ? 0 : kDirect, 1, level ? 1 : dic ? 2 : 4, iter);
     double solve_ms = ctx->timer.stop_ms(c.s);
     check_sweeps(c);
     Scalars hs = read_scalars(c);
@@ -1224,7 +1225,7 @@ fc_status solve_bicgstab64(fc_context *ctx, const SolveArgs &args, fc_solve_info
         k_pcg_xr64<<<c.gv, kRedBlock, 0, c.s>>>(n, args.fi, res, zk, vk, c.sc, c.pa, c.pb);
         fin(c, kFinBicgEnd, seq_or(c, c.gv, 1, res, nullptr), true);
     };
-    run_batches(c, 0, 1, 2, iter);
+    run_batches(c, c.sw.sf ? kDirect : 0, 1, c.sw.sf ? 2 : 1, iter);
     double solve_ms = ctx->timer.stop_ms(c.s);
     check_sweeps(c);
     Scalars hs = read_scalars(c);
