@@ -616,7 +616,7 @@ __global__ __launch_bounds__(64) void k_sweep_syncfree(int n, const int *__restr
             __builtin_amdgcn_s_sleep(1);
         }
         if (before < b) {
-            if (BWD && p < n) mk[i] = rhs;
+            if (p < n) mk[i] = rhs;   // read again where mk is in
             if (lane == naside) aside = b;
             if (lane == naside + 1) aside = before;
             naside += 2;

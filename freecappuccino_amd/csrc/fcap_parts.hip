@@ -161,10 +161,12 @@ struct PartView {
 // the prefetch of the next windows waits for that prefetch, which cost about 1 us more at
 // each entry of the chain into another part.
 //
-// What bounds a sweep: the windows along its longest chain, 160 to 180 ns each, and about
-// 2 us where the chain enters another part (a value stored by one workgroup is seen by
-// another's poll 0.6 to 0.75 us later); from some 5 M rows also the bytes (about 80 a row
-// at W = 3 in FP64, 165 us for the 192^3 box with every input there).  Per sweep, with the
+// What bounds a sweep: the windows along its longest chain, 160 to 180 ns each, and 2 to
+// 3 us where the chain enters another part (40^3 2.8, 128^3 3.1, 192^3 2.0, over 8, 30 and
+// 47 entries; a value stored by one workgroup is seen by another's poll 0.6 to 0.75 us
+// later); from some 5 M rows also the feeders' loads (about 80 B a row at W = 3 in FP64: the
+// 192^3 box's 0.57 GB take 118 us at a copy's rate and 165 us here with every input there).
+// Per sweep, with the
 // polls in three feeders and now: 40^3 box 45 and 36 us, 96 x 80 x 72 98 and 77, 128^3 190
 // and 139, 192^3 315 and 261, 163 x 75 x 1 49 and 43.  Feeders x batch, pollers at 128^3:
 // 3 x 3, 2 pollers of 4 windows 173; 6 x 2, 2 of 4 167; 6 x 2, 4 of 2 142; 6 x 2, 6 of 1

@@ -3,6 +3,7 @@ compiled for the CPU (tests/emulate) and run under a scheduler that takes the wa
 leaves some aside for long times.  The results must not depend on it."""
 import ctypes as C
 import os
+import platform
 import re
 import shutil
 import subprocess
@@ -54,8 +55,8 @@ def _run(grid, seed=1, freeze=0.0, freeze_store=0.0, freeze_steps=1, resident=0,
 
 @pytest.fixture(scope="module")
 def emu(tmp_path_factory):
-    if not os.path.exists(CLANG):
-        pytest.skip("no clang++")
+    if not os.path.exists(CLANG) or platform.machine() != "x86_64":
+        pytest.skip("needs clang++ and x86-64")
     d = str(tmp_path_factory.mktemp("emulate"))
     for name, text in _cuts():
         with open(os.path.join(d, name), "w") as f:
