@@ -834,13 +834,13 @@ void run_batches(Ctx &c, int direct, int per_graph, int launches, const std::fun
         return flags[batch & 1] != 0;
     };
     bool done = false;
-    if (!ge.exec && c.ctx->use_graphs && c.s != nullptr) {
+    if (!ge.exec) {
         for (int k = 0; k < direct && !done; ++k) {
             iter();
             flag();
             done = b > 1 && ended(b - 2);
         }
-        if (!done) {
+        if (!done && c.ctx->use_graphs && c.s != nullptr) {
             hipGraph_t g = nullptr;
             FC_HIP_CHECK(hipStreamBeginCapture(c.s, hipStreamCaptureModeThreadLocal));
             try {

@@ -984,3 +984,46 @@ def test_solves_around_the_limit_of_direct_sums(ctx, dims, method):
         assert rel < 1e-6 * 1.01, (rel, info)
     finally:
         s.close()
+
+
+@pytest.mark.gpu
+def test_row_sweeps_of_several_contexts_at_once():
+    """Three contexts in threads of their own, each with a wave for every 64 rows of its row-wise
+    sweeps -- together more than the GPU holds, so none has all of its workgroups running: the
+    iterates of a solve alone."""
+    import threading
+    m = M.tet_box(40, permute_seed=3)
+    su = np.random.default_rng(4).uniform(-1, 1, m.n_cells)
+    contexts = [fcap.Context(0) for _ in range(3)]
+    systems, out, errors = [], [None] * 3, []
+    try:
+        for c in contexts:
+            c.set_sweep_mode(fcap.SWEEP_DEPENDENT)
+            c.set_sweep_waves(65536)
+            s = fcap.System(m, c)
+            s.assemble_laplacian(np.full(m.n_cells, -1.0), None, su)
+            systems.append(s)
+
+        def solve(k):
+            try:
+                systems[k].set_solution(np.zeros(m.n_cells))
+                systems[k].solve(fcap.METHOD_ICCG, fcap.STOP_L2, 1e-15, 40)
+                out[k] = systems[k].solution()
+            except Exception as e:   # noqa: BLE001
+                errors.append(repr(e))
+
+        solve(0)
+        alone = out[0]
+        threads = [threading.Thread(target=solve, args=(k,)) for k in range(3)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not errors, errors
+        for x in out:
+            np.testing.assert_array_equal(x, alone)
+    finally:
+        for s in systems:
+            s.close()
+        for c in contexts:
+            c.close()
